@@ -91,42 +91,47 @@ struct DeviceArray
     }
 };
 
-// Incidence records (structure of arrays, see SweepArgs): the sweep reads sids
-// and sgeo (32 B); the adjoint's vertex kernel reads ids, g0, g1, g2 (the three
-// GP rows, 56 B); shape holds the rest-shape constants the sweep's records are
-// rebuilt from when the moduli change.
+// Incidence records of the adjoint's vertex kernel (structure of arrays, CSR rows):
+// ids = (a, b, c, w mu as bits) and the three GP rows with w lambda, 56 B.
 struct IncidenceRecords
 {
-    DeviceArray<int4> ids, sids;
-    DeviceArray<float4> g0, g1, sgeo, shape;
+    DeviceArray<int4> ids;
+    DeviceArray<float4> g0, g1;
     DeviceArray<float2> g2;
-    void reset() { ids.reset(), sids.reset(), g0.reset(), g1.reset(), sgeo.reset(), shape.reset(), g2.reset(); }
+    void reset() { ids.reset(), g0.reset(), g1.reset(), g2.reset(); }
 };
 
 struct HostIncidenceRecords
 {
-    std::vector<int4> ids, sids;
-    std::vector<float4> g0, g1, sgeo, shape;
+    std::vector<int4> ids;
+    std::vector<float4> g0, g1;
     std::vector<float2> g2;
-    void resize(size_t n)
-    {
-        ids.assign(n, make_int4(-1, 0, 0, 0)); // a = -1: unused fixed-stride slot
-        sids = ids;
-        g0.assign(n, make_float4(0.f, 0.f, 0.f, 0.f));
-        g1 = g0;
-        sgeo = g0;
-        shape = g0;
-        g2.assign(n, make_float2(0.f, 0.f));
-    }
+    void resize(size_t n) { ids.resize(n), g0.resize(n), g1.resize(n), g2.resize(n); }
     void upload(IncidenceRecords& d, hipStream_t s) const
     {
         d.ids.upload(ids, s);
-        d.sids.upload(sids, s);
         d.g0.upload(g0, s);
         d.g1.upload(g1, s);
         d.g2.upload(g2, s);
-        d.sgeo.upload(sgeo, s);
-        d.shape.upload(shape, s);
+    }
+};
+
+// Star records of the sweep (device::SweepArgs) in CSR rows and, when padding is
+// cheap, fixed-stride rows; shape and tet serve changes of the moduli.
+struct StarRecords
+{
+    DeviceArray<int2> rowPtr, nbr, nbrE;
+    DeviceArray<device::StarInc> inc, incE;
+    DeviceArray<float4> shape;
+    DeviceArray<int> tet;
+    DeviceArray<int4> wideIds;
+    DeviceArray<float4> wideGeo;
+    int maxNeighbours = 0; // of an updated vertex
+    bool wide = false;     // a vertex has more than device::kMaxStarNeighbours
+    void reset()
+    {
+        rowPtr.reset(), nbr.reset(), nbrE.reset(), inc.reset(), incE.reset(), shape.reset(), tet.reset();
+        wideIds.reset(), wideGeo.reset();
     }
 };
 
@@ -274,13 +279,13 @@ struct pbat_vbd_integrator
     pbat_vbd::DeviceArray<float4> xm, xtil, xt, vel, vprev, aext;
     pbat_vbd::DeviceArray<float4> tgp; // 3 per tet
     pbat_vbd::DeviceArray<int4> tetv;
-    pbat_vbd::IncidenceRecords rows, ell; // CSR rows, fixed-stride rows
-    int ellStride = 0;   // > 0 when the fixed-stride rows exist
+    pbat_vbd::IncidenceRecords rows;
+    pbat_vbd::StarRecords star;
+    int ellStride = 0;   // > 0 when the sweep may read fixed-stride rows
     bool useEll = false; // sweep reads the fixed-stride rows
     pbat_vbd::DeviceArray<int> vtp;
     pbat_vbd::DeviceArray<double> energy;
-    // record slot of (tet, local vertex) in the CSR and fixed-stride rows (-1: not swept)
-    pbat_vbd::DeviceArray<int4> slotsRows, slotsEll;
+    pbat_vbd::DeviceArray<int4> slotsRows; // record slot of (tet, local vertex) (-1: not swept)
     pbat_vbd::DeviceArray<float2> matBase; // (w mu / Y, w lambda / Y) per tet
     std::vector<float> logY0;              // log Young's modulus per tet at construction
     std::vector<float> logYCurrent;        // last value set (log Young's modulus per tet)
@@ -364,8 +369,8 @@ struct pbat_vbd_integrator
         if (stream)
             (void)hipStreamSynchronize(stream);
         xm.reset(), xtil.reset(), xt.reset(), vel.reset(), vprev.reset(), aext.reset();
-        tgp.reset(), tetv.reset(), rows.reset(), ell.reset(), vtp.reset(), energy.reset();
-        slotsRows.reset(), slotsEll.reset(), matBase.reset(), meshOf.reset(), xkm1.reset(), xkm2.reset();
+        tgp.reset(), tetv.reset(), rows.reset(), star.reset(), vtp.reset(), energy.reset();
+        slotsRows.reset(), matBase.reset(), meshOf.reset(), xkm1.reset(), xkm2.reset();
         aggOf.reset(), aggMesh.reset(), meshAggBegin.reset(), meshCoarseOffset.reset();
         aggVertPtr.reset(), aggVerts.reset();
         gkm1.reset(), fkm1.reset(), dgk.reset(), dfk.reset(), andersonAcc.reset(), andersonGram.reset();
@@ -398,6 +403,9 @@ int EffectiveLanes(pbat_vbd_integrator const& h);
 int EffectivePerLane(pbat_vbd_integrator const& h);
 // Launch one colour's sweep over nVerts vertices with the current shape.
 void LaunchSweep(pbat_vbd_integrator& h, device::SweepArgs const& a, int nVerts);
+// Star records of the current moduli (tgp): the CSR constants, then the fixed-stride rows.
+void RebuildStarMaterial(pbat_vbd_integrator& h);
+void FillFixedStride(pbat_vbd_integrator& h);
 device::SweepArgs MakeSweepArgs(pbat_vbd_integrator& h, float sdt, float sdt2);
 // One forward Step (gpu/impl/vbd/Integrator.cu:82-103): graph replay or eager launches.
 // sync = false (rollouts): the step is only queued; the caller clears the status

@@ -36,7 +36,7 @@ using device::AdjMode;
 device::AdjointArgs MakeAdjointArgs(pbat_vbd_integrator& h, float4 const* xs, float dt)
 {
     device::AdjointArgs a{};
-    IncidenceRecords const& r = (h.useEll && h.ellStride > 0) ? h.ell : h.rows;
+    IncidenceRecords const& r = h.rows;
     a.vtp = h.vtp.ptr;
     a.ids = r.ids.ptr;
     a.g0 = r.g0.ptr;
@@ -44,7 +44,6 @@ device::AdjointArgs MakeAdjointArgs(pbat_vbd_integrator& h, float4 const* xs, fl
     a.g2 = r.g2.ptr;
     a.xs = xs;
     a.meshOf = h.meshOf.ptr;
-    a.ellStride = (h.useEll && h.ellStride > 0) ? h.ellStride : 0;
     a.invDt2 = 1.f / (dt * dt);
     return a;
 }
@@ -1453,14 +1452,9 @@ void SetLogYoung(pbat_vbd_integrator& h, float const* logY, int64_t nT)
     RolloutState& R = h.rollout;
     std::vector<float> v(logY, logY + nT);
     R.logY.upload(v, h.stream);
-    bool const ell = h.ellStride > 0;
-    auto set = [](int4 const* slots, IncidenceRecords& r) {
-        return device::RecordSet{slots, r.ids.ptr, r.g2.ptr, r.sids.ptr, r.sgeo.ptr, r.shape.ptr};
-    };
-    device::RecordSet const rows = set(h.slotsRows.ptr, h.rows);
-    device::RecordSet const ellRows = ell ? set(h.slotsEll.ptr, h.ell) : device::RecordSet{};
     hipLaunchKernelGGL(device::SetLogYoung, dim3(Blocks(nT)), dim3(256), 0, h.stream, R.logY.ptr, h.matBase.ptr,
-                       h.tgp.ptr, rows, ellRows, static_cast<int>(nT));
+                       h.tgp.ptr, h.slotsRows.ptr, h.rows.ids.ptr, h.rows.g2.ptr, static_cast<int>(nT));
+    RebuildStarMaterial(h);
     PBAT_HIP(hipGetLastError());
     PBAT_HIP(hipStreamSynchronize(h.stream));
     for (int64_t e = 0; e < nT; ++e)

@@ -303,7 +303,6 @@ struct AdjointArgs
     int vbeg;
     int vend;
     int xcdChunk;
-    int ellStride;
     float invDt2; // 1 / h^2
 };
 
@@ -344,16 +343,8 @@ __global__ __launch_bounds__(256) void AdjointVertexKernel(AdjointArgs a)
     auto vec = [&](int k) { return a.y[k]; };
     if (active)
     {
-        if (a.ellStride > 0)
-        {
-            kb = v * a.ellStride;
-            ke = kb + a.ellStride;
-        }
-        else
-        {
-            kb = a.vtp[v];
-            ke = a.vtp[v + 1];
-        }
+        kb = a.vtp[v];
+        ke = a.vtp[v + 1];
         own = a.xs[v];
         yo = vec(v);
         if (kGS && lane == 0)
@@ -894,24 +885,12 @@ __global__ __launch_bounds__(256) void Fill4(float4* __restrict__ dst, int n)
         dst[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
-// Rescale per-tet Lame coefficients to Young's moduli exp(logY) (nu fixed):
-// w*mu and w*lambda of the tet constants and of its incidence records: the
-// adjoint's records (w*mu in the id words, w*lambda in g2.y) and the sweep's,
-// rebuilt from their rest-shape constants shape = (gamma_a, gamma_b, gamma_c,
-// kappa): A = w lambda kappa^2 in the id words, sgeo = (w mu gamma_k,
-// kappa (w lambda + w mu)), in FP64 as the host builds them.
-struct RecordSet
-{
-    int4 const* __restrict__ slots; // record slot of each (tet, local vertex), -1: none
-    int4* __restrict__ ids;
-    float2* __restrict__ g2;
-    int4* __restrict__ sids;
-    float4* __restrict__ sgeo;
-    float4 const* __restrict__ shape;
-};
-
+// New moduli per tet: (w mu, w lambda) of the tet table and of the adjoint's
+// incidence records (slots: record of each (tet, local vertex), -1: none). The
+// sweep's star records follow from the tet table (StarMaterial).
 __global__ __launch_bounds__(256) void SetLogYoung(float const* __restrict__ logY, float2 const* __restrict__ base,
-                                                   float4* __restrict__ tgp, RecordSet rows, RecordSet ell, int nT)
+                                                   float4* __restrict__ tgp, int4 const* __restrict__ slots,
+                                                   int4* __restrict__ ids, float2* __restrict__ g2, int nT)
 {
     int const e = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= nT)
@@ -922,31 +901,14 @@ __global__ __launch_bounds__(256) void SetLogYoung(float const* __restrict__ log
     float4 t = tgp[3 * e + 2];
     t.y = wmu, t.z = wlam;
     tgp[3 * e + 2] = t;
-    double const dmu = wmu, dlam = wlam;
-    auto update = [&](RecordSet const& R) {
-        int4 const sl = R.slots[e];
-        int const s4[4] = {sl.x, sl.y, sl.z, sl.w};
-        for (int k = 0; k < 4; ++k)
-        {
-            int const q = s4[k];
-            if (q < 0)
-                continue;
-            int4 r = R.ids[q];
-            r.w = __float_as_int(wmu);
-            R.ids[q] = r;
-            R.g2[q].y = wlam;
-            float4 const sh = R.shape[q];
-            double const kap = sh.w;
-            int4 si = R.sids[q];
-            si.w = __float_as_int(static_cast<float>(dlam * kap * kap));
-            R.sids[q] = si;
-            R.sgeo[q] = make_float4(static_cast<float>(dmu * sh.x), static_cast<float>(dmu * sh.y),
-                                    static_cast<float>(dmu * sh.z), static_cast<float>(kap * (dlam + dmu)));
-        }
-    };
-    update(rows);
-    if (ell.slots)
-        update(ell);
+    int4 const sl = slots[e];
+    for (int q : {sl.x, sl.y, sl.z, sl.w})
+    {
+        if (q < 0)
+            continue;
+        ids[q].w = __float_as_int(wmu);
+        g2[q].y = wlam;
+    }
 }
 
 } // namespace pbat_vbd::device

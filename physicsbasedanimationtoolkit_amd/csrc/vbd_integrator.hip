@@ -6,12 +6,11 @@
 //    range and a sweep over it reads per-vertex data coalesced; within a colour
 //    vertices are grouped by mesh (batches) and sorted by degree (stable) so
 //    lanes of a wave do equal work;
-//  - each vertex-tet incidence is a 56-byte record stored in sweep order: the
-//    tet's other three vertex ids, their three shape-function-gradient rows
-//    and the tet's w*mu, w*lambda (alpha = 1 + mu/lambda is derived in the
-//    kernel). A colour pass streams its records
-//    (instead of gathering per-tet data that straddles cache lines), and only
-//    the neighbour positions are gathered, one dependent load after the record;
+//  - each updated vertex has a star record stored in sweep order: its distinct
+//    neighbours (8 B each) and its incident tets (12 B each), whose constants fold
+//    the rest shape and the material. A colour pass streams the records (instead
+//    of gathering per-tet data that straddles cache lines), and each neighbour's
+//    position is gathered once, one dependent load after the record;
 //  - positions carry the lumped mass in their 4th component, so one 16-byte
 //    gather serves both;
 //  - workgroups are reordered so each XCD's L2 serves one contiguous range of
@@ -47,15 +46,39 @@
 
 namespace pbat_vbd {
 
+// Vertices per colour from which a lane takes 3 incidences by default.
+constexpr int64_t kLargeColour = 14000;
+
+// LDS a sweep workgroup may take for its vertices' neighbour offsets.
+constexpr int kStarLdsBytes = 64 * 1024;
+
+int StarLdsBytes(pbat_vbd_integrator const& h, int block, int L)
+{
+    return block / L * std::max(h.star.maxNeighbours, 1) * static_cast<int>(sizeof(float4));
+}
+
 int EffectiveLanes(pbat_vbd_integrator const& h)
 {
-    if (h.lanes > 0)
-        return h.lanes;
-    // enough lanes that each handles about 2 incidences of the busiest vertex
-    // (degree 24: 16 lanes x 2, the shape the autotuner picks on the 64^3 grid)
-    int const d = static_cast<int>(std::max<int64_t>(h.maxDegree, 1));
-    int L = 1;
-    while (L < 64 && (d + L - 1) / L > 2)
+    if (h.star.wide)
+        return 64;
+    int L = h.lanes;
+    if (L == 0)
+    {
+        // enough lanes that each handles about 2 incidences of the busiest vertex, or
+        // 3 when the colours are large: fewer lanes waste fewer of them on the
+        // reduction and the Newton step, more shorten the chain of a small launch.
+        // Degree 24, us per launch at 16 x 2 / 8 x 3: 10^3 3.14 / 3.32, 32^3 3.43 /
+        // 3.52, 48^3 (14,400 vertices a colour) 4.65 / 4.51, 64^3 6.33 / 6.37, 80^3
+        // 9.25 / 8.53, 256 meshes (107,000 a colour) 13.4 / 11.3
+        int const d = static_cast<int>(std::max<int64_t>(h.maxDegree, 1));
+        int64_t const colours = std::max<int64_t>(static_cast<int64_t>(h.colorBegin.size()) - 1, 1);
+        int const perLane = h.nUpdated >= kLargeColour * colours ? 3 : 2;
+        L = 1;
+        while (L < 64 && (d + L - 1) / L > perLane)
+            L <<= 1;
+    }
+    // a wave's vertices keep their offsets in LDS together
+    while (L < 64 && StarLdsBytes(h, 64, L) > kStarLdsBytes)
         L <<= 1;
     return L;
 }
@@ -71,15 +94,19 @@ int EffectivePerLane(pbat_vbd_integrator const& h)
     return std::clamp((d + L - 1) / L, 1, 4);
 }
 
-template <int L, int K>
-void LaunchSweepLK(pbat_vbd_integrator& h, device::SweepArgs a, int nVerts)
+// Launch of one colour's sweep kernel: the workgroup order and, with contact, the
+// pending range of the previous colour (gpu/impl/vbd/Integrator.cu:303-326: the
+// colour writes a buffer; the next colour's launch reads the pending range there
+// and copies it back).
+template <class Plain, class Contact>
+void LaunchColour(pbat_vbd_integrator& h, device::SweepArgs a, int nVerts, int L, int block, int lds, Plain plain,
+                  Contact contact)
 {
     int const vbeg = a.vbeg;
-    int const block = h.blockSize;
     int64_t const threads = static_cast<int64_t>(nVerts) * L;
     int64_t grid64 = (threads + block - 1) / block;
     a.xcdChunk = 0;
-    if (h.xcdRemap && grid64 >= 16)
+    if (h.xcdRemap && grid64 >= 16 && !h.star.wide)
     {
         // pad to a multiple of the 8 XCDs; padded blocks hold no vertex
         grid64 = (grid64 + 7) / 8 * 8;
@@ -90,19 +117,27 @@ void LaunchSweepLK(pbat_vbd_integrator& h, device::SweepArgs a, int nVerts)
         Fail(PBAT_VBD_ERROR_INVALID_ARGUMENT, "colour too large for the sweep launch: reduce lanes per vertex");
     if (!h.contact)
     {
-        hipLaunchKernelGGL((device::VbdSweep<L, K>), dim3(static_cast<int>(grid64)), dim3(block), 0, h.stream, a);
+        hipLaunchKernelGGL(plain, dim3(static_cast<int>(grid64)), dim3(block), lds, h.stream, a);
         return;
     }
-    // gpu/impl/vbd/Integrator.cu:303-326: the colour writes a buffer; the next colour's
-    // launch reads the pending range there and copies it back
     // the same colour again (a single colour), or a pending range larger than this
     // launch can copy: copy it back first
     if ((h.pendBeg == vbeg && h.pendEnd > h.pendBeg) || static_cast<int64_t>(h.pendEnd - h.pendBeg) > grid64 * block)
         FlushContactSweep(h);
     a.contact.rec = h.crec.ptr, a.contact.xb = h.xb.ptr, a.contact.muF = h.muF, a.contact.epsv = h.epsv;
     a.contact.pendBeg = h.pendBeg, a.contact.pendEnd = h.pendEnd;
-    hipLaunchKernelGGL((device::VbdSweep<L, K, true>), dim3(static_cast<int>(grid64)), dim3(block), 0, h.stream, a);
+    hipLaunchKernelGGL(contact, dim3(static_cast<int>(grid64)), dim3(block), lds, h.stream, a);
     h.pendBeg = vbeg, h.pendEnd = vbeg + nVerts;
+}
+
+template <int L, int K>
+void LaunchSweepLK(pbat_vbd_integrator& h, device::SweepArgs const& a, int nVerts)
+{
+    int block = h.blockSize;
+    while (block > 64 && StarLdsBytes(h, block, L) > kStarLdsBytes)
+        block -= 64;
+    LaunchColour(h, a, nVerts, L, block, StarLdsBytes(h, block, L), device::VbdSweep<L, K, false>,
+                 device::VbdSweep<L, K, true>);
 }
 
 template <int L>
@@ -119,6 +154,11 @@ void LaunchSweepL(pbat_vbd_integrator& h, device::SweepArgs const& a, int nVerts
 
 void LaunchSweep(pbat_vbd_integrator& h, device::SweepArgs const& a, int nVerts)
 {
+    if (h.star.wide)
+    {
+        LaunchColour(h, a, nVerts, 64, h.blockSize, 0, device::VbdSweepWide<false>, device::VbdSweepWide<true>);
+        return;
+    }
     switch (EffectiveLanes(h))
     {
         case 1: LaunchSweepL<1>(h, a, nVerts); break;
@@ -134,10 +174,15 @@ void LaunchSweep(pbat_vbd_integrator& h, device::SweepArgs const& a, int nVerts)
 device::SweepArgs MakeSweepArgs(pbat_vbd_integrator& h, float sdt, float sdt2)
 {
     device::SweepArgs a{};
-    pbat_vbd::IncidenceRecords const& r = (h.useEll && h.ellStride > 0) ? h.ell : h.rows;
-    a.vtp = h.vtp.ptr;
-    a.ids = r.sids.ptr;
-    a.geo = r.sgeo.ptr;
+    bool const fixed = h.useEll && h.star.incE.ptr;
+    a.rowPtr = h.star.rowPtr.ptr;
+    a.nbr = fixed ? h.star.nbrE.ptr : h.star.nbr.ptr;
+    a.inc = fixed ? h.star.incE.ptr : h.star.inc.ptr;
+    a.nbrStride = fixed ? h.star.maxNeighbours : 0;
+    a.incStride = fixed ? h.ellStride : 0;
+    a.ldsStride = std::max(h.star.maxNeighbours, 1);
+    a.wideIds = h.star.wideIds.ptr;
+    a.wideGeo = h.star.wideGeo.ptr;
     a.xm = h.xm.ptr;
     a.xtil = h.xtil.ptr;
     a.xt = h.xt.ptr;
@@ -147,9 +192,33 @@ device::SweepArgs MakeSweepArgs(pbat_vbd_integrator& h, float sdt, float sdt2)
     a.c.detHZero = h.detHZero;
     a.c.fp64Solves = h.fp64Solves.ptr;
     a.ntStream = h.ntStream ? 1 : 0;
-    if (h.useEll && h.ellStride > 0)
-        a.ellStride = h.ellStride;
     return a;
+}
+
+void FillFixedStride(pbat_vbd_integrator& h)
+{
+    if (!h.star.incE.ptr)
+        return;
+    int const width = std::max(h.star.maxNeighbours, h.ellStride);
+    int64_t const n = h.nUpdated * width;
+    hipLaunchKernelGGL(device::StarFixedStride, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, h.stream,
+                       h.star.rowPtr.ptr, h.star.nbr.ptr, h.star.inc.ptr, h.star.nbrE.ptr, h.star.incE.ptr,
+                       static_cast<int>(h.nUpdated), h.star.maxNeighbours, h.ellStride);
+}
+
+void RebuildStarMaterial(pbat_vbd_integrator& h)
+{
+    device::StarMaterialArgs a{};
+    a.rowPtr = h.star.rowPtr.ptr, a.nbr = h.star.nbr.ptr, a.inc = h.star.inc.ptr;
+    a.shape = h.star.shape.ptr, a.tet = h.star.tet.ptr, a.tgp = h.tgp.ptr;
+    a.wideIds = h.star.wideIds.ptr, a.wideGeo = h.star.wideGeo.ptr;
+    a.nRows = static_cast<int>(h.nUpdated);
+    a.width = std::max<int>(h.star.maxNeighbours, static_cast<int>(h.maxDegree));
+    int64_t const n = h.nUpdated * a.width;
+    if (n == 0)
+        return;
+    hipLaunchKernelGGL(device::StarMaterial, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, h.stream, a);
+    FillFixedStride(h);
 }
 
 hipEvent_t NextEvent(pbat_vbd_integrator& h)
@@ -649,6 +718,11 @@ void BuildAggregates(pbat_vbd_integrator& h, pbat_vbd_data const* d, std::vector
     PBAT_HIP(hipStreamSynchronize(h.stream));
 }
 
+// Last-level (Infinity) cache of the MI355X.
+constexpr int64_t kLastLevelCacheBytes = int64_t{256} << 20;
+
+static int TV4(int4 const& t, int l) { return l == 0 ? t.x : l == 1 ? t.y : l == 2 ? t.z : t.w; }
+
 // vertexOffsets (batches): first vertex of each mesh in d's numbering, count + 1
 // entries; vertices of one colour are then grouped by mesh.
 void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64_t> const* vertexOffsets = nullptr)
@@ -810,10 +884,7 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
         G4[3 * e + 2] = make_float4(gp(3, 2), static_cast<float>(w * mu), static_cast<float>(w * lam),
                                     static_cast<float>(1. + mu / lam));
     }
-    // Incidence records in internal numbering and sweep order: for each
-    // incidence the tet's other three vertices (local order) with their GP
-    // rows, and the tet's w*mu (in the id word) and w*lambda. Only updated
-    // vertices are swept, so only their rows are stored.
+    // Rows of the updated vertices in internal numbering and sweep order.
     std::vector<int> P(static_cast<size_t>(nV) + 1, 0);
     for (int64_t v = 0; v < nV; ++v)
     {
@@ -830,94 +901,145 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
     h->maxDegree = 0;
     for (int64_t v = 0; v < nUpd; ++v)
         h->maxDegree = std::max<int64_t>(h->maxDegree, P[v + 1] - P[v]);
-    int64_t const nIncUpd = P[nUpd];
-    std::vector<int4> slots(static_cast<size_t>(nT), make_int4(-1, -1, -1, -1));
-    auto setSlot = [](int4& s, int il, int slot) {
-        (il == 0 ? s.x : il == 1 ? s.y : il == 2 ? s.z : s.w) = slot;
-    };
-    auto fill = [&](HostIncidenceRecords& R, int64_t slot, int64_t k) {
-        int64_t const e = d->GVGe[k];
-        int const il = static_cast<int>(d->GVGilocal[k]);
-        setSlot(slots[e], il, static_cast<int>(slot));
-        double const* G = d->GP + 12 * e; // G(r, c) = G[4c + r]
-        double const w = d->wg[e], mu = d->lame[2 * e], lam = d->lame[2 * e + 1];
-        int ids[3];
-        float g[3][3];
-        double gd[3][3], own[3];
-        int n = 0;
-        for (int c = 0; c < 3; ++c)
-            own[c] = G[4 * c + il];
-        for (int j = 0; j < 4; ++j)
-        {
-            if (j == il)
-                continue;
-            ids[n] = h->iperm[d->E[4 * e + j]];
-            for (int c = 0; c < 3; ++c)
-            {
-                gd[n][c] = G[4 * c + j];
-                g[n][c] = static_cast<float>(gd[n][c]);
-            }
-            ++n;
-        }
-        float4 const m = G4[3 * e + 2]; // (., w*mu, w*lambda, alpha)
-        int wmuBits;
-        std::memcpy(&wmuBits, &m.y, sizeof(int));
-        R.ids[slot] = make_int4(ids[0], ids[1], ids[2], wmuBits);
-        R.g0[slot] = make_float4(g[0][0], g[0][1], g[0][2], g[1][0]);
-        R.g1[slot] = make_float4(g[1][1], g[1][2], g[2][0], g[2][1]);
-        R.g2[slot] = make_float2(g[2][2], m.z);
-        // sweep record (FP64 from the FP64 GP and material): with gamma_k = g_k . g
-        // (the other rows with the own row g) and kappa = det of the other three
-        // rows, sids.w = bits of w lambda kappa^2 and sgeo = (w mu gamma_a,
-        // w mu gamma_b, w mu gamma_c, kappa (w lambda + w mu)); shape keeps
-        // (gamma_a, gamma_b, gamma_c, kappa) for later changes of the moduli
-        auto dot = [](double const* a, double const* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; };
-        double const kappa = gd[0][0] * (gd[1][1] * gd[2][2] - gd[1][2] * gd[2][1]) -
-                             gd[0][1] * (gd[1][0] * gd[2][2] - gd[1][2] * gd[2][0]) +
-                             gd[0][2] * (gd[1][0] * gd[2][1] - gd[1][1] * gd[2][0]);
-        double const ga = dot(gd[0], own), gb = dot(gd[1], own), gc = dot(gd[2], own);
-        double const wmu = w * mu, wlam = w * lam;
-        float const A = static_cast<float>(wlam * kappa * kappa);
-        int Abits;
-        std::memcpy(&Abits, &A, sizeof(int));
-        R.sids[slot] = make_int4(ids[0], ids[1], ids[2], Abits);
-        R.sgeo[slot] = make_float4(static_cast<float>(wmu * ga), static_cast<float>(wmu * gb),
-                                   static_cast<float>(wmu * gc), static_cast<float>(kappa * (wlam + wmu)));
-        R.shape[slot] = make_float4(static_cast<float>(ga), static_cast<float>(gb), static_cast<float>(gc),
-                                    static_cast<float>(kappa));
-    };
+    size_t const nIncUpd = static_cast<size_t>(P[nUpd]);
+    // The adjoint's incidence records: the tet's other three vertices (local order)
+    // with their GP rows, w*mu (in the id word) and w*lambda. The sweep's star
+    // records: with gamma_k = g_k . g (the other rows with the own row g) and kappa =
+    // det of the other three rows, A = w lambda kappa^2 and B = kappa (w lambda +
+    // w mu) per tet and Gamma_j = sum of w mu gamma_k per neighbour, from the FP64 GP
+    // and material; shape keeps (gamma_a, gamma_b, gamma_c, kappa) for later changes
+    // of the moduli.
     {
+        std::vector<int4> slots(static_cast<size_t>(nT), make_int4(-1, -1, -1, -1));
         HostIncidenceRecords R;
-        R.resize(static_cast<size_t>(nIncUpd));
+        R.resize(nIncUpd);
+        std::vector<int2> rowPtr(static_cast<size_t>(nUpd) + 1, make_int2(0, 0)), nbr;
+        std::vector<device::StarInc> inc(nIncUpd);
+        std::vector<float4> shape(nIncUpd);
+        std::vector<int> tet(nIncUpd);
+        nbr.reserve(nIncUpd);
+        std::vector<int> at(static_cast<size_t>(nV), -1), row; // position of a vertex in the current row
+        std::vector<double> sum;
         for (int64_t v = 0; v < nUpd; ++v)
         {
-            int64_t const i = h->perm[v];
-            for (int64_t k = d->GVGp[i]; k < d->GVGp[i + 1]; ++k)
-                fill(R, P[v] + (k - d->GVGp[i]), k);
+            int64_t const i = h->perm[v], k0 = d->GVGp[i], k1 = d->GVGp[i + 1];
+            row.clear();
+            for (int64_t k = k0; k < k1; ++k)
+                for (int j = 0; j < 4; ++j)
+                {
+                    int const q = TV4(TV[d->GVGe[k]], j);
+                    if (q != static_cast<int>(v) && at[q] < 0)
+                        at[q] = 0, row.push_back(q);
+                }
+            for (size_t s = 0; s < row.size(); ++s)
+                at[row[s]] = static_cast<int>(s);
+            sum.assign(row.size(), 0.);
+            for (int64_t k = k0; k < k1; ++k)
+            {
+                int64_t const e = d->GVGe[k];
+                int const il = static_cast<int>(d->GVGilocal[k]);
+                size_t const slot = static_cast<size_t>(P[v] + (k - k0));
+                int4& sl = slots[e];
+                (il == 0 ? sl.x : il == 1 ? sl.y : il == 2 ? sl.z : sl.w) = static_cast<int>(slot);
+                double const* G = d->GP + 12 * e; // G(r, c) = G[4c + r]
+                double const wmu = d->wg[e] * d->lame[2 * e], wlam = d->wg[e] * d->lame[2 * e + 1];
+                int ids[3], n = 0;
+                double gd[3][3], own[3];
+                for (int c = 0; c < 3; ++c)
+                    own[c] = G[4 * c + il];
+                for (int j = 0; j < 4; ++j)
+                {
+                    if (j == il)
+                        continue;
+                    ids[n] = TV4(TV[e], j);
+                    for (int c = 0; c < 3; ++c)
+                        gd[n][c] = G[4 * c + j];
+                    ++n;
+                }
+                float4 const m = G4[3 * e + 2]; // (., w*mu, w*lambda, alpha)
+                int wmuBits;
+                std::memcpy(&wmuBits, &m.y, sizeof(int));
+                auto f = [&](int r, int c) { return static_cast<float>(gd[r][c]); };
+                R.ids[slot] = make_int4(ids[0], ids[1], ids[2], wmuBits);
+                R.g0[slot] = make_float4(f(0, 0), f(0, 1), f(0, 2), f(1, 0));
+                R.g1[slot] = make_float4(f(1, 1), f(1, 2), f(2, 0), f(2, 1));
+                R.g2[slot] = make_float2(f(2, 2), m.z);
+                auto dot = [](double const* a, double const* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; };
+                double const kappa = gd[0][0] * (gd[1][1] * gd[2][2] - gd[1][2] * gd[2][1]) -
+                                     gd[0][1] * (gd[1][0] * gd[2][2] - gd[1][2] * gd[2][0]) +
+                                     gd[0][2] * (gd[1][0] * gd[2][1] - gd[1][1] * gd[2][0]);
+                double const gamma[3] = {dot(gd[0], own), dot(gd[1], own), dot(gd[2], own)};
+                for (int j = 0; j < 3; ++j)
+                    sum[at[ids[j]]] += wmu * gamma[j];
+                // positions of a wide row do not fit; VbdSweepWide reads none
+                inc[slot] = device::StarInc{static_cast<unsigned>(at[ids[0]]) | static_cast<unsigned>(at[ids[1]]) << 8 |
+                                                static_cast<unsigned>(at[ids[2]]) << 16,
+                                            static_cast<float>(wlam * kappa * kappa),
+                                            static_cast<float>(kappa * (wlam + wmu))};
+                shape[slot] = make_float4(static_cast<float>(gamma[0]), static_cast<float>(gamma[1]),
+                                          static_cast<float>(gamma[2]), static_cast<float>(kappa));
+                tet[slot] = static_cast<int>(e);
+            }
+            // a row too long for the 8-bit positions, or more neighbours than 32 bits index
+            h->star.maxNeighbours = std::max(h->star.maxNeighbours, static_cast<int>(row.size()));
+            if (h->star.maxNeighbours > device::kMaxStarNeighbours ||
+                nbr.size() + row.size() > static_cast<size_t>(std::numeric_limits<int>::max()))
+                h->star.wide = true, nbr.clear();
+            for (size_t s = 0; s < row.size(); ++s)
+            {
+                float const Gj = static_cast<float>(sum[s]);
+                int bits;
+                std::memcpy(&bits, &Gj, sizeof(int));
+                if (!h->star.wide)
+                    nbr.push_back(make_int2(row[s], bits));
+                at[row[s]] = -1;
+            }
+            rowPtr[v + 1] = make_int2(static_cast<int>(nbr.size()), P[v + 1]);
         }
         R.upload(h->rows, h->stream);
         h->slotsRows.upload(slots, h->stream);
+        h->star.rowPtr.upload(rowPtr, h->stream);
+        h->star.nbr.upload(nbr, h->stream);
+        h->star.inc.upload(inc, h->stream);
+        h->star.shape.upload(shape, h->stream);
+        h->star.tet.upload(tet, h->stream);
+        if (h->star.wide)
+        {
+            std::vector<int4> wideIds(nIncUpd);
+            std::vector<float4> wideGeo(nIncUpd);
+            for (size_t k = 0; k < nIncUpd; ++k)
+            {
+                float const wmu = G4[3 * static_cast<size_t>(tet[k]) + 2].y;
+                int bits;
+                std::memcpy(&bits, &inc[k].A, sizeof(int));
+                wideIds[k] = make_int4(R.ids[k].x, R.ids[k].y, R.ids[k].z, bits);
+                wideGeo[k] = make_float4(wmu * shape[k].x, wmu * shape[k].y, wmu * shape[k].z, inc[k].B);
+            }
+            h->star.wideIds.upload(wideIds, h->stream);
+            h->star.wideGeo.upload(wideGeo, h->stream);
+            PBAT_HIP(hipStreamSynchronize(h->stream));
+        }
         PBAT_HIP(hipStreamSynchronize(h->stream));
     }
-    // Fixed-stride copy when padding every row to the maximum degree costs at
-    // most 35% more records than the CSR rows.
-    if (nUpd > 0 && h->maxDegree > 0 && h->maxDegree * nUpd * 100 <= 135 * nIncUpd &&
-        h->maxDegree * nUpd < (int64_t{1} << 31))
+    // Fixed-stride rows when padding every row to the maximum degree costs at most
+    // 35% more records than the CSR rows. The sweep reads them by default (one
+    // dependent load less: 6.33 instead of 6.76 us a launch on 64^3) while the records
+    // fit the 256 MB last-level cache; beyond it the unpadded CSR rows, read with
+    // non-temporal loads that leave the cache to the positions, are faster (256
+    // meshes, 373 MB of records: 11.3 us against 13.6).
+    if (nUpd > 0 && h->maxDegree > 0 &&
+        h->maxDegree * nUpd * 100 <= 135 * static_cast<int64_t>(nIncUpd) && h->maxDegree * nUpd < (int64_t{1} << 31))
     {
-        int64_t const S = h->maxDegree;
-        HostIncidenceRecords R;
-        R.resize(static_cast<size_t>(nUpd * S));
-        std::fill(slots.begin(), slots.end(), make_int4(-1, -1, -1, -1));
-        for (int64_t v = 0; v < nUpd; ++v)
+        h->ellStride = static_cast<int>(h->maxDegree);
+        int64_t const bytes = static_cast<int64_t>(h->star.nbr.n * sizeof(int2) + nIncUpd * sizeof(device::StarInc));
+        h->useEll = bytes <= kLastLevelCacheBytes;
+        h->ntStream = !h->useEll;
+        if (!h->star.wide)
         {
-            int64_t const i = h->perm[v];
-            for (int64_t k = d->GVGp[i]; k < d->GVGp[i + 1]; ++k)
-                fill(R, v * S + (k - d->GVGp[i]), k);
+            h->star.nbrE.allocate(static_cast<size_t>(nUpd) * h->star.maxNeighbours);
+            h->star.incE.allocate(static_cast<size_t>(nUpd) * h->maxDegree);
+            FillFixedStride(*h);
         }
-        R.upload(h->ell, h->stream);
-        h->slotsEll.upload(slots, h->stream);
-        PBAT_HIP(hipStreamSynchronize(h->stream));
-        h->ellStride = static_cast<int>(S);
     }
 
     h->wgHost.resize(static_cast<size_t>(nT));

@@ -6,10 +6,9 @@
 //   xtil[v]  float4 (x~, 0)           inertial target
 //   xt[v]    float4 (x_t, 0)          positions at the start of the substep
 //   vel[v], vprev[v], aext[v]  float4 velocities and external acceleration
-//   vtp[v]   int32 CSR prefix over vertex-tet incidences
-//   incidence records (32 B, structure of arrays, in sweep order): the other
-//            three vertex ids of the tet and four constants of its GP rows and
-//            material (see SweepArgs)
+//   star records (per updated vertex, in sweep order): its neighbours (8 B each)
+//            and its incident tets (12 B each) with constants of their GP rows
+//            and materials (see SweepArgs)
 //   tgp[3e..3e+2]  float4 x3 (48 B) per tet: rows 1..3 of the shape function
 //            gradients GP (row 0 = -(row1+row2+row3)), w*mu, w*lambda, alpha
 //   tetv[e]  int4 vertex ids of tet e
@@ -87,30 +86,28 @@ __device__ __forceinline__ void GroupSum(Block& B)
 // row and kappa = det G, F = D G with D = [d_a d_b d_c], so
 //   F g = sum_k gamma_k d_k (gamma_k = g_k . g),   J = kappa (d_a . n),
 //   c = cof(D) cof(G) g = -kappa n,   |g|^2 = -sum_k gamma_k,
-// where n = (x_b - x_a) x (x_c - x_a) (the column sum of cof D) and G^-T g =
-// -(1, 1, 1). With the record's A = w lambda kappa^2, B = kappa (w lambda + w mu)
-// and gamma'_k = w mu gamma_k (rest-shape and material constants, FP64 on the
-// host), the terms are
-//   grad_i += sum_k gamma'_k d_k - (A (d_a . n) - B) n
-//   Hess_i += -(sum_k gamma'_k) I + A n n^T.
-__device__ __forceinline__ void AccumulateElastic(float4 const& geo, float A, float4 const& own, float4 const& pa,
-                                                  float4 const& pb, float4 const& pc, Block& B)
+// where n = (d_b - d_a) x (d_c - d_a) (the column sum of cof D) and G^-T g =
+// -(1, 1, 1). The gamma terms are linear in the d_k, so over the whole star
+// they fold into one constant per neighbour j,
+//   Gamma_j = sum over the tets holding j of w mu gamma_k
+// (summed in FP64 on the host), and a tet is left with A = w lambda kappa^2 and
+// B = kappa (w lambda + w mu):
+//   grad_i = sum_j Gamma_j d_j - sum_e (A (d_a . n) - B) n
+//   Hess_i = -(sum_j Gamma_j) I + sum_e A n n^T.
+__device__ __forceinline__ void AccumulateTet(float A, float Bk, float4 const& da, float4 const& db,
+                                              float4 const& dc, Block& B)
 {
-    float const dax = pa.x - own.x, day = pa.y - own.y, daz = pa.z - own.z;
-    float const dbx = pb.x - own.x, dby = pb.y - own.y, dbz = pb.z - own.z;
-    float const dcx = pc.x - own.x, dcy = pc.y - own.y, dcz = pc.z - own.z;
-    float const ex = pb.x - pa.x, ey = pb.y - pa.y, ez = pb.z - pa.z;
-    float const fx = pc.x - pa.x, fy = pc.y - pa.y, fz = pc.z - pa.z;
+    float const ex = db.x - da.x, ey = db.y - da.y, ez = db.z - da.z;
+    float const fx = dc.x - da.x, fy = dc.y - da.y, fz = dc.z - da.z;
     float const nx = ey * fz - ez * fy, ny = ez * fx - ex * fz, nz = ex * fy - ey * fx;
-    float const coef = A * (dax * nx + day * ny + daz * nz) - geo.w;
-    B.g0 += geo.x * dax + geo.y * dbx + geo.z * dcx - coef * nx;
-    B.g1 += geo.x * day + geo.y * dby + geo.z * dcy - coef * ny;
-    B.g2 += geo.x * daz + geo.y * dbz + geo.z * dcz - coef * nz;
-    float const dg = -(geo.x + geo.y + geo.z);
+    float const coef = A * (da.x * nx + da.y * ny + da.z * nz) - Bk;
+    B.g0 -= coef * nx;
+    B.g1 -= coef * ny;
+    B.g2 -= coef * nz;
     float const anx = A * nx, any = A * ny, anz = A * nz;
-    B.h00 += dg + anx * nx;
-    B.h11 += dg + any * ny;
-    B.h22 += dg + anz * nz;
+    B.h00 += anx * nx;
+    B.h11 += any * ny;
+    B.h22 += anz * nz;
     B.h01 += anx * ny;
     B.h02 += anx * nz;
     B.h12 += any * nz;
@@ -191,80 +188,168 @@ __device__ __forceinline__ float3 InertiaNewtonStep(Block B, float4 const& xv, f
                        (a02 * B.g0 + a12 * B.g1 + a22 * B.g2) * inv);
 }
 
-// Incidence records, structure of arrays, row k of vertex v's incidences
-// (CSR rows through vtp, or fixed-stride rows of ellStride entries), 32 B:
-//   ids[k] int4   (a, b, c, A as bits): the tet's other three vertices in
-//                 local order; a = -1 marks an unused fixed-stride slot
-//   geo[k] float4 (gamma'_a, gamma'_b, gamma'_c, B) (AccumulateElastic)
-// Records are stored in sweep order, so a colour pass streams them.
+// Star records of the updated vertices, in sweep order, so a colour pass streams
+// them. Row v holds the vertex's distinct neighbours and its incident tets
+// (CSR rows through rowPtr = (first neighbour, first tet), or fixed-stride rows
+// of nbrStride and incStride entries, padded with (v, 0) and zero tets):
+//   nbr[k] int2      (neighbour j, Gamma_j as bits)
+//   inc[k] StarInc   positions a | b << 8 | c << 16 of the tet's other vertices
+//                    in the vertex's neighbour row, then A and B
+// 12 B per tet and 8 B per neighbour (AccumulateTet).
+struct StarInc
+{
+    unsigned int pk;
+    float A, B;
+};
+
+// Neighbours a star row may hold: its positions are 8 bits wide.
+constexpr int kMaxStarNeighbours = 256;
+
 struct SweepArgs
 {
-    int const* __restrict__ vtp;
-    int4 const* __restrict__ ids;
-    float4 const* __restrict__ geo;
+    int2 const* __restrict__ rowPtr;
+    int2 const* __restrict__ nbr;
+    StarInc const* __restrict__ inc;
     float4* __restrict__ xm;
     float4 const* __restrict__ xtil;
     float4 const* __restrict__ xt;
     int vbeg;
     int vend;
     int xcdChunk;  // > 0: blocks per XCD for the XCD-aware block order
-    int ntStream;  // != 0: read the incidence records with non-temporal loads
-    int ellStride; // > 0: fixed-stride rows of this many records
+    int ntStream;  // != 0: read the star records with non-temporal loads
+    int nbrStride; // > 0: fixed-stride rows
+    int incStride;
+    int ldsStride; // neighbour offsets a vertex keeps in LDS
     StepConstants c;
     ContactSweep contact; // contact sweeps only
+    // meshes with a vertex of more than kMaxStarNeighbours neighbours
+    // (VbdSweepWide): per tet the other vertices with A as bits, and
+    // (w mu gamma_a, w mu gamma_b, w mu gamma_c, B)
+    int4 const* __restrict__ wideIds;
+    float4 const* __restrict__ wideGeo;
 };
 
-typedef int v4i __attribute__((ext_vector_type(4)));
-typedef float v4f __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
-// Loads of the incidence stream, optionally with the non-temporal hint.
-__device__ __forceinline__ int4 LoadIds(int4 const* p, bool nt)
+// Loads of the star records and of the adjoint's incidence records, optionally
+// with the non-temporal hint.
+__device__ __forceinline__ int2 LoadNbr(int2 const* p, bool nt)
 {
     if (nt)
     {
-        v4i const r = __builtin_nontemporal_load(reinterpret_cast<v4i const*>(p));
-        return make_int4(r.x, r.y, r.z, r.w);
+        v2i const r = __builtin_nontemporal_load(reinterpret_cast<v2i const*>(p));
+        return make_int2(r.x, r.y);
     }
     return *p;
 }
 
-__device__ __forceinline__ float4 LoadConst(float4 const* p, bool nt)
+__device__ __forceinline__ StarInc LoadInc(StarInc const* p, bool nt)
 {
     if (nt)
-    {
-        v4f const r = __builtin_nontemporal_load(reinterpret_cast<v4f const*>(p));
-        return make_float4(r.x, r.y, r.z, r.w);
-    }
+        return StarInc{__builtin_nontemporal_load(&p->pk), __builtin_nontemporal_load(&p->A),
+                       __builtin_nontemporal_load(&p->B)};
     return *p;
 }
 
-__device__ __forceinline__ float2 LoadConst(float2 const* p, bool nt)
+// Inertia, Newton step and write of one vertex, with the contact block of a
+// contact sweep (added after damping and before inertia); the group's first lane.
+template <bool C>
+__device__ __forceinline__ void FinishVertex(SweepArgs const& a, int v, Block& B, Block const& Cb, float4 const& own,
+                                             float4 const& xl, float4 const& xto)
 {
-    if (nt)
+    if constexpr (C)
     {
-        v2f const r = __builtin_nontemporal_load(reinterpret_cast<v2f const*>(p));
-        return make_float2(r.x, r.y);
+        Damp(B, own, xto, a.c);
+        B.h00 += Cb.h00, B.h01 += Cb.h01, B.h02 += Cb.h02, B.h11 += Cb.h11, B.h12 += Cb.h12, B.h22 += Cb.h22;
+        B.g0 += Cb.g0, B.g1 += Cb.g1, B.g2 += Cb.g2;
+        float3 const dx = InertiaNewtonStep(B, own, xl, a.c);
+        a.contact.xb[v] = make_float4(own.x - dx.x, own.y - dx.y, own.z - dx.z, own.w);
     }
-    return *p;
+    else
+    {
+        // the start position only matters with damping: loaded here rather than
+        // held in registers through the incidence loop
+        float3 const dx = NewtonStep(B, own, xl, (a.c.kD != 0.f) ? a.xt[v] : own, a.c);
+        a.xm[v] = make_float4(own.x - dx.x, own.y - dx.y, own.z - dx.z, own.w);
+    }
 }
+
+// Position of vertex j as a sweep reads it.
+template <bool C>
+__device__ __forceinline__ float4 SweepPosition(SweepArgs const& a, int j)
+{
+    if constexpr (C)
+        return ContactPosition(a.contact, a.xm, j);
+    else
+        return a.xm[j];
+}
+
+// The contact part of a contact sweep: the lane's contact records (slots lane,
+// lane + L, ...), issued early, and the copy back of the previous colour's new
+// positions.
+template <int L>
+struct ContactSlots
+{
+    static constexpr int kSlots = (kMaxContacts + L - 1) / L;
+    int4 rec[kSlots];
+    float4 xto;
+    __device__ __forceinline__ void Load(SweepArgs const& a, int v, bool active, int lane, int tid, float4 const& own)
+    {
+        xto = own;
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j)
+        {
+            int const k = lane + j * L;
+            rec[j] = (active && k < kMaxContacts) ? a.contact.rec[static_cast<size_t>(v) * kMaxContacts + k]
+                                                  : make_int4(-1, -1, -1, 0);
+        }
+        if (active)
+            xto = a.xt[v];
+        int const pend = a.contact.pendBeg + tid;
+        if (pend < a.contact.pendEnd)
+            a.xm[pend] = a.contact.xb[pend];
+    }
+    __device__ __forceinline__ void Accumulate(SweepArgs const& a, float4 const& own, Block& Cb) const
+    {
+        float3 const xo = make_float3(own.x, own.y, own.z), xt3 = make_float3(xto.x, xto.y, xto.z);
+#pragma unroll
+        for (int j = 0; j < kSlots; ++j)
+            if (rec[j].x >= 0)
+                AccumulateContact(xt3, xo, a.contact, a.xm, a.xt, rec[j], a.c.dt, __int_as_float(rec[j].w),
+                                  a.contact.muF, a.contact.epsv, Cb);
+    }
+};
 
 // One colour of one VBD sweep (sim/vbd/Integrator.cpp:73-136,
-// gpu/impl/vbd/Kernels.cuh:148-233). L lanes cooperate on each vertex: lane l
-// of the group takes incidences l, l+L, ... of the vertex's row, first
-// issuing the loads of its first K incidences together, then accumulating.
+// gpu/impl/vbd/Kernels.cuh:148-233). L lanes of a wave cooperate on each vertex:
+// lane l takes neighbours and tets l, l + L, ... of the vertex's rows, the loads
+// of its first N neighbours and K tets issued together. A neighbour's position
+// is gathered once per vertex; its offset d_j goes to LDS (the group's own slots,
+// exchanged within the wave: no barrier), from which the tets read their three.
 // The group reduces its 9 partial sums with DPP and its first lane applies the
 // Newton update in place: vertices of one colour share no tet, so none reads
 // what another vertex of the colour writes.
+// What bounds it: on 256 meshes (107,000 vertices a colour, 373 MB of records,
+// beyond the last-level cache) the stream of records, 4.1 TB/s; on 64^3 that
+// stream (15 MB a launch) and the VALU next to a fixed ~3 us of launch ramp and
+// dependent loads; on small meshes the latter alone. Per launch, best shape: 64^3
+// 6.33 us, 80^3 8.5, 256 meshes 11.5. With 32 B and three 16-byte position gathers
+// per tet (72 gathers a vertex instead of 14) the L1's gather rate and the record
+// stream took 9.06, 16.2 and 22.0.
 // With C (scenes in contact), the vertex's contact terms join its block after
 // damping and before inertia (gpu/impl/vbd/Kernels.cuh:200-230), and the new
 // positions go to contact.xb, so contact terms of the colour read positions from
 // before its pass (the reference's write buffer, gpu/impl/vbd/Integrator.cu:303-326).
 // The previous colour's positions are read from xb and copied back to xm by
 // this launch; the last colour of an iteration is copied back by the host.
+// Dynamic LDS: blockDim / L x ldsStride float4.
 template <int L, int K, bool C = false>
 __global__ __launch_bounds__(256) void VbdSweep(SweepArgs a)
 {
+    constexpr int N = (K + 1) / 2; // about 0.6 neighbours per tet
+    extern __shared__ float4 starLds[];
     int block = static_cast<int>(blockIdx.x);
     if (a.xcdChunk > 0)
     {
@@ -278,136 +363,224 @@ __global__ __launch_bounds__(256) void VbdSweep(SweepArgs a)
     int const lane = tid & (L - 1);
     int const v = a.vbeg + tid / L;
     bool const active = v < a.vend;
-    int kb = 0, ke = 0;
+    float4* const d = starLds + (static_cast<int>(threadIdx.x) / L) * a.ldsStride;
+    int nb = 0, ne = 0, kb = 0, ke = 0;
     float4 own = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 xl = own;
     if (active)
     {
-        if (a.ellStride > 0)
+        if (a.incStride > 0)
         {
-            // fixed stride: the incidence address needs no prefix load
-            kb = v * a.ellStride;
-            ke = kb + a.ellStride;
+            // fixed stride: the rows' addresses need no prefix load
+            nb = v * a.nbrStride, ne = nb + a.nbrStride;
+            kb = v * a.incStride, ke = kb + a.incStride;
         }
         else
         {
-            kb = a.vtp[v];
-            ke = a.vtp[v + 1];
+            int2 const p0 = a.rowPtr[v], p1 = a.rowPtr[v + 1];
+            nb = p0.x, ne = p1.x, kb = p0.y, ke = p1.y;
         }
         own = a.xm[v];
-        if (lane == 0 && K < 3)
+        if (lane == 0)
             xl = a.xtil[v]; // issued now, used after the reduction
     }
-    Block B{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     bool const nt = a.ntStream != 0;
-    // contact sweeps: the start position and the lane's contact records (slots
-    // lane, lane + L, ...), issued now; then copy the previous colour's new
-    // positions back
-    constexpr int kSlots = C ? (kMaxContacts + L - 1) / L : 1;
-    int4 crec[kSlots];
-    float4 xto = own;
+    ContactSlots<L> contact;
     if constexpr (C)
-    {
+        contact.Load(a, v, active, lane, tid, own);
+    int2 J[N];
 #pragma unroll
-        for (int j = 0; j < kSlots; ++j)
-        {
-            int const k = lane + j * L;
-            crec[j] = (active && k < kMaxContacts) ? a.contact.rec[static_cast<size_t>(v) * kMaxContacts + k]
-                                                   : make_int4(-1, -1, -1, 0);
-        }
-        if (active)
-            xto = a.xt[v];
-        int const pend = a.contact.pendBeg + tid;
-        if (pend < a.contact.pendEnd)
-            a.xm[pend] = a.contact.xb[pend];
+    for (int j = 0; j < N; ++j)
+    {
+        int const k = nb + lane + j * L;
+        J[j] = make_int2(-1, 0);
+        if (k < ne)
+            J[j] = LoadNbr(a.nbr + k, nt);
     }
-    int4 I[K];
-    float4 q0[K];
+    StarInc I[K];
 #pragma unroll
     for (int j = 0; j < K; ++j)
     {
         int const k = kb + lane + j * L;
         if (k < ke)
-        {
-            I[j] = LoadIds(a.ids + k, nt);
-            q0[j] = LoadConst(a.geo + k, nt);
-        }
-        else
-            I[j] = make_int4(-1, 0, 0, 0);
+            I[j] = LoadInc(a.inc + k, nt);
     }
-    float4 pa[K], pb[K], pc[K];
+    float4 p[N];
 #pragma unroll
-    for (int j = 0; j < K; ++j)
+    for (int j = 0; j < N; ++j)
+        if (J[j].x >= 0)
+            p[j] = SweepPosition<C>(a, J[j].x);
+    // contact terms: summed apart from the elastic block, which is damped alone;
+    // here their dependent loads overlap the neighbours'
+    Block Cb{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if constexpr (C)
+        contact.Accumulate(a, own, Cb);
+    Block B{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float gsum = 0.f;
+    auto neighbour = [&](int slot, float G, float4 const& pj) {
+        float4 const dj = make_float4(pj.x - own.x, pj.y - own.y, pj.z - own.z, 0.f);
+        B.g0 += G * dj.x, B.g1 += G * dj.y, B.g2 += G * dj.z;
+        gsum += G;
+        d[slot] = dj;
+    };
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        if (J[j].x >= 0)
+            neighbour(lane + j * L, __int_as_float(J[j].y), p[j]);
+    // neighbours beyond N per lane (vertices of unusually many neighbours)
+    for (int k = nb + lane + N * L; k < ne; k += L)
     {
-        if (I[j].x >= 0)
-        {
-            if constexpr (C)
-            {
-                pa[j] = ContactPosition(a.contact, a.xm, I[j].x);
-                pb[j] = ContactPosition(a.contact, a.xm, I[j].y);
-                pc[j] = ContactPosition(a.contact, a.xm, I[j].z);
-            }
-            else
-            {
-                pa[j] = a.xm[I[j].x];
-                pb[j] = a.xm[I[j].y];
-                pc[j] = a.xm[I[j].z];
-            }
-        }
+        int2 const q = LoadNbr(a.nbr + k, nt);
+        neighbour(k - nb, __int_as_float(q.y), SweepPosition<C>(a, q.x));
     }
+    B.h00 -= gsum, B.h11 -= gsum, B.h22 -= gsum;
+    // the offsets are exchanged within the wave, whose LDS accesses stay in order
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
     for (int j = 0; j < K; ++j)
-        if (I[j].x >= 0)
-            AccumulateElastic(q0[j], __int_as_float(I[j].w), own, pa[j], pb[j], pc[j], B);
-    // incidences beyond K per lane (vertices of unusually high degree)
+        if (kb + lane + j * L < ke)
+            AccumulateTet(I[j].A, I[j].B, d[I[j].pk & 255u], d[(I[j].pk >> 8) & 255u], d[(I[j].pk >> 16) & 255u], B);
+    // tets beyond K per lane
     for (int k = kb + lane + K * L; k < ke; k += L)
     {
-        int4 const J = LoadIds(a.ids + k, nt);
-        if (J.x < 0)
-            continue;
-        if constexpr (C)
-            AccumulateElastic(LoadConst(a.geo + k, nt), __int_as_float(J.w), own,
-                              ContactPosition(a.contact, a.xm, J.x), ContactPosition(a.contact, a.xm, J.y),
-                              ContactPosition(a.contact, a.xm, J.z), B);
-        else
-            AccumulateElastic(LoadConst(a.geo + k, nt), __int_as_float(J.w), own, a.xm[J.x], a.xm[J.y],
-                              a.xm[J.z], B);
-    }
-    if constexpr (C)
-    {
-        // contact terms (after damping, before inertia): the group's lanes take
-        // the vertex's contact slots k = lane, lane + L, ... and sum them apart
-        // from the elastic block, which is damped alone
-        ContactSweep const& cs = a.contact;
-        Block Cb{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        float3 const xo = make_float3(own.x, own.y, own.z), xt3 = make_float3(xto.x, xto.y, xto.z);
-#pragma unroll
-        for (int j = 0; j < kSlots; ++j)
-            if (crec[j].x >= 0)
-                AccumulateContact(xt3, xo, cs, a.xm, a.xt, crec[j], a.c.dt, __int_as_float(crec[j].w), cs.muF,
-                                  cs.epsv, Cb);
-        GroupSum<L>(B);
-        GroupSum<L>(Cb);
-        if (!active || lane != 0)
-            return;
-        if constexpr (K >= 3)
-            xl = a.xtil[v];
-        Damp(B, own, xto, a.c);
-        B.h00 += Cb.h00, B.h01 += Cb.h01, B.h02 += Cb.h02, B.h11 += Cb.h11, B.h12 += Cb.h12, B.h22 += Cb.h22;
-        B.g0 += Cb.g0, B.g1 += Cb.g1, B.g2 += Cb.g2;
-        float3 const dx = InertiaNewtonStep(B, own, xl, a.c);
-        cs.xb[v] = make_float4(own.x - dx.x, own.y - dx.y, own.z - dx.z, own.w);
-        return;
+        StarInc const q = LoadInc(a.inc + k, nt);
+        AccumulateTet(q.A, q.B, d[q.pk & 255u], d[(q.pk >> 8) & 255u], d[(q.pk >> 16) & 255u], B);
     }
     GroupSum<L>(B);
+    if constexpr (C)
+        GroupSum<L>(Cb);
     if (!active || lane != 0)
         return;
-    if constexpr (K >= 3)
-        xl = a.xtil[v];
-    // the start position only matters with damping: loaded here rather than
-    // held in registers through the incidence loop
-    float3 const dx = NewtonStep(B, own, xl, (a.c.kD != 0.f) ? a.xt[v] : own, a.c);
-    a.xm[v] = make_float4(own.x - dx.x, own.y - dx.y, own.z - dx.z, own.w);
+    FinishVertex<C>(a, v, B, Cb, own, xl, contact.xto);
+}
+
+// The sweep of a mesh that has a vertex of more than kMaxStarNeighbours
+// neighbours: one wave per vertex, every tet with its own three gathers and
+// gradient constants (CSR rows).
+template <bool C>
+__global__ __launch_bounds__(256) void VbdSweepWide(SweepArgs a)
+{
+    constexpr int L = 64;
+    int const tid = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    int const lane = tid & (L - 1);
+    int const v = a.vbeg + tid / L;
+    bool const active = v < a.vend;
+    int kb = 0, ke = 0;
+    float4 own = make_float4(0.f, 0.f, 0.f, 0.f);
+    float4 xl = own;
+    if (active)
+    {
+        kb = a.rowPtr[v].y, ke = a.rowPtr[v + 1].y;
+        own = a.xm[v];
+        if (lane == 0)
+            xl = a.xtil[v];
+    }
+    ContactSlots<L> contact;
+    if constexpr (C)
+        contact.Load(a, v, active, lane, tid, own);
+    Block B{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int k = kb + lane; k < ke; k += L)
+    {
+        int4 const id = a.wideIds[k];
+        float4 const geo = a.wideGeo[k];
+        float4 const pa = SweepPosition<C>(a, id.x), pb = SweepPosition<C>(a, id.y), pc = SweepPosition<C>(a, id.z);
+        float4 const da = make_float4(pa.x - own.x, pa.y - own.y, pa.z - own.z, 0.f);
+        float4 const db = make_float4(pb.x - own.x, pb.y - own.y, pb.z - own.z, 0.f);
+        float4 const dc = make_float4(pc.x - own.x, pc.y - own.y, pc.z - own.z, 0.f);
+        B.g0 += geo.x * da.x + geo.y * db.x + geo.z * dc.x;
+        B.g1 += geo.x * da.y + geo.y * db.y + geo.z * dc.y;
+        B.g2 += geo.x * da.z + geo.y * db.z + geo.z * dc.z;
+        float const dg = geo.x + geo.y + geo.z;
+        B.h00 -= dg, B.h11 -= dg, B.h22 -= dg;
+        AccumulateTet(__int_as_float(id.w), geo.w, da, db, dc, B);
+    }
+    GroupSum<L>(B);
+    Block Cb{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if constexpr (C)
+    {
+        contact.Accumulate(a, own, Cb);
+        GroupSum<L>(Cb);
+    }
+    if (!active || lane != 0)
+        return;
+    FinishVertex<C>(a, v, B, Cb, own, xl, contact.xto);
+}
+
+// Star records in fixed-stride rows from the CSR rows, one thread per
+// (vertex, entry) of the longer row; unused entries are (v, 0) and zero tets.
+[[maybe_unused]] static __global__ __launch_bounds__(256) void StarFixedStride(
+    int2 const* __restrict__ rowPtr, int2 const* __restrict__ nbr, StarInc const* __restrict__ inc,
+    int2* __restrict__ nbrE, StarInc* __restrict__ incE, int nRows, int nbrStride, int incStride)
+{
+    int const W = max(nbrStride, incStride);
+    long long const t = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+    int const v = static_cast<int>(t / W), k = static_cast<int>(t % W);
+    if (v >= nRows)
+        return;
+    int2 const p0 = rowPtr[v], p1 = rowPtr[v + 1];
+    if (k < nbrStride)
+        nbrE[static_cast<size_t>(v) * nbrStride + k] = p0.x + k < p1.x ? nbr[p0.x + k] : make_int2(v, 0);
+    if (k < incStride)
+        incE[static_cast<size_t>(v) * incStride + k] = p0.y + k < p1.y ? inc[p0.y + k] : StarInc{0u, 0.f, 0.f};
+}
+
+// Star constants of changed moduli, one thread per (vertex, entry) of the longer
+// row: a tet entry's A = w lambda kappa^2 and B = kappa (w lambda + w mu), a
+// neighbour's Gamma_j = sum of w mu gamma_k over the row's tets holding it, in
+// FP64 and in row order as the host builds them. shape[k] = (gamma_a, gamma_b,
+// gamma_c, kappa) and tet[k] the tet of CSR entry k; tgp holds (., w mu, w lambda,
+// .) in its third float4 per tet. In wide rows (wideGeo given) the tets carry
+// their own gradient constants instead.
+struct StarMaterialArgs
+{
+    int2 const* __restrict__ rowPtr;
+    int2* __restrict__ nbr;
+    StarInc* __restrict__ inc;
+    float4 const* __restrict__ shape;
+    int const* __restrict__ tet;
+    float4 const* __restrict__ tgp;
+    int4* __restrict__ wideIds;
+    float4* __restrict__ wideGeo;
+    int nRows, width;
+};
+
+[[maybe_unused]] static __global__ __launch_bounds__(256) void StarMaterial(StarMaterialArgs a)
+{
+    long long const t = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+    int const v = static_cast<int>(t / a.width), k = static_cast<int>(t % a.width);
+    if (v >= a.nRows)
+        return;
+    int2 const p0 = a.rowPtr[v], p1 = a.rowPtr[v + 1];
+    int const e = p0.y + k;
+    if (e < p1.y)
+    {
+        float4 const m = a.tgp[3 * static_cast<size_t>(a.tet[e]) + 2], s = a.shape[e];
+        double const wmu = m.y, wlam = m.z, kappa = s.w;
+        float const A = static_cast<float>(wlam * kappa * kappa), B = static_cast<float>(kappa * (wlam + wmu));
+        if (a.wideGeo)
+        {
+            a.wideIds[e].w = __float_as_int(A);
+            a.wideGeo[e] = make_float4(static_cast<float>(wmu * s.x), static_cast<float>(wmu * s.y),
+                                       static_cast<float>(wmu * s.z), B);
+        }
+        else
+            a.inc[e].A = A, a.inc[e].B = B;
+    }
+    if (a.wideGeo || p0.x + k >= p1.x)
+        return;
+    double G = 0.;
+    for (int q = p0.y; q < p1.y; ++q)
+    {
+        unsigned const pk = a.inc[q].pk, me = static_cast<unsigned>(k);
+        bool const ia = (pk & 255u) == me, ib = ((pk >> 8) & 255u) == me, ic = ((pk >> 16) & 255u) == me;
+        if (!(ia || ib || ic))
+            continue;
+        float4 const s = a.shape[q];
+        G += double(a.tgp[3 * static_cast<size_t>(a.tet[q]) + 2].y) * double(ia ? s.x : ib ? s.y : s.z);
+    }
+    a.nbr[p0.x + k].y = __float_as_int(static_cast<float>(G));
 }
 
 // Substep begin (gpu/impl/vbd/Integrator.cu:190-248; sim/vbd/Kernels.h:24-94):
