@@ -170,7 +170,8 @@ struct RolloutState
     DeviceArray<int4> coarseInfo;                             // per aggregate: (b0, n, rows begin, rows end)
     DeviceArray<long long> coarseRowOffset;                   // per aggregate: its first row in coarseF
     int coarseMaxN = 0;                                       // rows of the largest mesh's coarse operator
-    DeviceArray<double> rc, zc;                               // coarse residual and correction
+    DeviceArray<double> rc;                                   // coarse residual
+    DeviceArray<float4> zc;                                   // coarse correction, 2 per aggregate
     DeviceArray<double> scal;                                 // per-mesh solver scalars (kScalarCount x nMeshes)
     DeviceArray<int> flags;                                   // per-mesh done flags, iteration counts, live count
     DeviceArray<double> grad;                                 // d L / d log Y per tet
@@ -178,8 +179,7 @@ struct RolloutState
     // step Hessian assembled per solve as 3x3 blocks over the updated vertices:
     // the pattern and assembly sources (built once per handle: per row its
     // incidences and their tets' row positions, or, for rows too long for the
-    // row-major assembly, per block its sources), the values, the longest row,
-    // and the fused iteration's second direction buffer
+    // row-major assembly, per block its sources), the values, the longest row
     DeviceArray<int> bsrRowPtr, bsrCol, bsrBlockRow, bsrSrcPtr, bsrSrc;
     // row order of the pattern (-1: none yet, 0: the vertices' own, 1: aggregate-
     // major), the vertex of each row, and each row's mesh and aggregate, and each
@@ -191,18 +191,18 @@ struct RolloutState
     DeviceArray<float4> bsrA, bsrB;
     DeviceArray<float> bsrC;
     int bsrMaxRow = 0;
-    DeviceArray<float4> p2;
-    // row chunks of the fused iteration (begin, end, mesh, 0), mesh-major, and
-    // for each aggregate the chunks of its mesh (begin, end); chunks hold at
-    // most bsrChunkRows rows
-    DeviceArray<int4> bsrChunks;
-    DeviceArray<int2> aggChunks;
-    // per aggregate: its first kAggFirst vertices (-1 past its size) and its
-    // mesh's done flag as of the last finish kernel
-    DeviceArray<int> aggFirst, aggDone;
+    // fused solvers: the polynomial's iterate; y, r, p, H p and H z in FP64 (3 per row)
+    DeviceArray<float4> z2;
+    DeviceArray<double> yD, rD, pD, sD, wD;
+    // row chunks of the fused solvers (begin, end, mesh, 0), mesh-major, of at most
+    // bsrChunkRows rows; per aggregate (mesh, first row, end row, first of its
+    // mesh) and its mesh's chunks and aggregates
+    DeviceArray<int4> bsrChunks, aggInfo, aggRange;
+    DeviceArray<int> aggDone; // per aggregate: its mesh's done flag
     int bsrChunkRows = 0;
-    // per-chunk p . H p, per-aggregate r . z, r . r, b . b, per-coarse-row rc . zc
-    DeviceArray<double> pqPart, rzPart, rrPart, bbPart, rczcPart;
+    // per chunk r . z and z . H z; per aggregate r . r and r . z of the even and odd
+    // iterations, b . b
+    DeviceArray<double> gammaPart, deltaPart, rrPart[2], rzPart[2], bbPart;
     // Galerkin coarse operator from the blocks: coarse block k couples aggregates
     // (cbA[k], cbB[k]) and sums the fine blocks cbSrc[cbSrcPtr[k] .. cbSrcPtr[k + 1])
     DeviceArray<int> cbA, cbB, cbSrcPtr, cbSrc;

@@ -130,9 +130,13 @@ void EnsureBuffers(pbat_vbd_integrator& h)
 {
     RolloutState& R = h.rollout;
     size_t const n = static_cast<size_t>(h.nV);
-    for (auto* b : {&R.y, &R.yS, &R.bS, &R.r, &R.z, &R.p, &R.p2, &R.q, &R.rhs, &R.xbar, &R.vbar, &R.hold})
+    for (auto* b : {&R.y, &R.yS, &R.bS, &R.r, &R.z, &R.z2, &R.p, &R.q, &R.rhs, &R.xbar, &R.vbar, &R.hold})
         if (b->n != n)
             b->allocate(n);
+    static_assert(sizeof(device::Vec3d) == 3 * sizeof(double), "FP64 vectors are packed");
+    for (auto* b : {&R.yD, &R.rD, &R.pD, &R.sD, &R.wD})
+        if (b->n != 3 * n)
+            b->allocate(3 * n);
     static_assert(device::kProjMax == sizeof(R.hist) / sizeof(R.hist[0]), "history ring size");
     for (int j = 0; j < device::kProjMax; ++j)
         for (auto* b : {&R.hist[j], &R.projBasis[j], &R.projHb[j]})
@@ -184,7 +188,7 @@ void BuildCoarse(pbat_vbd_integrator& h, float4 const* xs, float dt)
     if (R.rc.n != nCoarse)
     {
         R.rc.allocate(nCoarse);
-        R.zc.allocate(nCoarse);
+        R.zc.allocate(2 * static_cast<size_t>(h.nAggregates));
     }
     if (total == 0 || h.nAggregates == 0)
         return;
@@ -240,21 +244,19 @@ void BuildCoarse(pbat_vbd_integrator& h, float4 const* xs, float dt)
         R.coarseFinal.allocate(finalBuf.size());
     PBAT_HIP(hipMemcpyAsync(R.coarseFinal.ptr, finalBuf.data(), finalBuf.size() * sizeof(int),
                             hipMemcpyHostToDevice, h.stream));
-    // per aggregate: its mesh's coarse rows (b0, n), its fine rows' range and
-    // the offset of its first row of the inverse (allocated once per size: the
-    // captured CG chunk graph holds these pointers)
+    // per aggregate: its mesh's coarse rows (b0, n) and the offset of its first row
+    // of the inverse (allocated once per size: the captured CG chunk graph holds
+    // these pointers)
     {
         std::vector<int4> info(static_cast<size_t>(h.nAggregates));
         std::vector<long long> rowOff(static_cast<size_t>(h.nAggregates));
-        std::vector<int> aggPtr(static_cast<size_t>(h.nAggregates) + 1);
-        PBAT_HIP(hipMemcpy(aggPtr.data(), h.aggVertPtr.ptr, aggPtr.size() * sizeof(int), hipMemcpyDeviceToHost));
         for (int m = 0; m < nM; ++m)
         {
             int const b0 = device::kCoarseDofs * h.aggBegin[m];
             int const n = device::kCoarseDofs * (h.aggBegin[m + 1] - h.aggBegin[m]);
             for (int g = h.aggBegin[m]; g < h.aggBegin[m + 1]; ++g)
             {
-                info[g] = make_int4(b0, n, aggPtr[g], aggPtr[g + 1]);
+                info[g] = make_int4(b0, n, 0, 0);
                 rowOff[g] = static_cast<long long>(h.coarseOffset[m]) +
                             static_cast<long long>(device::kCoarseDofs * g - b0) * n;
             }
@@ -541,10 +543,10 @@ void BuildBsrPattern(pbat_vbd_integrator& h, bool aggregateOrder)
     for (size_t k = 0; k < nBlocks; ++k)
         colAgg[k] = aggOfRow[col[k]];
     // row chunks: every run of rows of one mesh (and, in the vertices' own order,
-    // one colour) cut into chunks of at most 256 / L rows, then ordered
+    // one colour) cut into chunks of at most kChunkThreads / L rows, then ordered
     // mesh-major (stable: colour, then row order)
     int const nM = h.nMeshes;
-    int const chunkRows = 256 / BsrLanes(h);
+    int const chunkRows = device::kChunkThreads / BsrLanes(h);
     struct Chunk
     {
         int mesh, begin, end;
@@ -581,25 +583,23 @@ void BuildBsrPattern(pbat_vbd_integrator& h, bool aggregateOrder)
     for (int m = 0; m < nM; ++m)
         meshChunk[m + 1] += meshChunk[m];
     R.bsrChunks.upload(chunkRange, h.stream);
-    std::vector<int2> aggChunk(static_cast<size_t>(std::max(h.nAggregates, 1)), make_int2(0, 0));
+    size_t const nAggAlloc = static_cast<size_t>(std::max(h.nAggregates, 1));
+    std::vector<int4> aggInfo(nAggAlloc, make_int4(0, 0, 0, 0)), aggRange(nAggAlloc, make_int4(0, 0, 0, 0));
     for (int m = 0; m < nM; ++m)
         for (int g = h.aggBegin[m]; g < h.aggBegin[m + 1]; ++g)
-            aggChunk[g] = make_int2(meshChunk[m], meshChunk[m + 1]);
-    R.aggChunks.upload(aggChunk, h.stream);
-    // each aggregate's first rows, one per AggUpdate thread
-    {
-        std::vector<int> first(static_cast<size_t>(std::max(h.nAggregates, 1)) * device::kAggFirst, -1);
-        for (int g = 0; g < h.nAggregates; ++g)
-            for (int k = aggPtr[g]; k < std::min(aggPtr[g + 1], aggPtr[g] + device::kAggFirst); ++k)
-                first[static_cast<size_t>(g) * device::kAggFirst + (k - aggPtr[g])] = aggRows[k];
-        R.aggFirst.upload(first, h.stream);
-        R.aggDone.allocate(static_cast<size_t>(std::max(h.nAggregates, 1)));
-    }
+        {
+            // aggregate-major rows: aggregate g's are its range of the CSR itself
+            aggInfo[g] = make_int4(m, aggPtr[g], aggPtr[g + 1], g == h.aggBegin[m] ? 1 : 0);
+            aggRange[g] = make_int4(meshChunk[m], meshChunk[m + 1], h.aggBegin[m], h.aggBegin[m + 1]);
+        }
+    R.aggInfo.upload(aggInfo, h.stream);
+    R.aggRange.upload(aggRange, h.stream);
+    R.aggDone.allocate(nAggAlloc);
     R.bsrChunkRows = chunkRows;
-    R.pqPart.allocate(std::max<size_t>(chunks.size(), 1));
-    size_t const nAggAlloc = static_cast<size_t>(std::max(h.nAggregates, 1));
-    R.rzPart.allocate(nAggAlloc), R.rrPart.allocate(nAggAlloc), R.bbPart.allocate(nAggAlloc);
-    R.rczcPart.allocate(static_cast<size_t>(device::kCoarseDofs) * nAggAlloc);
+    for (auto* b : {&R.gammaPart, &R.deltaPart})
+        b->allocate(std::max<size_t>(chunks.size(), 1));
+    for (auto* b : {&R.rrPart[0], &R.rrPart[1], &R.rzPart[0], &R.rzPart[1], &R.bbPart})
+        b->allocate(nAggAlloc);
 
     // coarse blocks: the fine blocks grouped by (aggregate of the row, aggregate
     // of the column), ascending within each group. Built per row aggregate, in
@@ -796,55 +796,73 @@ void BsrPass(pbat_vbd_integrator& h, device::BsrArgs a, int vbeg, int vend)
     }
 }
 
-template <int L, int K>
-void LaunchDirectionLK(pbat_vbd_integrator& h, device::BsrArgs a)
+// Launches of the fused solvers (vbd_hessian_kernels.hpp).
+template <int L>
+void LaunchCoarsePolyL(pbat_vbd_integrator& h, device::FusedArgs a, int grid)
 {
-    RolloutState& R = h.rollout;
-    int const nChunks = static_cast<int>(R.bsrChunks.n);
-    int64_t grid64 = std::max(nChunks, 1);
+    // 64-column chunks per wave of the largest mesh, rounded up to a kernel's
+    int const perWave = ((h.rollout.coarseMaxN + 63) / 64 + device::kCoarseWaves - 1) / device::kCoarseWaves;
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(a.coarseBlocks + grid), dim3(256), 0, h.stream, a);
+    };
+    if (perWave <= 1)
+        launch(device::CoarsePoly<L, 1>);
+    else if (perWave <= 2)
+        launch(device::CoarsePoly<L, 2>);
+    else if (perWave <= 4)
+        launch(device::CoarsePoly<L, 4>);
+    else // several passes beyond 2,304 rows
+        launch(device::CoarsePoly<L, 9>);
+}
+
+enum class FusedPass
+{
+    kCoarsePoly,
+    kPolyLast,
+    kPolyProduct,
+    kResidual
+};
+
+template <int L>
+void LaunchFusedL(pbat_vbd_integrator& h, device::FusedArgs a, FusedPass pass)
+{
+    int64_t grid64 = pass == FusedPass::kCoarsePoly ? 2 * int64_t(a.nChunks) : a.nChunks;
     a.xcdChunk = 0;
     if (h.xcdRemap && grid64 >= 16)
     {
         grid64 = (grid64 + 7) / 8 * 8;
         a.xcdChunk = static_cast<int>(grid64 / 8);
     }
-    hipLaunchKernelGGL((device::BsrDirection<L, K>), dim3(static_cast<int>(grid64)), dim3(256), 0, h.stream, a,
-                       static_cast<int4 const*>(R.bsrChunks.ptr), nChunks, R.pqPart.ptr);
+    int const grid = static_cast<int>(grid64);
+    a.coarseBlocks = (a.nAgg + 7) / 8 * 8; // keeps the row workgroups' XCD order
+    if (pass == FusedPass::kCoarsePoly)
+        LaunchCoarsePolyL<L>(h, a, grid);
+    else if (pass == FusedPass::kPolyLast)
+        hipLaunchKernelGGL((device::BsrPoly<L, device::PolyMode::kPolyLast>), dim3(grid),
+                           dim3(device::kChunkThreads), 0, h.stream, a);
+    else if (pass == FusedPass::kPolyProduct)
+        hipLaunchKernelGGL((device::BsrPoly<L, device::PolyMode::kPolyProduct>), dim3(grid),
+                           dim3(device::kChunkThreads), 0, h.stream, a);
+    else
+        hipLaunchKernelGGL((device::BsrPoly<L, device::PolyMode::kResidual>), dim3(grid),
+                           dim3(device::kChunkThreads), 0, h.stream, a);
 }
 
-template <int L>
-void LaunchDirectionL(pbat_vbd_integrator& h, device::BsrArgs const& a)
+void LaunchFused(pbat_vbd_integrator& h, device::FusedArgs const& a, FusedPass pass)
 {
-    switch (BsrPerLane(h))
-    {
-        case 1: LaunchDirectionLK<L, 1>(h, a); break;
-        case 2: LaunchDirectionLK<L, 2>(h, a); break;
-        case 3: LaunchDirectionLK<L, 3>(h, a); break;
-        default: LaunchDirectionLK<L, 4>(h, a); break;
-    }
-}
-
-// The fused iteration's direction product over the row chunks (BsrDirection):
-// a.y = p (written), a.out = H p, a.z, a.pOld as BsrArgs describes them.
-void DirectionPass(pbat_vbd_integrator& h, device::BsrArgs a)
-{
-    RolloutState& R = h.rollout;
-    if (R.bsrChunks.n == 0)
+    if (a.nChunks == 0)
         return;
-    if (256 / BsrLanes(h) != R.bsrChunkRows)
+    if (device::kChunkThreads / BsrLanes(h) != h.rollout.bsrChunkRows)
         Fail(PBAT_VBD_ERROR_INVALID_ARGUMENT, "row chunks built for another lane count");
-    a.rowPtr = R.bsrRowPtr.ptr, a.col = R.bsrCol.ptr;
-    a.va = R.bsrA.ptr, a.vb = R.bsrB.ptr, a.vc = R.bsrC.ptr;
-    a.meshOf = R.meshOfRow.ptr;
     switch (BsrLanes(h))
     {
-        case 1: LaunchDirectionL<1>(h, a); break;
-        case 2: LaunchDirectionL<2>(h, a); break;
-        case 4: LaunchDirectionL<4>(h, a); break;
-        case 8: LaunchDirectionL<8>(h, a); break;
-        case 16: LaunchDirectionL<16>(h, a); break;
-        case 32: LaunchDirectionL<32>(h, a); break;
-        default: LaunchDirectionL<64>(h, a); break;
+        case 1: LaunchFusedL<1>(h, a, pass); break;
+        case 2: LaunchFusedL<2>(h, a, pass); break;
+        case 4: LaunchFusedL<4>(h, a, pass); break;
+        case 8: LaunchFusedL<8>(h, a, pass); break;
+        case 16: LaunchFusedL<16>(h, a, pass); break;
+        case 32: LaunchFusedL<32>(h, a, pass); break;
+        default: LaunchFusedL<64>(h, a, pass); break;
     }
 }
 
@@ -950,19 +968,15 @@ SolveResult ReadResult(pbat_vbd_integrator& h)
 // cfg.check_every iterations, and the iteration kernels do nothing once every
 // mesh has converged.
 //
-// Block Jacobi and two-level preconditioners (the fused iteration), per iteration:
-//   (1) per row chunk: p = z + beta p_old formed on the fly, q = H p, the
-//       chunk's p . q;
-//   (2) one workgroup per aggregate: alpha = rz / pq from its mesh's chunk sums,
-//       y += alpha p, r -= alpha q, z = D^-1 r, the aggregate's r . z, r . r and
-//       restriction rc = Z^T r;
-//   (3) two-level, one workgroup per aggregate: its rows of zc = (Z^T H Z)^-1 rc,
-//       each coarse row's rc . zc, and z += Z zc on its rows;
-//   (4) one workgroup: per mesh, r . z = r . D^-1 r + rc . zc and r . r summed
-//       over its partials, stopping test, beta.
-// No atomics: every sum is taken in a fixed order, so a solve gives the same
-// bits on every run, and a mesh gives the same bits alone or in a batch (its
-// row chunks, aggregates and coarse rows are the same).
+// Block Jacobi and two-level preconditioners (the fused iteration,
+// vbd_hessian_kernels.hpp), per iteration:
+//   (1) CgUpdate1, one workgroup per aggregate: its mesh's sums, stopping test,
+//       alpha and beta, p, s, y, r, z (two-level: z1) and rc = Z^T r;
+//   (2) two-level, CoarsePoly: zc = (Z^T H Z)^-1 rc next to z2;
+//   (3) two-level, BsrPoly: z = z3 + Z zc, r . z;
+//   (4) BsrPoly: w = H z, z . w.
+// 32^3 workload, per iteration: 27.4 us in four launches with the classical
+// recurrences and the coarse correction of block Jacobi alone.
 // The symmetric Gauss-Seidel preconditioner keeps the four-launch iteration
 //   q = H p and p . q; y, r update with z = 0; a forward and a reverse coloured
 //   Gauss-Seidel pass for z with r . z; one workgroup: scalars; p = z + beta p.
@@ -1070,72 +1084,69 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
         PBAT_HIP(hipGetLastError());
         return out;
     }
-    auto aggUpdate = [&](int init, float4 const* p) {
-        device::AggUpdateArgs u{};
-        u.aggPtr = h.aggVertPtr.ptr, u.aggVerts = R.aggRows.ptr, u.aggMesh = h.aggMesh.ptr;
-        u.y = y, u.r = R.r.ptr, u.z = R.z.ptr, u.p = p, u.q = R.q.ptr, u.b = b, u.dinv = R.dinv.ptr;
-        u.rc = twoLevel ? R.rc.ptr : nullptr;
-        u.coarseD = R.coarseD.ptr;
-        u.pqPart = R.pqPart.ptr, u.aggChunks = R.aggChunks.ptr;
-        u.aggFirst = R.aggFirst.ptr, u.aggDone = R.aggDone.ptr;
-        u.rzPart = R.rzPart.ptr, u.rrPart = R.rrPart.ptr, u.bbPart = R.bbPart.ptr;
-        u.cg = cg, u.init = init;
-        if (h.nAggregates > 0)
-            hipLaunchKernelGGL(device::AggUpdate, dim3(h.nAggregates), dim3(128), 0, h.stream, u);
+    device::FusedArgs fa{};
+    fa.rowPtr = R.bsrRowPtr.ptr, fa.col = R.bsrCol.ptr, fa.va = R.bsrA.ptr, fa.vb = R.bsrB.ptr, fa.vc = R.bsrC.ptr;
+    auto vec = [](DeviceArray<double> const& v) { return reinterpret_cast<device::Vec3d*>(v.ptr); };
+    fa.dinv = R.dinv.ptr, fa.y = vec(R.yD), fa.r = vec(R.rD), fa.p = vec(R.pD), fa.s = vec(R.sD);
+    fa.z = R.z.ptr, fa.z2 = R.z2.ptr, fa.w = vec(R.wD), fa.y0 = y, fa.b = b, fa.chunks = R.bsrChunks.ptr, fa.gammaPart = R.gammaPart.ptr;
+    fa.deltaPart = R.deltaPart.ptr, fa.nChunks = static_cast<int>(R.bsrChunks.n);
+    fa.aggInfo = R.aggInfo.ptr;
+    for (int k = 0; k < 2; ++k)
+        fa.rrPart[k] = R.rrPart[k].ptr, fa.rzPart[k] = R.rzPart[k].ptr;
+    fa.aggDone = R.aggDone.ptr;
+    fa.bbPart = R.bbPart.ptr, fa.nAgg = h.nAggregates, fa.rc = R.rc.ptr, fa.zc = R.zc.ptr;
+    fa.coarseD = R.coarseD.ptr, fa.aggOfRow = R.aggOfRow.ptr, fa.coarseF = R.coarseF.ptr;
+    fa.coarseInfo = R.coarseInfo.ptr, fa.coarseRowOffset = R.coarseRowOffset.ptr;
+    fa.q = device::MakeCheby(), fa.cg = cg;
+    auto precondition = [&] {
+        if (twoLevel)
+        {
+            LaunchFused(h, fa, FusedPass::kCoarsePoly);
+            LaunchFused(h, fa, FusedPass::kPolyLast);
+        }
+        LaunchFused(h, fa, FusedPass::kPolyProduct);
     };
-    auto coarseRows = [&](int first) {
-        device::CoarseApplyArgs ca{};
-        ca.coarseF = R.coarseF.ptr, ca.rc = R.rc.ptr, ca.zc = R.zc.ptr, ca.rczcPart = R.rczcPart.ptr;
-        ca.info = R.coarseInfo.ptr, ca.rowOffset = R.coarseRowOffset.ptr, ca.aggDone = R.aggDone.ptr;
-        ca.coarseD = R.coarseD.ptr, ca.z = R.z.ptr;
-        // 64-column chunks per wave of the largest mesh, rounded up to a kernel's
-        int const perWave = ((R.coarseMaxN + 63) / 64 + device::kCoarseWaves - 1) / device::kCoarseWaves;
-        dim3 const grid(h.nAggregates), block(64 * device::kCoarseWaves);
-        if (perWave <= 1)
-            hipLaunchKernelGGL(device::CoarseApplyRows<1>, grid, block, 0, h.stream, ca, first);
-        else if (perWave <= 2)
-            hipLaunchKernelGGL(device::CoarseApplyRows<2>, grid, block, 0, h.stream, ca, first);
-        else if (perWave <= 3)
-            hipLaunchKernelGGL(device::CoarseApplyRows<3>, grid, block, 0, h.stream, ca, first);
-        else if (perWave <= 4)
-            hipLaunchKernelGGL(device::CoarseApplyRows<4>, grid, block, 0, h.stream, ca, first);
-        else if (perWave <= 6)
-            hipLaunchKernelGGL(device::CoarseApplyRows<6>, grid, block, 0, h.stream, ca, first);
-        else if (perWave <= 9)
-            hipLaunchKernelGGL(device::CoarseApplyRows<9>, grid, block, 0, h.stream, ca, first);
-        else // several passes beyond 3,072 rows
-            hipLaunchKernelGGL(device::CoarseApplyRows<12>, grid, block, 0, h.stream, ca, first);
+    auto update = [&](int k) {
+        if (h.nAggregates == 0)
+            return;
+        int const now = k & 1, next = now ^ 1;
+        auto plain = [&](device::PlainArray x) { return cg.P + static_cast<size_t>(x) * nM; };
+        device::CgUpdateArgs u{};
+        u.aggInfo = R.aggInfo.ptr, u.aggRange = R.aggRange.ptr, u.aggDone = R.aggDone.ptr;
+        u.gammaOld = plain(now ? device::kGamma1 : device::kGamma);
+        u.alphaOld = plain(now ? device::kAlpha1 : device::kAlpha);
+        u.gammaNew = plain(next ? device::kGamma1 : device::kGamma);
+        u.alphaNew = plain(next ? device::kAlpha1 : device::kAlpha);
+        u.bb = plain(device::kBb), u.rrLast = plain(device::kRrLast);
+        u.gammaPart = twoLevel ? R.gammaPart.ptr : R.rzPart[now].ptr, u.deltaPart = R.deltaPart.ptr;
+        u.rrOld = R.rrPart[now].ptr, u.rrNew = R.rrPart[next].ptr, u.rzNew = R.rzPart[next].ptr;
+        u.w = fa.w, u.z = fa.z, u.p = fa.p, u.s = fa.s, u.y = fa.y, u.r = fa.r;
+        u.dinv = fa.dinv, u.coarseD = fa.coarseD, u.rc = fa.rc, u.tol2 = cg.tol2, u.invTheta = fa.q.invTheta;
+        u.done = cg.F + device::kDone * nM, u.iters = cg.F + device::kIters * nM, u.doneOut = fa.doneOut;
+        if (twoLevel)
+            hipLaunchKernelGGL(device::CgUpdate1<true>, dim3(h.nAggregates), dim3(128), 0, h.stream, u);
+        else
+            hipLaunchKernelGGL(device::CgUpdate1<false>, dim3(h.nAggregates), dim3(128), 0, h.stream, u);
     };
-    auto finish = [&](int first) {
-        device::CgFinishArgs f{};
-        f.cg = cg, f.meshAggBegin = h.meshAggBegin.ptr;
-        f.rzPart = R.rzPart.ptr, f.rrPart = R.rrPart.ptr, f.bbPart = R.bbPart.ptr;
-        f.rczcPart = twoLevel ? R.rczcPart.ptr : nullptr;
-        f.doneOut = R.doneDev, f.aggDone = R.aggDone.ptr;
-        hipLaunchKernelGGL(device::CgFinish, dim3(nM), dim3(256), 0, h.stream, f, first);
+    auto meshScalars = [&](int start, int parity) {
+        hipLaunchKernelGGL(device::CgMesh, dim3(nM), dim3(64), 0, h.stream, fa,
+                           static_cast<int const*>(h.meshAggBegin.ptr), start, parity);
     };
     std::function<void(int)> iteration;
     if (fused)
     {
         EnsureDoneHost(h);
-        // r = b - H y, z = D^-1 r, (rc, zc); p_old = 0 for the first direction
-        product(y, R.q.ptr, nullptr);
-        aggUpdate(1, nullptr);
-        if (twoLevel && h.nAggregates > 0)
-            coarseRows(1);
-        finish(1);
-        Zero4(h, R.p.ptr, nV);
+        fa.doneOut = R.doneDev;
+        LaunchFused(h, fa, FusedPass::kResidual);
+        if (h.nAggregates > 0 && twoLevel)
+            hipLaunchKernelGGL(device::CgStartRows<true>, dim3(h.nAggregates), dim3(128), 0, h.stream, fa);
+        else if (h.nAggregates > 0)
+            hipLaunchKernelGGL(device::CgStartRows<false>, dim3(h.nAggregates), dim3(128), 0, h.stream, fa);
+        meshScalars(1, 0);
+        precondition();
         iteration = [&](int k) {
-            float4* const pOld = (k & 1) ? R.p2.ptr : R.p.ptr;
-            float4* const pNew = (k & 1) ? R.p.ptr : R.p2.ptr;
-            device::BsrArgs a{};
-            a.y = pNew, a.out = R.q.ptr, a.z = R.z.ptr, a.pOld = pOld;
-            a.cg = cg;
-            DirectionPass(h, a);
-            aggUpdate(0, pNew);
-            if (twoLevel && h.nAggregates > 0)
-                coarseRows(0);
-            finish(0);
+            update(k);
+            precondition();
         };
     }
     else
@@ -1159,7 +1170,7 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
                                static_cast<float4 const*>(R.z.ptr), h.meshOf.ptr, n, cg);
         };
     }
-    bool const graph = h.useGraph && fixedBuffers;
+    bool const graph = h.useGraph && fixedBuffers && n > 0;
     if (graph)
     {
         std::vector<double> const key{double(dt),        double(cfg.solver), double(check),       cg.tol2,
@@ -1168,15 +1179,15 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
         // every device address the captured kernels take: a buffer reallocated at
         // another address forces a new capture
         std::vector<void const*> const ptrs{
-            R.y.ptr,           R.r.ptr,         R.z.ptr,       R.p.ptr,          R.p2.ptr,        R.q.ptr,
-            R.rhs.ptr,         R.hold.ptr,      R.dinv.ptr,    R.scal.ptr,       R.flags.ptr,     R.coarse[0].ptr,
-            R.coarse[1].ptr,   R.coarseF.ptr,     R.rc.ptr,    R.zc.ptr,         R.bsrRowPtr.ptr, R.bsrCol.ptr,
-            R.bsrA.ptr,        R.bsrB.ptr,      R.bsrC.ptr,    h.meshOf.ptr,     h.aggOf.ptr,     h.aggVertPtr.ptr,
-            h.aggVerts.ptr,    h.aggMesh.ptr,   h.meshAggBegin.ptr, R.bsrChunks.ptr, R.aggChunks.ptr,
-            R.pqPart.ptr,      R.rzPart.ptr,    R.rrPart.ptr,  R.bbPart.ptr,     R.rczcPart.ptr,
-            R.doneDev,       R.aggFirst.ptr, R.aggDone.ptr,    R.yS.ptr,        R.bS.ptr,
-            R.aggRows.ptr,     R.aggOfRow.ptr,  R.meshOfRow.ptr, R.coarseD.ptr, R.coarseInfo.ptr,
-            R.coarseRowOffset.ptr};
+            R.y.ptr,         R.r.ptr,           R.z.ptr,           R.z2.ptr,         R.p.ptr,
+            R.yD.ptr,        R.rD.ptr,          R.pD.ptr,          R.sD.ptr,         R.wD.ptr,
+            R.aggDone.ptr,           R.rhs.ptr,         R.hold.ptr,       R.dinv.ptr,
+            R.scal.ptr,      R.flags.ptr,       R.coarseF.ptr,     R.rc.ptr,         R.zc.ptr,
+            R.bsrRowPtr.ptr, R.bsrCol.ptr,      R.bsrA.ptr,        R.bsrB.ptr,       R.bsrC.ptr,
+            h.meshOf.ptr,    R.meshOfRow.ptr,   R.aggOfRow.ptr,    R.bsrChunks.ptr,  R.aggInfo.ptr,
+            R.aggRange.ptr,  R.gammaPart.ptr,   R.deltaPart.ptr,   R.rrPart[0].ptr,  R.rrPart[1].ptr,
+            R.rzPart[0].ptr, R.rzPart[1].ptr,   R.bbPart.ptr,      R.doneDev,        R.yS.ptr,
+            R.bS.ptr,        R.coarseD.ptr,     R.coarseInfo.ptr,  R.coarseRowOffset.ptr};
         if (!R.cgExec || R.cgKey != key || R.cgPtrs != ptrs)
         {
             R.ResetGraph();
@@ -1225,9 +1236,12 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
                 break;
         }
     }
+    if (fused)
+        meshScalars(0, it & 1);
     if (fused && n > 0)
-        hipLaunchKernelGGL(device::ScatterRows, dim3(gridN), dim3(256), 0, h.stream, yIn,
-                           static_cast<float4 const*>(y), static_cast<int const*>(R.rowVertex.ptr), n);
+        hipLaunchKernelGGL(device::CgSolution, dim3(gridN), dim3(256), 0, h.stream,
+                           static_cast<device::Vec3d const*>(fa.y), R.yS.ptr, yIn,
+                           static_cast<int const*>(R.rowVertex.ptr), n);
     PBAT_HIP(hipGetLastError());
     if (statsOut)
     {

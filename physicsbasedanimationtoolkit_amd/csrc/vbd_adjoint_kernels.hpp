@@ -95,7 +95,11 @@ enum PlainArray : int
     kBeta = 1,   // CG direction coefficient
     kRrLast = 2, // r . r at the last completed iteration
     kBb = 3,     // b . b
-    kPlainCount = 4
+    kGamma = 4,  // fused solvers: r . z and alpha of the previous iteration, for even
+    kAlpha = 5,  // iterations (4, 5) and odd ones (6, 7)
+    kGamma1 = 6,
+    kAlpha1 = 7,
+    kPlainCount = 8
 };
 // Accumulated dot products: each (array, mesh) is spread over kSpread atomic
 // targets kSlotStride doubles (128 B) apart, so that thousands of workgroups

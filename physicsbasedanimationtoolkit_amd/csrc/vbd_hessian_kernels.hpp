@@ -21,6 +21,8 @@
 
 #include "vbd_adjoint_kernels.hpp"
 
+#include <type_traits>
+
 namespace pbat_vbd::device {
 
 // Values of the block-sparse step Hessian, structure of arrays per block:
@@ -366,9 +368,7 @@ enum class BsrMode : int
     kProduct = 0,        // out = H y
     kProductDot = 1,     // out = H y, acc[mesh] += y . H y
     kGaussSeidel = 2,    // rows of one colour: y_i += D_i^-1 (b_i - (H y)_i)
-    kGaussSeidelDot = 3, // same, then acc[mesh] += b_i . y_i
-    kDirection = 4       // p = z + beta p_old formed on the fly (written to y);
-                         // out = H p, p . H p per row chunk (BsrDirection)
+    kGaussSeidelDot = 3  // same, then acc[mesh] += b_i . y_i
 };
 
 struct BsrArgs
@@ -383,10 +383,6 @@ struct BsrArgs
     float4* __restrict__ out;        // product
     float4 const* __restrict__ dinv; // inverse diagonal blocks (Gauss-Seidel)
     int const* __restrict__ meshOf;
-    // kDirection: p_j = z_j + beta p_old_j of mesh m (p_old_j when m is done); z
-    // holds the whole preconditioned residual, its coarse part included
-    float4 const* __restrict__ z;
-    float4 const* __restrict__ pOld;
     CgState cg;
     double* __restrict__ acc; // accumulators (dot modes), array accArray
     int accArray;
@@ -394,23 +390,12 @@ struct BsrArgs
     int xcdChunk;
 };
 
-// p_j = z_j + beta p_old_j (p_old_j when the mesh has converged)
-__device__ __forceinline__ float4 DirectionVector(BsrArgs const& a, int j, float beta, bool frozen)
-{
-    float4 const po = a.pOld[j];
-    if (frozen)
-        return po;
-    float4 const zj = a.z[j];
-    return make_float4(zj.x + beta * po.x, zj.y + beta * po.y, zj.z + beta * po.z, 0.f);
-}
-
 // (H v)_row over blocks [kb, ke) of one row: lane l of the row's L lanes takes
 // blocks l, l + L, ..., the first K of them loaded together before
 // accumulating; the group sum leaves the product in every lane of the group.
-template <int L, int K, BsrMode M>
-__device__ __forceinline__ float3 RowProduct(BsrArgs const& a, int kb, int ke, int lane, float beta, bool frozen)
+template <int L, int K>
+__device__ __forceinline__ float3 RowProduct(BsrArgs const& a, int kb, int ke, int lane)
 {
-    constexpr bool kDir = M == BsrMode::kDirection;
     float hx = 0.f, hy = 0.f, hz = 0.f;
     int cj[K];
     float4 A[K], B[K];
@@ -432,12 +417,7 @@ __device__ __forceinline__ float3 RowProduct(BsrArgs const& a, int kb, int ke, i
 #pragma unroll
     for (int u = 0; u < K; ++u)
         if (cj[u] >= 0)
-        {
-            if constexpr (kDir)
-                P[u] = DirectionVector(a, cj[u], beta, frozen);
-            else
-                P[u] = a.y[cj[u]];
-        }
+            P[u] = a.y[cj[u]];
 #pragma unroll
     for (int u = 0; u < K; ++u)
         if (cj[u] >= 0)
@@ -450,11 +430,7 @@ __device__ __forceinline__ float3 RowProduct(BsrArgs const& a, int kb, int ke, i
     {
         float4 const Ak = a.va[k], Bk = a.vb[k];
         float const Ck = a.vc[k];
-        float4 Pk;
-        if constexpr (kDir)
-            Pk = DirectionVector(a, a.col[k], beta, frozen);
-        else
-            Pk = a.y[a.col[k]];
+        float4 const Pk = a.y[a.col[k]];
         hx += Ak.x * Pk.x + Ak.y * Pk.y + Ak.z * Pk.z;
         hy += Ak.w * Pk.x + Bk.x * Pk.y + Bk.y * Pk.z;
         hz += Bk.z * Pk.x + Bk.w * Pk.y + Ck * Pk.z;
@@ -466,7 +442,6 @@ __device__ __forceinline__ float3 RowProduct(BsrArgs const& a, int kb, int ke, i
 template <int L, int K, BsrMode M>
 __global__ __launch_bounds__(256) void BsrKernel(BsrArgs a)
 {
-    static_assert(M != BsrMode::kDirection, "the direction product runs over row chunks (BsrDirection)");
     constexpr bool kGS = M == BsrMode::kGaussSeidel || M == BsrMode::kGaussSeidelDot;
     constexpr bool kDot = M == BsrMode::kGaussSeidelDot || M == BsrMode::kProductDot;
     int block = static_cast<int>(blockIdx.x);
@@ -482,7 +457,7 @@ __global__ __launch_bounds__(256) void BsrKernel(BsrArgs a)
         kb = a.rowPtr[row];
         ke = a.rowPtr[row + 1];
     }
-    float3 const h = RowProduct<L, K, M>(a, kb, ke, lane, 0.f, false);
+    float3 const h = RowProduct<L, K>(a, kb, ke, lane);
     bool const leader = active && lane == 0;
     double dot = 0.;
     if (leader)
@@ -512,75 +487,83 @@ __global__ __launch_bounds__(256) void BsrKernel(BsrArgs a)
         BlockAccumulate(dot, leader ? a.meshOf[row] : -1, a.acc, a.accArray, a.cg.nM);
 }
 
-// Row chunks of the fused CG iteration: each (mesh, colour) run of rows is cut
-// into chunks of at most 256 / L rows, numbered mesh-major, so the chunks of
-// a mesh are consecutive (aggChunks holds each aggregate's mesh's range) and every chunk holds
-// rows of one mesh. A chunk's sums depend only on its own rows, so a mesh gets
-// the same partial sums whether it is stepped alone or in a batch.
+// ---- fused conjugate gradients -----------------------------------------------
+// Preconditioned CG in the one-reduction form of Chronopoulos and Gear: with
+// z = M^-1 r and w = H z, delta = z . w and gamma = r . z give
+//   beta = gamma / gamma_old,  alpha = gamma / (delta - beta gamma / alpha_old),
+//   p = z + beta p,  s = w + beta s (= H p),  y += alpha p,  r -= alpha s,
+// so the product needs no direction and an iteration has one point where every
+// sum of the mesh is needed (CgUpdate1), at the head of a launch that has to wait
+// for the product anyway. The product reads one vector per block instead of two
+// (z and p_old), and no launch of its own takes the scalars (32^3: 4.6 us of 27).
 //
-// One workgroup per chunk (XCD-aware order when xcdChunk > 0): the direction
-// p = z + beta p_old of each of its rows is formed on the fly for every block
-// (z includes the coarse correction), written to y, q = H p to out, and the chunk's p . q, summed over its
-// rows in order, to pqPart[chunk]. Chunks of a converged mesh do nothing.
-template <int L, int K>
-__global__ __launch_bounds__(256) void BsrDirection(BsrArgs a, int4 const* __restrict__ chunks, int nChunks,
-                                                    double* __restrict__ pqPart)
+// Two-level: M^-1 = q(D^-1 H) D^-1 + Z (Z^T H Z)^-1 Z^T, q the degree-2 Chebyshev
+// polynomial for the spectrum [kChebyMax / kChebyRatio, kChebyMax] of D^-1 H (the
+// smoother of the modes the coarse space leaves). kChebyMax = 4 bounds the
+// spectrum when the tets' Hessians are positive semi-definite (each couples 4
+// vertices); above it q lambda = 1 - T_3 stays positive (T_3 is odd), so M^-1 stays
+// positive definite where indefinite tets push the spectrum past it. It halves the
+// iterations for two more products each (24^3: 241 -> 120 iterations from zero),
+// and one of them shares its launch with the coarse product.
+// Per iteration: CgUpdate1 (y, r, z1 = D^-1 r / theta, rc = Z^T r); CoarsePoly
+// (coarse product, z2); BsrPoly<kPolyLast> (z3 + Z zc, r . z); BsrPoly<kPolyProduct>
+// (w, z . w).
+//
+// Row chunks: each run of rows of one mesh (and one colour) is cut into chunks of
+// at most kChunkThreads / L rows, numbered mesh-major, so the chunks of a mesh are
+// consecutive and every chunk holds rows of one mesh. A chunk's sums depend only
+// on its own rows, every sum is taken in a fixed order and no atomics are used, so
+// a solve gives the same bits on every run and a mesh gives the same bits alone or
+// in a batch.
+constexpr int kChunkThreads = 512;
+constexpr double kChebyMax = 4., kChebyRatio = 45.;
+
+struct ChebyConstants
 {
-    constexpr int R = 256 / L;
-    int const nM = a.cg.nM;
-    int w = static_cast<int>(blockIdx.x);
-    if (a.xcdChunk > 0)
-        w = (w & 7) * a.xcdChunk + (w >> 3);
-    if (w >= nChunks)
-        return; // padding of the XCD order
-    // the chunk (rows and mesh), then its mesh's done flag and beta together
-    // with the row's extent
-    int4 const ch = chunks[w];
-    int const m = ch.z;
-    constexpr bool frozen = false;
-    int const r = static_cast<int>(threadIdx.x) / L, lane = static_cast<int>(threadIdx.x) & (L - 1);
-    int const row = ch.x + r;
-    bool const active = row < ch.y;
-    int const done = a.cg.F[kDone * nM + m];
-    float const beta = static_cast<float>(a.cg.P[kBeta * nM + m]);
-    int kb = 0, ke = 0;
-    if (active)
-    {
-        kb = a.rowPtr[row];
-        ke = a.rowPtr[row + 1];
-    }
-    if (done != 0)
-        return; // the chunk's mesh has converged: its vectors no longer change
-    float4 pr = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (active && lane == 0) // the row's own direction, in flight during the product
-        pr = DirectionVector(a, row, beta, frozen);
-    float3 const h = RowProduct<L, K, BsrMode::kDirection>(a, kb, ke, lane, beta, frozen);
-    __shared__ double sdot[R];
-    if (lane == 0)
-    {
-        double dot = 0.;
-        if (active)
-        {
-            a.y[row] = pr; // the direction of this iteration (the p_old of the next)
-            a.out[row] = make_float4(h.x, h.y, h.z, 0.f);
-            dot = double(pr.x) * h.x + double(pr.y) * h.y + double(pr.z) * h.z;
-        }
-        sdot[r] = dot;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0)
-    {
-        double s = 0.;
-        for (int k = 0; k < R; ++k)
-            s += sdot[k];
-        pqPart[w] = s;
-    }
+    float invTheta; // z1 = invTheta D^-1 r
+    float a2, b2;   // z2 = z1 + a2 z1 + b2 D^-1 (r - H z1)
+    float a3, b3;   // z3 = z2 + a3 (z2 - z1) + b3 D^-1 (r - H z2)
+};
+
+inline ChebyConstants MakeCheby()
+{
+    double const lo = kChebyMax / kChebyRatio, theta = 0.5 * (kChebyMax + lo), half = 0.5 * (kChebyMax - lo);
+    double const sigma = theta / half, r1 = 1. / sigma, r2 = 1. / (2. * sigma - r1), r3 = 1. / (2. * sigma - r2);
+    return ChebyConstants{static_cast<float>(1. / theta), static_cast<float>(r2 * r1),
+                          static_cast<float>(2. * r2 / half), static_cast<float>(r3 * r2),
+                          static_cast<float>(2. * r3 / half)};
+}
+
+// Sum over the wave in a fixed order, in every lane: 16-lane rows by DPP, then
+// the four row sums in order.
+template <int kCtrl>
+__device__ __forceinline__ double DppRead(double x)
+{
+    int const lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), kCtrl, 0xF, 0xF, false);
+    int const hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), kCtrl, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double ReadLane(double x, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
+                            __builtin_amdgcn_readlane(__double2loint(x), lane));
+}
+
+__device__ __forceinline__ double WaveSum(double x)
+{
+    x += DppRead<0xB1>(x);
+    x += DppRead<0x4E>(x);
+    x += DppRead<0x141>(x);
+    x += DppRead<0x140>(x);
+    return ((ReadLane(x, 0) + ReadLane(x, 16)) + ReadLane(x, 32)) + ReadLane(x, 48);
 }
 
 // Thread t of a group of N threads sums v[b + t], v[b + t + N], ... in that
 // order, issuing the loads U at a time (the order, and so the bits, do not
-// depend on U: out-of-range entries add an exact 0).
-template <int N, int U = 16>
+// depend on U). Out-of-range entries load the last one and add an exact 0:
+// written as a guarded load the compiler branches around each and waits after it.
+template <int N, int U = 8>
 __device__ __forceinline__ double StridedSum(double const* __restrict__ v, int b, int e, int t)
 {
     double s = 0.;
@@ -589,27 +572,22 @@ __device__ __forceinline__ double StridedSum(double const* __restrict__ v, int b
         double x[U];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-        {
-            int const k = k0 + u * N;
-            x[u] = k < e ? v[k] : 0.;
-        }
+            x[u] = v[min(k0 + u * N, e - 1)];
 #pragma unroll
         for (int u = 0; u < U; ++u)
-            s += x[u];
+            s += k0 + u * N < e ? x[u] : 0.;
     }
     return s;
 }
 
 // Sums of V values over the 128 threads of a workgroup in a fixed order (each
-// wave's butterfly, then wave 0 + wave 1); every thread calls it and gets the
-// sums in v.
+// wave's sum, then wave 0 + wave 1); every thread calls it and gets the sums in v.
 template <int V>
 __device__ __forceinline__ void Sum128(double (&v)[V], double (*lds)[V])
 {
 #pragma unroll
     for (int i = 0; i < V; ++i)
-        for (int off = 32; off > 0; off >>= 1)
-            v[i] += __shfl_xor(v[i], off);
+        v[i] = WaveSum(v[i]);
     __syncthreads();
     if ((threadIdx.x & 63) == 0)
 #pragma unroll
@@ -621,191 +599,142 @@ __device__ __forceinline__ void Sum128(double (&v)[V], double (*lds)[V])
         v[i] = lds[0][i] + lds[1][i];
 }
 
-// One workgroup of 128 threads per aggregate g of mesh m, alpha = rz / pq with
-// pq the sum of m's chunk partials in order (0 once m has converged); over the
-// aggregate's vertices:
-//   init:   r = b - q               (q = H y0)
-//   update: y += alpha p, r -= alpha q
-// then z = D^-1 r, and the aggregate's r . z, r . r (and b . b at init) and,
-// when rc is given, its restriction rc = Z^T r = (sum r_i, sum d_i x r_i),
-// summed in a fixed order and written to the per-aggregate partials. Every updated vertex belongs to
-// exactly one aggregate and every aggregate to one mesh.
-struct AggUpdateArgs
+// The recurrence's vectors y, r, p and s are kept in FP64: the one-reduction form
+// never forms H p, so an FP32 s drifts from it and an FP32 p from what s and y
+// have seen (errors of 3e-6 against 1.9e-6 of the classical form at the same
+// tolerance); w = H z is summed and kept in FP64 too. z and the preconditioner stay
+// FP32.
+struct Vec3d
 {
-    int const* __restrict__ aggPtr;
-    int const* __restrict__ aggVerts;
-    int const* __restrict__ aggMesh;
-    float4* __restrict__ y;
-    float4* __restrict__ r;
-    float4* __restrict__ z;
-    float4 const* __restrict__ p;
-    float4 const* __restrict__ q;
-    float4 const* __restrict__ b; // init only
-    float4 const* __restrict__ dinv;
-    double* __restrict__ rc;      // nullable
-    float4 const* __restrict__ coarseD; // per row: d_i of the coarse rotations (with rc)
-    double const* __restrict__ pqPart;
-    int2 const* __restrict__ aggChunks; // chunks of the aggregate's mesh
-    int const* __restrict__ aggFirst;   // kAggFirst vertices per aggregate (-1: none)
-    int const* __restrict__ aggDone;    // done flag of the aggregate's mesh
-    double* __restrict__ rzPart;
-    double* __restrict__ rrPart;
-    double* __restrict__ bbPart; // init only
-    CgState cg;
-    int init;
+    double x, y, z;
 };
 
-constexpr int kAggFirst = 128; // = AggUpdate's workgroup size
-
-__global__ __launch_bounds__(128) void AggUpdate(AggUpdateArgs u)
+// Device arrays of the fused solvers, rows aggregate-major.
+struct FusedArgs
 {
-    int const nM = u.cg.nM;
-    __shared__ double lds1[2][1];
-    __shared__ double lds9[2][9];
-    int const g = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x);
-    // independent loads first: the mesh, its chunk range, the aggregate's vertex
-    // range, its mesh's done flag and the thread's first vertex. A converged
-    // mesh's workgroups leave after those; the others load the mesh's chunk
-    // partials, r . z and the first vertex's data together.
-    int const m = u.aggMesh[g];
-    int2 const cr = u.aggChunks[g];
-    int const kBeg = u.aggPtr[g] + t, kEnd = u.aggPtr[g + 1];
-    int const done = u.init ? 0 : u.aggDone[g];
-    int const i0 = u.aggFirst[static_cast<size_t>(g) * kAggFirst + t];
-    if (done != 0)
-        return; // the aggregate's mesh has converged (uniform over the workgroup)
-    double pq[1] = {u.init ? 0. : StridedSum<128, 32>(u.pqPart, cr.x, cr.y, t)};
-    double const rzOld = u.init ? 0. : u.cg.P[kRz * nM + m];
-    // the thread's first vertex: loads issued before alpha is known
-    float4 const zero4 = make_float4(0.f, 0.f, 0.f, 0.f);
-    float4 q0 = zero4, a0 = zero4, y0 = zero4, r0 = zero4, d0 = zero4, d1 = zero4, o0 = zero4;
-    if (i0 >= 0)
-    {
-        if (u.rc)
-            o0 = u.coarseD[i0];
-        q0 = u.q[i0];
-        a0 = u.init ? u.b[i0] : u.p[i0];
-        if (!u.init)
-        {
-            y0 = u.y[i0];
-            r0 = u.r[i0];
-        }
-        d0 = u.dinv[2 * i0];
-        d1 = u.dinv[2 * i0 + 1];
-    }
-    float alpha = 0.f;
-    if (!u.init)
-    {
-        Sum128<1>(pq, lds1);
-        alpha = pq[0] != 0. ? static_cast<float>(rzOld / pq[0]) : 0.f;
-    }
-    double sx = 0., sy = 0., sz = 0., ox = 0., oy = 0., oz = 0., rz = 0., rr = 0., bb = 0.;
-    // init: a = b, r = b - q; update: a = p, y += alpha p, r -= alpha q
-    auto update = [&](int i, float4 const& qi, float4 const& ai, float4 yi, float4 ri, float4 const& D0,
-                      float4 const& D1, float4 const& d) {
-        if (u.init)
-        {
-            ri = make_float4(ai.x - qi.x, ai.y - qi.y, ai.z - qi.z, 0.f);
-            bb += Dot3(ai, ai);
-        }
-        else
-        {
-            yi.x += alpha * ai.x, yi.y += alpha * ai.y, yi.z += alpha * ai.z;
-            ri.x -= alpha * qi.x, ri.y -= alpha * qi.y, ri.z -= alpha * qi.z;
-            u.y[i] = yi;
-        }
-        u.r[i] = ri;
-        float4 const zi = make_float4(D0.x * ri.x + D0.y * ri.y + D0.z * ri.z,
-                                      D0.y * ri.x + D0.w * ri.y + D1.x * ri.z,
-                                      D0.z * ri.x + D1.x * ri.y + D1.y * ri.z, 0.f);
-        u.z[i] = zi;
-        sx += ri.x, sy += ri.y, sz += ri.z;
-        ox += d.y * ri.z - d.z * ri.y, oy += d.z * ri.x - d.x * ri.z, oz += d.x * ri.y - d.y * ri.x;
-        rz += Dot3(ri, zi);
-        rr += Dot3(ri, ri);
-    };
-    if (i0 >= 0)
-        update(i0, q0, a0, y0, r0, d0, d1, o0);
-    for (int k = kBeg + 128; k < kEnd; k += 128)
-    {
-        int const i = u.aggVerts[k];
-        float4 const qi = u.q[i], ai = u.init ? u.b[i] : u.p[i];
-        float4 yi = qi, ri = qi;
-        if (!u.init)
-        {
-            yi = u.y[i];
-            ri = u.r[i];
-        }
-        update(i, qi, ai, yi, ri, u.dinv[2 * i], u.dinv[2 * i + 1], u.rc ? u.coarseD[i] : zero4);
-    }
-    double sums[9] = {rz, rr, bb, sx, sy, sz, ox, oy, oz};
-    Sum128<9>(sums, lds9);
-    if (t == 0)
-    {
-        if (u.rc)
-            for (int c = 0; c < kCoarseDofs; ++c)
-                u.rc[kCoarseDofs * g + c] = sums[3 + c];
-        u.rzPart[g] = sums[0];
-        u.rrPart[g] = sums[1];
-        if (u.init)
-            u.bbPart[g] = sums[2];
-    }
+    // Hessian blocks
+    int const* __restrict__ rowPtr;
+    int const* __restrict__ col;
+    float4 const* __restrict__ va;
+    float4 const* __restrict__ vb;
+    float const* __restrict__ vc;
+    float4 const* __restrict__ dinv;
+    // vectors
+    Vec3d* y;
+    Vec3d* r;
+    Vec3d* p;
+    Vec3d* s;
+    float4* z;  // z1 of the polynomial, then z
+    float4* z2;
+    Vec3d* w; // H z
+    float4 const* y0; // initial guess
+    float4 const* b;
+    // per chunk: (first row, end row, mesh, 0); its r . z and z . w
+    int4 const* __restrict__ chunks;
+    double* gammaPart;
+    double* deltaPart;
+    int nChunks;
+    // per aggregate: (mesh, first row, end row, whether it is its mesh's first), its r . r (and r . z for block Jacobi) of the even and odd iterations, b . b
+    int4 const* __restrict__ aggInfo;
+    double* rrPart[2];
+    double* rzPart[2];
+    double* bbPart;
+    int* aggDone; // its mesh's done flag
+    int nAgg;
+    // coarse space (two-level): restriction, correction (2 float4 per aggregate:
+    // translation, rotation), offsets d and aggregate of each row
+    double* rc;
+    float4* zc;
+    float4 const* __restrict__ coarseD;
+    int const* __restrict__ aggOfRow;
+    float const* __restrict__ coarseF;
+    int4 const* __restrict__ coarseInfo;           // per aggregate: (b0, n, ., .)
+    long long const* __restrict__ coarseRowOffset; // per aggregate: its first row in coarseF
+    int xcdChunk; // > 0: row workgroups per XCD
+    int coarseBlocks; // CoarsePoly: workgroups of the coarse product (a multiple of 8)
+    ChebyConstants q;
+    CgState cg;
+    int* doneOut; // host-mapped copy of the done flags
+};
+
+__device__ __forceinline__ float4 ApplyInverse(float4 const& D0, float4 const& D1, float x, float y, float z)
+{
+    return make_float4(D0.x * x + D0.y * y + D0.z * z, D0.y * x + D0.w * y + D1.x * z, D0.z * x + D1.x * y + D1.y * z,
+                       0.f);
 }
 
-// zc = (Z^T H Z)^-1 rc per mesh and each coarse row's share of rc . zc, the
-// coarse part of the mesh's r . z, into rczcPart; then the coarse correction
-// Z_i zc_g = t_g + w_g x d_i (zc_g = (t_g, w_g)) added to z_i for the
-// aggregate's rows, so that z = D^-1 r + Z zc. One workgroup of kCoarseWaves
-// waves per aggregate g computes its kCoarseDofs rows: wave w takes the
-// 64-column chunks w, w + kCoarseWaves, ... of its mesh's n columns, loads rc
-// and the rows' entries of kU of them at once, then accumulates (kU chosen for
-// the largest mesh; the order of the terms does not depend on it); the waves'
-// sums are added in order. The order depends on n only, so a mesh gets the
-// same zc alone or in a batch. The aggregate's descriptor (its mesh's first
-// coarse row b0 and size n, its rows' range) and the offset of its first
-// inverse row are precomputed, and the rows' z and d are loaded before the
-// product, so the kernel waits on memory about twice. The fused solvers number
-// the rows aggregate-major: aggregate g's rows are the range info.z .. info.w
-// itself.
+template <int L>
+__device__ __forceinline__ double GroupSum(double x)
+{
+    if constexpr (L >= 2)
+        x += DppRead<0xB1>(x);
+    if constexpr (L >= 4)
+        x += DppRead<0x4E>(x);
+    if constexpr (L >= 8)
+        x += DppRead<0x141>(x);
+    if constexpr (L >= 16)
+        x += DppRead<0x140>(x);
+    if constexpr (L >= 32)
+        x += __shfl_xor(x, 16);
+    if constexpr (L >= 64)
+        x += __shfl_xor(x, 32);
+    return x;
+}
+
+// Blocks of the row that thread t works on, of the rows [first, end).
+template <int L>
+__device__ __forceinline__ int2 RowExtent(FusedArgs const& a, int first, int end)
+{
+    int const row = first + static_cast<int>(threadIdx.x) / L;
+    return row < end ? make_int2(a.rowPtr[row], a.rowPtr[row + 1]) : make_int2(0, 0);
+}
+
+// H v of threads / L consecutive rows (the thread's extent given), L lanes per row:
+// lane l takes blocks l, l + L, ... The products land in LDS; after the barrier
+// thread t < R finishes row first + t, its loads issued before the product (one
+// thread per row reads whole lines; a leader per row would read a quarter of each).
+// Sums in T.
+template <int L, class T>
+__device__ __forceinline__ void RowProducts(FusedArgs const& a, float4 const* v, int2 extent, T (*h)[3])
+{
+    int const t = static_cast<int>(threadIdx.x), lane = t & (L - 1);
+    T hx = 0, hy = 0, hz = 0;
+    for (int k = extent.x + lane; k < extent.y; k += L)
+    {
+        int const j = a.col[k];
+        float4 const A = a.va[k], B = a.vb[k];
+        float const C = a.vc[k];
+        float4 const P = v[j];
+        T const px = P.x, py = P.y, pz = P.z;
+        hx += A.x * px + A.y * py + A.z * pz;
+        hy += A.w * px + B.x * py + B.y * pz;
+        hz += B.z * px + B.w * py + C * pz;
+    }
+    hx = GroupSum<L>(hx), hy = GroupSum<L>(hy), hz = GroupSum<L>(hz);
+    if (lane == 0)
+        h[t / L][0] = hx, h[t / L][1] = hy, h[t / L][2] = hz;
+}
+
+// zc = (Z^T H Z)^-1 rc for aggregate g's kCoarseDofs rows, by the kCoarseWaves
+// waves of the workgroup: wave w takes the 64-column chunks w, w + kCoarseWaves,
+// ... of its mesh's n columns, loads rc and the rows' entries of kU of them at
+// once, then accumulates in FP64 (kU chosen for the largest mesh; the order of
+// the terms does not depend on it, and on n only); the waves' sums are added in
+// order. Out-of-range lanes load column n - 1 and drop it, so that every load of
+// a pass is in flight together.
 constexpr int kCoarseWaves = 4;
 
-struct CoarseApplyArgs
-{
-    float const* __restrict__ coarseF;
-    double const* __restrict__ rc;
-    double* __restrict__ zc;
-    double* __restrict__ rczcPart;
-    int4 const* __restrict__ info;            // per aggregate: (b0, n, first row, end row)
-    long long const* __restrict__ rowOffset;  // per aggregate: its first row in coarseF
-    int const* __restrict__ aggDone;          // per aggregate: its mesh's done flag
-    float4 const* __restrict__ coarseD;
-    float4* __restrict__ z;
-};
-
 template <int kU>
-__global__ __launch_bounds__(64 * kCoarseWaves) void CoarseApplyRows(CoarseApplyArgs a, int first)
+__device__ __forceinline__ void CoarseRows(FusedArgs const& a, int g)
 {
     constexpr int kR = kCoarseDofs, kW = kCoarseWaves;
     __shared__ double part[kW][kR];
-    __shared__ float zcS[kR];
-    int const g = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x);
-    int const wave = t >> 6, lane = t & 63;
-    int4 const inf = a.info[g];
-    long long const off = a.rowOffset[g];
-    int const done = first ? 0 : a.aggDone[g];
-    if (done != 0)
-        return; // the mesh has converged
+    int const t = static_cast<int>(threadIdx.x), wave = t >> 6, lane = t & 63;
+    int4 const inf = a.coarseInfo[g];
+    long long const off = a.coarseRowOffset[g];
+    if (a.aggDone[g] != 0)
+        return; // the mesh has converged (uniform over the workgroup)
     int const b0 = inf.x, n = inf.y;
-    // the thread's first row of the aggregate, its d and z, in flight during the product
-    int const k0 = inf.z + t;
-    int i0 = -1;
-    float4 d0 = make_float4(0.f, 0.f, 0.f, 0.f), z0 = d0;
-    if (k0 < inf.w)
-    {
-        i0 = k0;
-        d0 = a.coarseD[i0];
-        z0 = a.z[i0];
-    }
     float const* A = a.coarseF + off;
     double s[kR];
 #pragma unroll
@@ -815,8 +744,6 @@ __global__ __launch_bounds__(64 * kCoarseWaves) void CoarseApplyRows(CoarseApply
     {
         double x[kU];
         float v[kR][kU];
-        // branch-free: out-of-range lanes load column n - 1 and drop it, so
-        // every load of the pass is in flight together
 #pragma unroll
         for (int u = 0; u < kU; ++u)
         {
@@ -838,8 +765,7 @@ __global__ __launch_bounds__(64 * kCoarseWaves) void CoarseApplyRows(CoarseApply
     }
 #pragma unroll
     for (int i = 0; i < kR; ++i)
-        for (int o = 32; o > 0; o >>= 1)
-            s[i] += __shfl_xor(s[i], o);
+        s[i] = WaveSum(s[i]);
     if (lane == 0)
 #pragma unroll
         for (int i = 0; i < kR; ++i)
@@ -847,26 +773,385 @@ __global__ __launch_bounds__(64 * kCoarseWaves) void CoarseApplyRows(CoarseApply
     __syncthreads();
     if (t < kR)
     {
-        int const row = kR * g + t;
         double tot = part[0][t];
         for (int w = 1; w < kW; ++w)
             tot += part[w][t];
-        a.zc[row] = tot;
-        a.rczcPart[row] = tot * a.rc[row];
-        zcS[t] = static_cast<float>(tot);
+        reinterpret_cast<float*>(a.zc)[8 * static_cast<size_t>(g) + (t < 3 ? t : t + 1)] = static_cast<float>(tot);
     }
+}
+
+// The coarse product (workgroups below coarseBlocks, one per aggregate) next to
+// the polynomial's first product (half a chunk each): both read what CgUpdate1
+// wrote and neither needs the other.
+template <int L, int kU>
+__global__ __launch_bounds__(256) void CoarsePoly(FusedArgs a)
+{
+    int w = static_cast<int>(blockIdx.x);
+    if (w < a.coarseBlocks)
+    {
+        if (w < a.nAgg)
+            CoarseRows<kU>(a, w);
+        return;
+    }
+    w -= a.coarseBlocks;
+    if (a.xcdChunk > 0)
+        w = (w & 7) * a.xcdChunk + (w >> 3);
+    if (w >= 2 * a.nChunks)
+        return; // padding of the XCD order
+    constexpr int R = 256 / L;
+    __shared__ float h[R][3];
+    int4 const ch = a.chunks[w >> 1];
+    int const t = static_cast<int>(threadIdx.x), first = ch.x + (w & 1) * R, i = first + t;
+    bool const mine = t < R && i < ch.y;
+    int2 const extent = RowExtent<L>(a, first, ch.y); // in flight with the done flag
+    if (a.cg.F[kDone * a.cg.nM + ch.z] != 0)
+        return;
+    Vec3d r{0., 0., 0.};
+    float4 z1 = make_float4(0.f, 0.f, 0.f, 0.f), D0 = z1, D1 = z1;
+    if (mine)
+        r = a.r[i], z1 = a.z[i], D0 = a.dinv[2 * i], D1 = a.dinv[2 * i + 1];
+    RowProducts<L>(a, a.z, extent, h);
     __syncthreads();
-    float const tx = zcS[0], ty = zcS[1], tz = zcS[2], wx = zcS[3], wy = zcS[4], wz = zcS[5];
-    auto correct = [&](int i, float4 const& d, float4 zi) {
-        zi.x += tx + (wy * d.z - wz * d.y);
-        zi.y += ty + (wz * d.x - wx * d.z);
-        zi.z += tz + (wx * d.y - wy * d.x);
-        a.z[i] = zi;
+    if (!mine)
+        return;
+    // z2 = (1 + a2) z1 + b2 D^-1 (r - H z1)
+    float4 const q = ApplyInverse(D0, D1, static_cast<float>(r.x) - h[t][0], static_cast<float>(r.y) - h[t][1],
+                                  static_cast<float>(r.z) - h[t][2]);
+    a.z2[i] = make_float4(z1.x + (a.q.a2 * z1.x + a.q.b2 * q.x), z1.y + (a.q.a2 * z1.y + a.q.b2 * q.y),
+                          z1.z + (a.q.a2 * z1.z + a.q.b2 * q.z), 0.f);
+}
+
+enum class PolyMode : int
+{
+    kPolyLast,    // z = z3 + Z zc, r . z per chunk
+    kPolyProduct, // w = H z, z . w per chunk
+    kResidual     // r = b - H y0
+};
+
+// One workgroup of kChunkThreads per row chunk (XCD-aware order when xcdChunk > 0).
+template <int L, PolyMode M>
+__global__ __launch_bounds__(kChunkThreads) void BsrPoly(FusedArgs a)
+{
+    constexpr int R = kChunkThreads / L;
+    using T = std::conditional_t<M == PolyMode::kPolyLast, float, double>;
+    __shared__ T h[R][3];
+    __shared__ double part[kChunkThreads / 64];
+    int w = static_cast<int>(blockIdx.x);
+    if (a.xcdChunk > 0)
+        w = (w & 7) * a.xcdChunk + (w >> 3);
+    if (w >= a.nChunks)
+        return;
+    int4 const ch = a.chunks[w];
+    int const t = static_cast<int>(threadIdx.x), i = ch.x + t;
+    bool const mine = t < R && i < ch.y;
+    int2 const extent = RowExtent<L>(a, ch.x, ch.y); // in flight with the done flag
+    if (M != PolyMode::kResidual && a.cg.F[kDone * a.cg.nM + ch.z] != 0)
+        return; // the chunk's mesh has converged: its vectors no longer change
+    float4 const zero = make_float4(0.f, 0.f, 0.f, 0.f);
+    Vec3d r{0., 0., 0.};
+    float4 z1 = zero, z2 = zero, D0 = zero, D1 = zero, d = zero, ct = zero, cr = zero;
+    if (mine)
+    {
+        z1 = M == PolyMode::kResidual ? a.b[i] : a.z[i];
+        if constexpr (M == PolyMode::kPolyLast)
+        {
+            int const g = a.aggOfRow[i];
+            r = a.r[i], z2 = a.z2[i], D0 = a.dinv[2 * i], D1 = a.dinv[2 * i + 1];
+            d = a.coarseD[i], ct = a.zc[2 * g], cr = a.zc[2 * g + 1];
+        }
+    }
+    RowProducts<L>(a, M == PolyMode::kPolyLast ? a.z2 : M == PolyMode::kResidual ? a.y0 : a.z, extent, h);
+    __syncthreads();
+    double dot = 0.;
+    if (mine)
+    {
+        if constexpr (M == PolyMode::kPolyLast)
+        {
+            float4 const q =
+                ApplyInverse(D0, D1, static_cast<float>(r.x) - h[t][0], static_cast<float>(r.y) - h[t][1],
+                             static_cast<float>(r.z) - h[t][2]);
+            float4 const z = make_float4(
+                z2.x + (a.q.a3 * (z2.x - z1.x) + a.q.b3 * q.x) + (ct.x + (cr.y * d.z - cr.z * d.y)),
+                z2.y + (a.q.a3 * (z2.y - z1.y) + a.q.b3 * q.y) + (ct.y + (cr.z * d.x - cr.x * d.z)),
+                z2.z + (a.q.a3 * (z2.z - z1.z) + a.q.b3 * q.z) + (ct.z + (cr.x * d.y - cr.y * d.x)), 0.f);
+            a.z[i] = z; // nobody else reads z in this launch
+            dot = r.x * z.x + r.y * z.y + r.z * z.z;
+        }
+        else if constexpr (M == PolyMode::kPolyProduct)
+        {
+            a.w[i] = Vec3d{h[t][0], h[t][1], h[t][2]};
+            dot = z1.x * h[t][0] + z1.y * h[t][1] + z1.z * h[t][2];
+        }
+        else
+            a.r[i] = Vec3d{z1.x - h[t][0], z1.y - h[t][1], z1.z - h[t][2]};
+    }
+    if constexpr (M == PolyMode::kResidual)
+        return;
+    // the chunk's rows in a fixed order: each wave's, then the waves in order
+    double* const out = M == PolyMode::kPolyLast ? a.gammaPart : a.deltaPart;
+    if constexpr (R <= 64)
+    {
+        if (t < 64)
+        {
+            dot = WaveSum(dot);
+            if (t == 0)
+                out[w] = dot;
+        }
+    }
+    else
+    {
+        dot = WaveSum(dot);
+        if ((t & 63) == 0)
+            part[t >> 6] = dot;
+        __syncthreads();
+        if (t == 0)
+        {
+            for (int k = 1; k < kChunkThreads / 64; ++k)
+                dot += part[k];
+            out[w] = dot;
+        }
+    }
+}
+
+// z1 (two-level) or z = D^-1 r of one row, and its share of an aggregate's sums
+// (r . r, r . z, sum r_i, sum d_i x r_i).
+template <bool kTwoLevel>
+__device__ __forceinline__ void RowResidual(float4* zOut, float invTheta, int i, Vec3d const& r, float4 const& D0,
+                                            float4 const& D1, float4 const& d, double (&s)[8])
+{
+    float4 z = ApplyInverse(D0, D1, static_cast<float>(r.x), static_cast<float>(r.y), static_cast<float>(r.z));
+    if constexpr (kTwoLevel)
+        z.x *= invTheta, z.y *= invTheta, z.z *= invTheta;
+    zOut[i] = z;
+    s[0] += r.x * r.x + r.y * r.y + r.z * r.z;
+    s[1] += r.x * z.x + r.y * z.y + r.z * z.z;
+    if constexpr (kTwoLevel)
+    {
+        s[2] += r.x, s[3] += r.y, s[4] += r.z;
+        s[5] += d.y * r.z - d.z * r.y, s[6] += d.z * r.x - d.x * r.z, s[7] += d.x * r.y - d.y * r.x;
+    }
+}
+
+template <bool kTwoLevel>
+__device__ __forceinline__ void StoreAggregate(double* rr, double* rz, double* rc, int g, double const (&s)[8])
+{
+    rr[g] = s[0];
+    rz[g] = s[1];
+    if constexpr (kTwoLevel)
+        for (int c = 0; c < kCoarseDofs; ++c)
+            rc[kCoarseDofs * g + c] = s[2 + c];
+}
+
+// Start of a solve, one workgroup of 128 per aggregate (r = b - H y0 formed before):
+// y = y0, p = s = 0, z and the aggregate's sums, b . b among them.
+template <bool kTwoLevel>
+__global__ __launch_bounds__(128) void CgStartRows(FusedArgs a)
+{
+    __shared__ double lds[2][8], ldsB[2][1];
+    int const g = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x);
+    int4 const inf = a.aggInfo[g];
+    double s[8] = {0., 0., 0., 0., 0., 0., 0., 0.}, bb[1] = {0.};
+    for (int i = inf.y + t; i < inf.z; i += 128)
+    {
+        float4 const b = a.b[i], y = a.y0[i];
+        a.y[i] = Vec3d{y.x, y.y, y.z};
+        a.p[i] = a.s[i] = Vec3d{0., 0., 0.};
+        bb[0] += Dot3(b, b);
+        RowResidual<kTwoLevel>(a.z, a.q.invTheta, i, a.r[i], a.dinv[2 * i], a.dinv[2 * i + 1],
+                               kTwoLevel ? a.coarseD[i] : make_float4(0.f, 0.f, 0.f, 0.f), s);
+    }
+    Sum128<8>(s, lds);
+    Sum128<1>(bb, ldsB);
+    if (t == 0)
+    {
+        StoreAggregate<kTwoLevel>(a.rrPart[0], a.rzPart[0], a.rc, g, s);
+        a.bbPart[g] = bb[0];
+        a.aggDone[g] = 0;
+    }
+}
+
+// End of a solve: y into the rows' FP32 vector and into the vertices' order.
+__global__ __launch_bounds__(256) void CgSolution(Vec3d const* __restrict__ y, float4* __restrict__ rows,
+                                                  float4* __restrict__ out, int const* __restrict__ rowVertex, int n)
+{
+    int const i = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    if (i >= n)
+        return;
+    Vec3d const v = y[i];
+    float4 const f = make_float4(static_cast<float>(v.x), static_cast<float>(v.y), static_cast<float>(v.z), 0.f);
+    rows[i] = f;
+    out[rowVertex[i]] = f;
+}
+
+// Start and end of a solve, one workgroup of 64 per mesh: b . b and r . r from the
+// aggregates' sums of iteration parity `parity`. The start clears the recurrence's
+// scalars; the end records the residual of a mesh that ran out of iterations.
+__global__ __launch_bounds__(64) void CgMesh(FusedArgs a, int const* __restrict__ meshAggBegin, int start, int parity)
+{
+    int const m = static_cast<int>(blockIdx.x), nM = a.cg.nM, t = static_cast<int>(threadIdx.x);
+    int const done = a.cg.F[kDone * nM + m];
+    if (!start && done != 0)
+        return;
+    int const a0 = meshAggBegin[m], a1 = meshAggBegin[m + 1];
+    double const rr = WaveSum(StridedSum<64>(a.rrPart[parity], a0, a1, t));
+    double const bb = start ? WaveSum(StridedSum<64>(a.bbPart, a0, a1, t)) : a.cg.P[kBb * nM + m];
+    if (t != 0)
+        return;
+    int const d = !(bb > 0.) || rr <= a.cg.tol2 * bb ? 1 : 0;
+    if (start)
+    {
+        a.cg.P[kBb * nM + m] = bb;
+        a.cg.P[kGamma * nM + m] = 0., a.cg.P[kAlpha * nM + m] = 1.;
+        a.cg.F[kIters * nM + m] = 0;
+    }
+    a.cg.P[kRrLast * nM + m] = rr;
+    a.cg.F[kDone * nM + m] = d;
+    a.doneOut[m] = d;
+}
+
+// Head of an iteration, one workgroup of 128 threads per aggregate: the mesh's
+// gamma, delta and r . r from the partial sums (in a fixed order, by every
+// workgroup of the mesh), the stopping test |r| <= tol |b|, alpha and beta, then
+// over the aggregate's rows p, s, y, r, z (z1) and the aggregate's sums. Scalars
+// and r . r are kept per iteration parity (the old and new arrays of the
+// arguments): a workgroup may run before another of its mesh has read the old
+// ones. The mesh's first aggregate records them and the done flag; every workgroup
+// comes to the same test and sets its aggregate's own flag.
+// Bound by latency: the arguments, the descriptor, the sums with the scalars and
+// rows, and the stores are one memory trip each. So the arguments are a struct of
+// their own read at once, nothing but the descriptor and the flag decides whether
+// to go on, and rows and sums are loaded branch-free (out-of-range threads read
+// the last entry and drop it): guarded and looped loads waited for each other, 8.6
+// us a launch on 32^3 against 6.3 (5.5 at 10,000 rows).
+struct CgUpdateArgs
+{
+    int4 const* __restrict__ aggInfo;
+    int4 const* __restrict__ aggRange;
+    int* aggDone;
+    double const* gammaOld; // per mesh
+    double const* alphaOld;
+    double const* bb;
+    double const* gammaPart; // per chunk (two-level) or per aggregate
+    double const* deltaPart;
+    double const* rrOld;
+    Vec3d const* __restrict__ w;
+    float4* z;
+    Vec3d* p;
+    Vec3d* s;
+    Vec3d* y;
+    Vec3d* r;
+    float4 const* __restrict__ dinv;
+    float4 const* __restrict__ coarseD;
+    double tol2;
+    double* gammaNew;
+    double* alphaNew;
+    double* rrNew;
+    double* rzNew;
+    double* rc;
+    double* rrLast; // per mesh
+    int* done;
+    int* iters;
+    int* doneOut;
+    float invTheta;
+};
+
+// Entries b + t, b + t + 128, ... of v, the first U loaded at once.
+template <int U>
+struct PartialSum
+{
+    double x[U];
+    __device__ __forceinline__ void Load(double const* __restrict__ v, int b, int e, int t)
+    {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            x[u] = v[min(b + t + 128 * u, e - 1)];
+    }
+    __device__ __forceinline__ double Sum(double const* __restrict__ v, int b, int e, int t) const
+    {
+        double s = 0.;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            s += b + t + 128 * u < e ? x[u] : 0.;
+        if (e - b > 128 * U)
+            s += StridedSum<128>(v, b + 128 * U, e, t);
+        return s;
+    }
+};
+
+template <bool kTwoLevel>
+__global__ __launch_bounds__(128) void CgUpdate1(CgUpdateArgs a)
+{
+    __shared__ double lds3[2][3], lds8[2][8];
+    int const g = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x);
+    int4 const inf = a.aggInfo[g], rg = a.aggRange[g];
+    int const done = a.aggDone[g];
+    // keep the descriptor's loads together with the flag's
+    asm volatile("" ::"s"(inf.x), "s"(inf.y), "s"(rg.x), "s"(rg.z), "s"(done));
+    if (done != 0)
+        return;
+    int const m = inf.x, i0 = min(inf.y + t, inf.z - 1);
+    bool const mine = inf.y + t < inf.z;
+    int const gb = kTwoLevel ? rg.x : rg.z, ge = kTwoLevel ? rg.y : rg.w;
+    PartialSum<9> pg, pd;
+    PartialSum<4> pr;
+    pg.Load(a.gammaPart, gb, ge, t);
+    pd.Load(a.deltaPart, rg.x, rg.y, t);
+    pr.Load(a.rrOld, rg.z, rg.w, t);
+    double const gammaOld = a.gammaOld[m], alphaOld = a.alphaOld[m], bb = a.bb[m];
+    Vec3d const w0 = a.w[i0], p0 = a.p[i0], s0 = a.s[i0], y0 = a.y[i0], r0 = a.r[i0];
+    float4 const z0 = a.z[i0], D0 = a.dinv[2 * i0], D1 = a.dinv[2 * i0 + 1];
+    float4 d0 = make_float4(0.f, 0.f, 0.f, 0.f);
+    if constexpr (kTwoLevel)
+        d0 = a.coarseD[i0];
+    double v[3] = {pg.Sum(a.gammaPart, gb, ge, t), pd.Sum(a.deltaPart, rg.x, rg.y, t),
+                   pr.Sum(a.rrOld, rg.z, rg.w, t)};
+    Sum128<3>(v, lds3);
+    double const gamma = v[0], rr = v[2];
+    // beta = gamma / gammaOld, alpha = gamma / (delta - beta gamma / alphaOld)
+    double const beta = gammaOld != 0. ? gamma / gammaOld : 0.;
+    double const den = v[1] - beta * gamma / alphaOld;
+    double const alpha = den != 0. ? gamma / den : 0.;
+    bool const stop = rr <= a.tol2 * bb;
+    if (inf.w != 0 && t == 0)
+    {
+        a.rrLast[m] = rr;
+        if (stop)
+        {
+            a.done[m] = 1;
+            a.doneOut[m] = 1;
+        }
+        else
+        {
+            a.iters[m] += 1;
+            a.gammaNew[m] = gamma;
+            // alpha = 0 only after a breakdown (gamma = 0 or den = 0)
+            a.alphaNew[m] = alpha != 0. ? alpha : 1.;
+        }
+    }
+    if (stop)
+    {
+        if (t == 0)
+            a.aggDone[g] = 1;
+        return;
+    }
+    double sum[8] = {0., 0., 0., 0., 0., 0., 0., 0.};
+    auto update = [&](int i, Vec3d const& w, float4 const& z, Vec3d p, Vec3d s, Vec3d y, Vec3d r, float4 const& E0,
+                      float4 const& E1, float4 const& d) {
+        p.x = z.x + beta * p.x, p.y = z.y + beta * p.y, p.z = z.z + beta * p.z;
+        s.x = w.x + beta * s.x, s.y = w.y + beta * s.y, s.z = w.z + beta * s.z;
+        y.x += alpha * p.x, y.y += alpha * p.y, y.z += alpha * p.z;
+        r.x -= alpha * s.x, r.y -= alpha * s.y, r.z -= alpha * s.z;
+        a.p[i] = p, a.s[i] = s, a.y[i] = y, a.r[i] = r;
+        RowResidual<kTwoLevel>(a.z, a.invTheta, i, r, E0, E1, d, sum);
     };
-    if (i0 >= 0)
-        correct(i0, d0, z0);
-    for (int i = k0 + 64 * kW; i < inf.w; i += 64 * kW)
-        correct(i, a.coarseD[i], a.z[i]);
+    if (mine)
+        update(i0, w0, z0, p0, s0, y0, r0, D0, D1, d0);
+    for (int i = inf.y + t + 128; i < inf.z; i += 128)
+        update(i, a.w[i], a.z[i], a.p[i], a.s[i], a.y[i], a.r[i], a.dinv[2 * i], a.dinv[2 * i + 1],
+               kTwoLevel ? a.coarseD[i] : make_float4(0.f, 0.f, 0.f, 0.f));
+    Sum128<8>(sum, lds8);
+    if (t == 0)
+        StoreAggregate<kTwoLevel>(a.rrNew, a.rzNew, a.rc, g, sum);
 }
 
 // A solve's statistics without a host round trip: out = (largest per-mesh
@@ -895,21 +1180,13 @@ __global__ __launch_bounds__(64) void SolveStats(CgState cg, double* __restrict_
     }
 }
 
-// Vectors between the vertices' order and the solver's row order.
+// A vector from the vertices' order into the solver's row order.
 __global__ __launch_bounds__(256) void GatherRows(float4* __restrict__ out, float4 const* __restrict__ in,
                                                   int const* __restrict__ rowVertex, int n)
 {
     int const s = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
     if (s < n)
         out[s] = in[rowVertex[s]];
-}
-
-__global__ __launch_bounds__(256) void ScatterRows(float4* __restrict__ out, float4 const* __restrict__ in,
-                                                   int const* __restrict__ rowVertex, int n)
-{
-    int const s = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
-    if (s < n)
-        out[rowVertex[s]] = in[s];
 }
 
 // ---- initial guess of a backward solve from the previous solutions ----
@@ -1184,60 +1461,6 @@ __global__ __launch_bounds__(256) void ProjCombine(ProjArgs a)
         x += c[j] * b.x, y += c[j] * b.y, z += c[j] * b.z;
     }
     a.y[i] = make_float4(static_cast<float>(x), static_cast<float>(y), static_cast<float>(z), 0.f);
-}
-
-// End of an iteration of the fused CG, one workgroup per mesh: the mesh's
-// partials summed in a fixed order (one sum per wave), r . z = the aggregates'
-// r . D^-1 r + the coarse rows' rc . zc, then the stopping test and beta
-// (FinishMesh). Converged meshes are skipped; the host counts live meshes from
-// their done flags.
-struct CgFinishArgs
-{
-    CgState cg;
-    int const* __restrict__ meshAggBegin;
-    double const* __restrict__ rzPart;
-    double const* __restrict__ rrPart;
-    double const* __restrict__ bbPart;
-    double const* __restrict__ rczcPart; // nullable (block Jacobi)
-    int* __restrict__ doneOut;           // nullable: host-mapped copy of the done flags
-    int* __restrict__ aggDone;           // per aggregate: its mesh's done flag
-};
-
-__global__ __launch_bounds__(256) void CgFinish(CgFinishArgs f, int first)
-{
-    __shared__ double part[4];
-    int const nM = f.cg.nM;
-    int const m = static_cast<int>(blockIdx.x);
-    int const wave = static_cast<int>(threadIdx.x >> 6), lane = static_cast<int>(threadIdx.x & 63);
-    if (!first && f.cg.F[kDone * nM + m] != 0)
-        return;
-    int const a0 = f.meshAggBegin[m], a1 = f.meshAggBegin[m + 1];
-    // one sum per wave, all in flight together: r . D^-1 r, r . r, rc . zc, b . b
-    double v = 0.;
-    if (wave == 0)
-        v = StridedSum<64>(f.rzPart, a0, a1, lane);
-    else if (wave == 1)
-        v = StridedSum<64>(f.rrPart, a0, a1, lane);
-    else if (wave == 2 && f.rczcPart)
-        v = StridedSum<64, 32>(f.rczcPart, kCoarseDofs * a0, kCoarseDofs * a1, lane);
-    else if (wave == 3 && first)
-        v = StridedSum<64>(f.bbPart, a0, a1, lane);
-    for (int off = 32; off > 0; off >>= 1)
-        v += __shfl_xor(v, off);
-    if (lane == 0)
-        part[wave] = v;
-    __syncthreads();
-    __shared__ int doneS;
-    if (threadIdx.x == 0)
-    {
-        bool const live = FinishMesh(f.cg, m, part[1], part[0] + part[2], part[3], first);
-        if (f.doneOut)
-            f.doneOut[m] = live ? 0 : 1;
-        doneS = live ? 0 : 1;
-    }
-    __syncthreads();
-    for (int g = a0 + static_cast<int>(threadIdx.x); g < a1; g += static_cast<int>(blockDim.x))
-        f.aggDone[g] = doneS;
 }
 
 // Rotation offsets of the coarse space, one workgroup of 128 per aggregate g
