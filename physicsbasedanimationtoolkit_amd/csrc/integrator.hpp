@@ -162,11 +162,10 @@ struct RolloutState
     DeviceArray<double> solveStats; // per solve of a backward pass: iterations, relative residual
     int histHead = 0, histCount = 0;
     DeviceArray<float4> dinv;                                 // inverse diagonal blocks, 2 per vertex
-    DeviceArray<double> coarse[2];                            // coarse operator / its inverse (ping-pong)
-    DeviceArray<int> coarseFinal;                             // per mesh: buffer holding its inverse
+    DeviceArray<double> coarse;                               // coarse operator, inverted in place
     DeviceArray<float> coarseF;                               // the inverse, symmetrised, FP32
     DeviceArray<float4> coarseD;                              // per solver row: rotation offset of the coarse space
-    DeviceArray<double> pivotRows;                            // pivot rows of a Gauss-Jordan step, per mesh
+    DeviceArray<double> coarsePanel, coarsePivot;             // the sweeps' pivot columns and inverses, twice
     DeviceArray<int4> coarseInfo;                             // per aggregate: (b0, n, rows begin, rows end)
     DeviceArray<long long> coarseRowOffset;                   // per aggregate: its first row in coarseF
     int coarseMaxN = 0;                                       // rows of the largest mesh's coarse operator

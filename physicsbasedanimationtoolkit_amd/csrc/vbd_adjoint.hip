@@ -179,11 +179,8 @@ void BuildCoarse(pbat_vbd_integrator& h, float4 const* xs, float dt)
     RolloutState& R = h.rollout;
     size_t const total = static_cast<size_t>(h.coarseOffset.back());
     int const nM = h.nMeshes;
-    if (R.coarse[0].n != total)
-    {
-        R.coarse[0].allocate(total);
-        R.coarse[1].allocate(total);
-    }
+    if (R.coarse.n != total)
+        R.coarse.allocate(total);
     size_t const nCoarse = static_cast<size_t>(device::kCoarseDofs) * h.nAggregates;
     if (R.rc.n != nCoarse)
     {
@@ -193,7 +190,7 @@ void BuildCoarse(pbat_vbd_integrator& h, float4 const* xs, float dt)
     if (total == 0 || h.nAggregates == 0)
         return;
     device::CoarseArgs const c = MakeCoarseArgs(h);
-    hipLaunchKernelGGL(device::ZeroDoublesLong, dim3(1024), dim3(256), 0, h.stream, R.coarse[0].ptr,
+    hipLaunchKernelGGL(device::ZeroDoublesLong, dim3(1024), dim3(256), 0, h.stream, R.coarse.ptr,
                        static_cast<long long>(total));
     hipLaunchKernelGGL(device::ZeroDoublesLong, dim3(64), dim3(256), 0, h.stream, R.rc.ptr,
                        static_cast<long long>(R.rc.n));
@@ -212,41 +209,30 @@ void BuildCoarse(pbat_vbd_integrator& h, float4 const* xs, float dt)
         g.nCoarseBlocks = nCB;
         g.va = R.bsrA.ptr, g.vb = R.bsrB.ptr, g.vc = R.bsrC.ptr;
         g.blockRow = R.bsrBlockRow.ptr, g.col = R.bsrCol.ptr, g.coarseD = R.coarseD.ptr;
-        g.c = c, g.Ac = R.coarse[0].ptr;
+        g.c = c, g.Ac = R.coarse.ptr;
         hipLaunchKernelGGL(device::CoarseFromBsr, dim3((nCB + 3) / 4), dim3(256), 0, h.stream, g);
     }
     int maxN = 0;
-    std::vector<int> finalBuf(static_cast<size_t>(nM));
     for (int m = 0; m < nM; ++m)
-    {
-        int const n = device::kCoarseDofs * (h.aggBegin[m + 1] - h.aggBegin[m]);
-        maxN = std::max(maxN, n);
-        finalBuf[m] = ((n + device::kPivot - 1) / device::kPivot) % 2; // parity of its step count
-    }
+        maxN = std::max(maxN, device::kCoarseDofs * (h.aggBegin[m + 1] - h.aggBegin[m]));
     R.coarseMaxN = maxN;
-    int64_t const maxEntries = int64_t(maxN) * maxN;
-    dim3 const grid(static_cast<unsigned>((maxEntries + 255) / 256), static_cast<unsigned>(nM));
-    // block Gauss-Jordan: per step the pivot rows, then the rest in 64 x 64 tiles
-    int const tilesPerRow = (maxN + 63) / 64;
-    if (R.pivotRows.n != static_cast<size_t>(nM) * device::kPivot * maxN)
-        R.pivotRows.allocate(static_cast<size_t>(nM) * device::kPivot * maxN);
+    // block sweeps over the lower triangle's 64 x 64 tiles
+    size_t const panel = static_cast<size_t>(nM) * device::kPivot * maxN;
+    size_t const pivot = static_cast<size_t>(nM) * device::kPivot * device::kPivot;
+    if (R.coarsePanel.n != 2 * panel)
+        R.coarsePanel.allocate(2 * panel), R.coarsePivot.allocate(2 * pivot);
+    device::CoarseSweepArgs sw{};
+    sw.A = R.coarse.ptr, sw.stride = maxN, sw.c = c;
+    for (int k = 0; k < 2; ++k)
+        sw.panel[k] = R.coarsePanel.ptr + k * panel, sw.inv[k] = R.coarsePivot.ptr + k * pivot;
+    int const tiles = (maxN + 63) / 64;
+    hipLaunchKernelGGL(device::CoarseSweepFirst, dim3(tiles, nM), dim3(256), 0, h.stream, sw);
     for (int s = 0, k = 0; k < maxN; ++s, k += device::kPivot)
-    {
-        double const* Ak = R.coarse[s & 1].ptr;
-        hipLaunchKernelGGL(device::CoarsePivotRows, dim3(tilesPerRow, nM), dim3(256), 0, h.stream, Ak,
-                           R.pivotRows.ptr, k, maxN, c);
-        hipLaunchKernelGGL(device::CoarsePivotUpdate, dim3(tilesPerRow * tilesPerRow, nM), dim3(256), 0, h.stream,
-                           Ak, R.coarse[(s + 1) & 1].ptr, static_cast<double const*>(R.pivotRows.ptr), k, maxN,
-                           tilesPerRow, c);
-    }
-    // allocated once per size: the captured CG chunk graph holds this pointer
-    if (R.coarseFinal.n != finalBuf.size())
-        R.coarseFinal.allocate(finalBuf.size());
-    PBAT_HIP(hipMemcpyAsync(R.coarseFinal.ptr, finalBuf.data(), finalBuf.size() * sizeof(int),
-                            hipMemcpyHostToDevice, h.stream));
+        hipLaunchKernelGGL(device::CoarseSweep, dim3(tiles * (tiles + 1) / 2, nM), dim3(256), 0, h.stream, sw, k,
+                           s & 1);
     // per aggregate: its mesh's coarse rows (b0, n) and the offset of its first row
-    // of the inverse (allocated once per size: the captured CG chunk graph holds
-    // these pointers)
+    // of the inverse (once per handle: the captured CG chunk graph holds them)
+    if (R.coarseInfo.n != static_cast<size_t>(h.nAggregates))
     {
         std::vector<int4> info(static_cast<size_t>(h.nAggregates));
         std::vector<long long> rowOff(static_cast<size_t>(h.nAggregates));
@@ -261,25 +247,16 @@ void BuildCoarse(pbat_vbd_integrator& h, float4 const* xs, float dt)
                             static_cast<long long>(device::kCoarseDofs * g - b0) * n;
             }
         }
-        if (R.coarseInfo.n != info.size())
-        {
-            R.coarseInfo.allocate(info.size());
-            R.coarseRowOffset.allocate(rowOff.size());
-        }
-        PBAT_HIP(hipMemcpyAsync(R.coarseInfo.ptr, info.data(), info.size() * sizeof(int4), hipMemcpyHostToDevice,
-                                h.stream));
-        PBAT_HIP(hipMemcpyAsync(R.coarseRowOffset.ptr, rowOff.data(), rowOff.size() * sizeof(long long),
-                                hipMemcpyHostToDevice, h.stream));
+        R.coarseInfo.upload(info, h.stream);
+        R.coarseRowOffset.upload(rowOff, h.stream);
         PBAT_HIP(hipStreamSynchronize(h.stream)); // host temporaries
     }
-    PBAT_HIP(hipStreamSynchronize(h.stream)); // finalBuf is a host temporary
-    hipLaunchKernelGGL(device::CoarseGuard, dim3(nM), dim3(256), 0, h.stream, R.coarse[0].ptr, R.coarse[1].ptr,
-                       static_cast<int const*>(R.coarseFinal.ptr), c);
+    hipLaunchKernelGGL(device::CoarseGuard, dim3(nM), dim3(256), 0, h.stream, R.coarse.ptr, c);
     if (R.coarseF.n != total)
         R.coarseF.allocate(total);
-    hipLaunchKernelGGL(device::CoarseToFloat, grid, dim3(256), 0, h.stream,
-                       static_cast<double const*>(R.coarse[0].ptr), static_cast<double const*>(R.coarse[1].ptr),
-                       static_cast<int const*>(R.coarseFinal.ptr), c, R.coarseF.ptr);
+    int64_t const maxEntries = int64_t(maxN) * maxN;
+    hipLaunchKernelGGL(device::CoarseToFloat, dim3(static_cast<unsigned>((maxEntries + 255) / 256), nM), dim3(256), 0,
+                       h.stream, static_cast<double const*>(R.coarse.ptr), c, R.coarseF.ptr);
     PBAT_HIP(hipGetLastError());
 }
 

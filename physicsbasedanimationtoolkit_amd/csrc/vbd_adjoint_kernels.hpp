@@ -645,216 +645,6 @@ struct CoarseArgs
     int nAgg;
 };
 
-// Block Gauss-Jordan step on every mesh block (blockIdx.y = mesh): with the
-// pivot block P = A[K, K] of the rows and columns K = [k, k + b) (b = min(kPivot,
-// n - k)), Bk = step(Ak) is
-//   B[K, K] = P^-1,   B[K, j] = P^-1 A[K, j],   B[i, K] = -A[i, K] P^-1,
-//   B[i, j] = A[i, j] - A[i, K] P^-1 A[K, j]     (i, j outside K),
-// the same as b scalar steps; after ceil(n / kPivot) steps an n x n SPD block
-// holds its inverse. A step is two launches: CoarsePivotRows forms the b rows
-// W = B[K, :] (P^-1 in the K columns), CoarsePivotUpdate every other row from
-// Ak and W: B[i, j] = (j in K ? 0 : A[i, j]) - A[i, K] W[:, j].
-constexpr int kPivot = 32;
-
-// P inverted in LDS (SPD, no pivoting, Gauss-Jordan one entry per thread step)
-// by every workgroup, then W[:, j] for its 64 columns, 4 threads per column
-// each forming kPivot / 4 of its b entries. W holds kPivot rows of wStride
-// doubles per mesh.
-__global__ __launch_bounds__(256) void CoarsePivotRows(double const* __restrict__ Ak, double* __restrict__ W,
-                                                       int k, int wStride, CoarseArgs c)
-{
-    int const m = static_cast<int>(blockIdx.y);
-    int const n = kCoarseDofs * (c.meshAggBegin[m + 1] - c.meshAggBegin[m]);
-    int const j0 = static_cast<int>(blockIdx.x) * 64;
-    if (k >= n || j0 >= n)
-        return;
-    int const b = min(kPivot, n - k);
-    double const* A = Ak + c.meshOffset[m];
-    __shared__ double P[kPivot][kPivot + 1];
-    int const t = static_cast<int>(threadIdx.x);
-    for (int e = t; e < kPivot * kPivot; e += 256)
-    {
-        int const r = e / kPivot, q = e % kPivot;
-        P[r][q] = (r < b && q < b) ? A[static_cast<size_t>(k + r) * n + k + q] : 0.;
-    }
-    __syncthreads();
-    for (int q = 0; q < b; ++q)
-    {
-        double v[kPivot * kPivot / 256];
-#pragma unroll
-        for (int u = 0; u < kPivot * kPivot / 256; ++u)
-        {
-            int const e = t + 256 * u, r = e / kPivot, cc = e % kPivot;
-            double const inv = 1. / P[q][q];
-            if (r >= b || cc >= b)
-                v[u] = 0.;
-            else if (r == q && cc == q)
-                v[u] = inv;
-            else if (r == q)
-                v[u] = P[q][cc] * inv;
-            else if (cc == q)
-                v[u] = -P[r][q] * inv;
-            else
-                v[u] = P[r][cc] - P[r][q] * P[q][cc] * inv;
-        }
-        __syncthreads();
-#pragma unroll
-        for (int u = 0; u < kPivot * kPivot / 256; ++u)
-        {
-            int const e = t + 256 * u;
-            P[e / kPivot][e % kPivot] = v[u];
-        }
-        __syncthreads();
-    }
-    int const j = j0 + (t & 63), l0 = (t >> 6) * (kPivot / 4);
-    if (j >= n)
-        return;
-    double* Wm = W + static_cast<size_t>(m) * kPivot * wStride;
-    if (j >= k && j < k + b)
-    {
-        for (int l = l0; l < l0 + kPivot / 4 && l < b; ++l)
-            Wm[static_cast<size_t>(l) * wStride + j] = P[l][j - k];
-        return;
-    }
-    double w[kPivot / 4];
-#pragma unroll
-    for (int l = 0; l < kPivot / 4; ++l)
-        w[l] = 0.;
-    for (int q = 0; q < b; ++q)
-    {
-        double const aq = A[static_cast<size_t>(k + q) * n + j];
-#pragma unroll
-        for (int l = 0; l < kPivot / 4; ++l)
-            w[l] += P[l0 + l][q] * aq;
-    }
-#pragma unroll
-    for (int l = 0; l < kPivot / 4; ++l)
-        if (l0 + l < b)
-            Wm[static_cast<size_t>(l0 + l) * wStride + j] = w[l];
-}
-
-// The other rows of step k, one 64 x 64 tile of (i, j) per workgroup
-// (blockIdx.x over the tiles of the largest block, blockIdx.y = mesh): A[i, K]
-// and W[:, j] staged in LDS, a 4 x 4 group of entries per thread. Rows in K
-// copy W.
-__global__ __launch_bounds__(256) void CoarsePivotUpdate(double const* __restrict__ Ak, double* __restrict__ Bk,
-                                                         double const* __restrict__ W, int k, int wStride,
-                                                         int tilesPerRow, CoarseArgs c)
-{
-    int const m = static_cast<int>(blockIdx.y);
-    int const n = kCoarseDofs * (c.meshAggBegin[m + 1] - c.meshAggBegin[m]);
-    int const i0 = (static_cast<int>(blockIdx.x) / tilesPerRow) * 64, j0 = (static_cast<int>(blockIdx.x) % tilesPerRow) * 64;
-    if (k >= n || i0 >= n || j0 >= n)
-        return;
-    int const b = min(kPivot, n - k);
-    double const* A = Ak + c.meshOffset[m];
-    double* B = Bk + c.meshOffset[m];
-    double const* Wm = W + static_cast<size_t>(m) * kPivot * wStride;
-    __shared__ double Ai[64][kPivot + 1];
-    __shared__ double Wj[kPivot][64 + 1];
-    int const t = static_cast<int>(threadIdx.x);
-    for (int e = t; e < 64 * kPivot; e += 256)
-    {
-        int const r = e / kPivot, q = e % kPivot, i = i0 + r;
-        Ai[r][q] = (i < n && q < b) ? A[static_cast<size_t>(i) * n + k + q] : 0.;
-    }
-    for (int e = t; e < kPivot * 64; e += 256)
-    {
-        int const q = e / 64, cc = e % 64, j = j0 + cc;
-        Wj[q][cc] = (j < n && q < b) ? Wm[static_cast<size_t>(q) * wStride + j] : 0.;
-    }
-    __syncthreads();
-    // the 4 x 4 entries (r0 + u, c0 + v) of this thread, A[i, K] W[K, j] summed
-    // over K from registers
-    int const r0 = (t >> 4) * 4, c0 = (t & 15) * 4;
-    double acc[4][4];
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            acc[u][v] = 0.;
-#pragma unroll 8
-    for (int q = 0; q < kPivot; ++q)
-    {
-        double ai[4], wj[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            ai[u] = Ai[r0 + u][q];
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-            wj[v] = Wj[q][c0 + v];
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int v = 0; v < 4; ++v)
-                acc[u][v] += ai[u] * wj[v];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-    {
-        int const i = i0 + r0 + u;
-        if (i >= n)
-            break;
-        bool const iK = i >= k && i < k + b;
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-        {
-            int const j = j0 + c0 + v;
-            if (j >= n)
-                break;
-            double out;
-            if (iK)
-                out = Wj[i - k][c0 + v];
-            else
-                out = ((j >= k && j < k + b) ? 0. : A[static_cast<size_t>(i) * n + j]) - acc[u][v];
-            B[static_cast<size_t>(i) * n + j] = out;
-        }
-    }
-}
-
-// Guard after inversion: a mesh block whose inverse has a non-positive or
-// non-finite diagonal entry (an indefinite coarse operator) is zeroed, which
-// leaves that mesh with the block-Jacobi preconditioner. One workgroup per mesh.
-__global__ __launch_bounds__(256) void CoarseGuard(double* __restrict__ buf0, double* __restrict__ buf1,
-                                                   int const* __restrict__ finalBuf, CoarseArgs c)
-{
-    __shared__ int bad;
-    int const m = static_cast<int>(blockIdx.x);
-    int const n = kCoarseDofs * (c.meshAggBegin[m + 1] - c.meshAggBegin[m]);
-    double* A = (finalBuf[m] ? buf1 : buf0) + c.meshOffset[m];
-    if (threadIdx.x == 0)
-        bad = 0;
-    __syncthreads();
-    for (int i = static_cast<int>(threadIdx.x); i < n; i += static_cast<int>(blockDim.x))
-    {
-        double const d = A[static_cast<size_t>(i) * n + i];
-        if (!(d > 0.) || !isfinite(d))
-            bad = 1;
-    }
-    __syncthreads();
-    if (!bad)
-        return;
-    for (int64_t k = threadIdx.x; k < static_cast<int64_t>(n) * n; k += blockDim.x)
-        A[k] = 0.;
-}
-
-// The guarded inverse, symmetrised and rounded to FP32 for the CG's coarse
-// products (grid.y = mesh): it halves the bytes every iteration reads; the
-// preconditioner stays symmetric.
-__global__ __launch_bounds__(256) void CoarseToFloat(double const* __restrict__ buf0, double const* __restrict__ buf1,
-                                                     int const* __restrict__ finalBuf, CoarseArgs c,
-                                                     float* __restrict__ out)
-{
-    int const m = static_cast<int>(blockIdx.y);
-    int const n = kCoarseDofs * (c.meshAggBegin[m + 1] - c.meshAggBegin[m]);
-    int64_t const idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (idx >= static_cast<int64_t>(n) * n)
-        return;
-    int64_t const i = idx / n, j = idx % n;
-    double const* A = (finalBuf[m] ? buf1 : buf0) + c.meshOffset[m];
-    out[c.meshOffset[m] + idx] = static_cast<float>(0.5 * (A[i * n + j] + A[j * n + i]));
-}
-
 __global__ __launch_bounds__(256) void ZeroDoublesLong(double* __restrict__ p, long long n)
 {
     for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n;

@@ -1463,6 +1463,325 @@ __global__ __launch_bounds__(256) void ProjCombine(ProjArgs a)
     a.y[i] = make_float4(static_cast<float>(x), static_cast<float>(y), static_cast<float>(z), 0.f);
 }
 
+// In-place inversion of every mesh's symmetric positive definite block by block
+// sweeps: with the pivot block P = A[K, K] of the rows and columns K = [k, k + b)
+// (b = min(kPivot, n - k)), a step is
+//   A[K, K] <- -P^-1,   A[i, K] <- A[i, K] P^-1,   A[K, j] <- P^-1 A[K, j],
+//   A[i, j] <- A[i, j] - A[i, K] P^-1 A[K, j]     (i, j outside K),
+// which keeps A symmetric, so only the 64 x 64 tiles (I, J), I >= J, are stored and
+// updated; after ceil(n / kPivot) steps they hold -A^-1. A step is one launch
+// (CoarseSweep): it reads the pivot's columns from a panel of their own and
+// P^-1 from a buffer of its own, both left by the launch before it, which wrote
+// them from the tiles it updated; the tile that holds the next pivot block comes
+// first and inverts it while the others update. The panel and P^-1 alternate
+// between two buffers, so a launch reads none of what it writes.
+// Bound by latency: the tile's trip to memory and back (12 us a step on 752 rows)
+// and, on the tile of the next pivot, the 32 elimination steps (8.6 us). The 2,058 x
+// 2,058 block of a 32^3 mesh: 24.6 us a step (65 steps), 752 rows 20.5. As two
+// launches over all tiles, the pivot block inverted entry-parallel in LDS, a step
+// took 66 and 45 us.
+constexpr int kPivot = 32;
+// LDS row strides (doubles) for which the MFMA operand reads hit distinct banks
+constexpr int kPivotStride = 48, kPanelStride = 80, kWStride = 34;
+
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+struct CoarseSweepArgs
+{
+    double* A;
+    double* panel[2]; // nM x kPivot x stride: panel[q][i] = A[i][k + q]
+    double* inv[2];   // nM x kPivot x kPivot
+    int stride;
+    CoarseArgs c;
+};
+
+// 1 / x to FP64 accuracy without the range handling of a division (pivots of an
+// SPD matrix).
+__device__ __forceinline__ double Reciprocal(double x)
+{
+    double r = __builtin_amdgcn_rcp(x);
+    r = fma(r, fma(-x, r, 1.), r);
+    return fma(r, fma(-x, r, 1.), r);
+}
+
+// Inverse of the kPivot x kPivot SPD matrix S (LDS) into out, by a workgroup of 256
+// (Gauss-Jordan, no pivoting): thread (wave w, half h, lane j < 32) keeps column j of
+// rows 8 w + 4 h .. + 3 in registers. Per step the pivot row goes through LDS (one
+// barrier, two buffers) and the rows' entries of the pivot column come from the
+// wave's own lanes (8.6 us in all).
+__device__ __forceinline__ void InvertPivot(double (*S)[kPivotStride], double* __restrict__ out)
+{
+    static_assert(kPivot == 32, "a half-wave per row");
+    __shared__ double pivotRow[2][kPivot];
+    int const t = static_cast<int>(threadIdx.x), w = t >> 6, half = (t >> 5) & 1, j = t & 31;
+    int const i0 = 8 * w + 4 * half;
+    double a[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        a[u] = S[i0 + u][j];
+#pragma unroll 1
+    for (int q4 = 0; q4 < kPivot; q4 += 4)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+        {
+            int const q = q4 + v;
+            if (i0 == q4)
+                pivotRow[v & 1][j] = a[v];
+            double f[4]; // the rows' entries of column q
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+            {
+                double const lo = ReadLane(a[u], q), hi = ReadLane(a[u], 32 + q);
+                f[u] = half ? hi : lo;
+            }
+            __syncthreads();
+            double const inv = Reciprocal(pivotRow[v & 1][q]);
+            bool const own = j == q;
+            double const row = own ? inv : pivotRow[v & 1][j] * inv;
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                a[u] = i0 + u == q ? row : (own ? 0. : a[u]) - f[u] * row;
+        }
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+        out[(i0 + u) * kPivot + j] = a[u];
+}
+
+// What step k needs of the matrix before the first step: its panel and, by the
+// first workgroup of each mesh, its pivot block's inverse (grid.x = 64-row tiles).
+__global__ __launch_bounds__(256) void CoarseSweepFirst(CoarseSweepArgs a)
+{
+    __shared__ double S[kPivot][kPivotStride];
+    int const m = static_cast<int>(blockIdx.y), t = static_cast<int>(threadIdx.x);
+    int const n = kCoarseDofs * (a.c.meshAggBegin[m + 1] - a.c.meshAggBegin[m]);
+    int const i0 = static_cast<int>(blockIdx.x) * 64;
+    if (i0 >= n)
+        return;
+    int const b = min(kPivot, n);
+    double const* A = a.A + a.c.meshOffset[m];
+    double* V = a.panel[0] + static_cast<size_t>(m) * kPivot * a.stride;
+    for (int e = t; e < 64 * kPivot; e += 256)
+    {
+        int const i = i0 + e / kPivot, q = e % kPivot;
+        if (i < n)
+            V[static_cast<size_t>(q) * a.stride + i] = q < b ? A[static_cast<size_t>(i) * n + q] : 0.;
+    }
+    if (i0 != 0)
+        return;
+    for (int e = t; e < kPivot * kPivot; e += 256)
+    {
+        int const r = e / kPivot, q = e % kPivot;
+        S[r][q] = (r < b && q < b) ? A[static_cast<size_t>(r) * n + q] : r == q ? 1. : 0.;
+    }
+    __syncthreads();
+    InvertPivot(S, a.inv[0] + static_cast<size_t>(m) * kPivot * kPivot);
+}
+
+// One step on the tiles (I, J), I >= J, numbered I (I + 1) / 2 + J over the tiles
+// of the largest mesh (grid.y = mesh): W = A[I, K] P^-1 formed in LDS, then A[I, J] -=
+// W A[K, J], both by FP64 MFMA (16 x 16 x 4; operands: lane l holds row or column l
+// mod 16 and k = l / 16; results: column l mod 16 and rows l / 16 + 4 r). On the
+// vector units the products waited on their LDS operands (4 times the reads).
+__global__ __launch_bounds__(256) void CoarseSweep(CoarseSweepArgs a, int k, int parity)
+{
+    __shared__ double Vi[kPivot][kPanelStride], Vj[kPivot][kPanelStride], W[64][kWStride], P[kPivot][kPivotStride];
+    int const m = static_cast<int>(blockIdx.y), t = static_cast<int>(threadIdx.x);
+    int const n = kCoarseDofs * (a.c.meshAggBegin[m + 1] - a.c.meshAggBegin[m]);
+    if (k >= n)
+        return;
+    int const kn = k + kPivot, tn = kn / 64; // the next pivot and its tile
+    // the tile of the next pivot block trades places with the first
+    int idx = static_cast<int>(blockIdx.x);
+    int const diag = kn < n ? tn * (tn + 1) / 2 + tn : 0;
+    idx = idx == 0 ? diag : idx == diag ? 0 : idx;
+    int I = static_cast<int>((sqrtf(8.f * static_cast<float>(idx) + 1.f) - 1.f) * 0.5f);
+    while (I * (I + 1) / 2 > idx)
+        --I;
+    while ((I + 1) * (I + 2) / 2 <= idx)
+        ++I;
+    int const J = idx - I * (I + 1) / 2, i0 = 64 * I, j0 = 64 * J;
+    if (i0 >= n)
+        return;
+    int const b = min(kPivot, n - k), bn = kn < n ? min(kPivot, n - kn) : 0;
+    double* const A = a.A + a.c.meshOffset[m];
+    size_t const at = static_cast<size_t>(m) * kPivot * a.stride;
+    double const* V = a.panel[parity] + at;
+    double* const Vn = a.panel[parity ^ 1] + at;
+    double const* inv = a.inv[parity] + static_cast<size_t>(m) * kPivot * kPivot;
+    int const lane = t & 63, wave = t >> 6, l16 = lane & 15, l4 = lane >> 4;
+    // the wave's 32 x 32 quadrant as 2 x 2 MFMA tiles; entry (x, y, r) of a thread:
+    auto rowOf = [&](int x, int r) { return 32 * (wave >> 1) + 16 * x + l4 + 4 * r; };
+    auto colOf = [&](int y) { return 32 * (wave & 1) + 16 * y + l16; };
+    // in flight while the panels are staged
+    v4d acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                acc[x][y][r] = A[static_cast<size_t>(min(i0 + rowOf(x, r), n - 1)) * n + min(j0 + colOf(y), n - 1)];
+#pragma unroll
+    for (int u = 0; u < kPivot * 64 / 256; ++u)
+    {
+        int const e = t + 256 * u, q = e / 64, cc = e % 64;
+        Vi[q][cc] = i0 + cc < n ? V[static_cast<size_t>(q) * a.stride + min(i0 + cc, n - 1)] : 0.;
+        Vj[q][cc] = j0 + cc < n ? V[static_cast<size_t>(q) * a.stride + min(j0 + cc, n - 1)] : 0.;
+    }
+#pragma unroll
+    for (int u = 0; u < kPivot * kPivot / 256; ++u)
+    {
+        int const e = t + 256 * u;
+        P[e / kPivot][e % kPivot] = inv[e];
+    }
+    __syncthreads();
+    // X^T P^-1 for rows 16 wave .. + 15 (columns 16 y + l16 of the result)
+    auto form = [&](double (*X)[kPanelStride], v4d (&w)[2]) {
+        w[0] = w[1] = v4d{0., 0., 0., 0.};
+#pragma unroll
+        for (int q = 0; q < kPivot; q += 4)
+        {
+            double const x = X[q + l4][16 * wave + l16];
+            w[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, P[q + l4][l16], w[0], 0, 0, 0);
+            w[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, P[q + l4][16 + l16], w[1], 0, 0, 0);
+        }
+    };
+    v4d w[2];
+    form(Vi, w);
+#pragma unroll
+    for (int y = 0; y < 2; ++y)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            W[16 * wave + l4 + 4 * r][16 * y + l16] = -w[y][r];
+    __syncthreads();
+    // rows in K take P^-1 A[K, j] = (A[j, K] P^-1)^T: formed in Vi's place
+    bool const rowsInK = k >= i0 && k < i0 + 64, colsInK = k >= j0 && k < j0 + 64;
+    if (rowsInK)
+    {
+        form(Vj, w);
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                Vi[16 * y + l16][16 * wave + l4 + 4 * r] = w[y][r];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < kPivot; q += 4)
+    {
+        double x[2], y[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+        {
+            x[u] = W[32 * (wave >> 1) + 16 * u + l16][q + l4];
+            y[u] = Vj[q + l4][32 * (wave & 1) + 16 * u + l16];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int v = 0; v < 2; ++v)
+                acc[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[u], y[v], acc[u][v], 0, 0, 0);
+    }
+    // f(local row, local column, entry) over the thread's entries
+    auto each = [&](auto&& f) {
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                {
+                    double e = acc[x][y][r];
+                    f(rowOf(x, r), colOf(y), e);
+                    acc[x][y][r] = e;
+                }
+    };
+    if (rowsInK || colsInK)
+        each([&](int r, int c, double& e) {
+            int const iq = i0 + r - k, jq = j0 + c - k;
+            bool const iK = iq >= 0 && iq < b, jK = jq >= 0 && jq < b;
+            if (iK && jK)
+                e = -P[iq][jq];
+            else if (iK)
+                e = Vi[iq][c];
+            else if (jK)
+                e = -W[r][jq];
+        });
+    each([&](int r, int c, double& e) {
+        if (i0 + r < n && j0 + c < n)
+            A[static_cast<size_t>(i0 + r) * n + j0 + c] = e;
+    });
+    if (bn == 0 || (I != tn && J != tn))
+        return;
+    // the next panel: columns of tiles (I, tn), rows of tiles (tn, J) to its left
+    int const kk = kn - 64 * tn;
+    each([&](int r, int c, double& e) {
+        int const q = (J == tn ? c : r) - kk, i = J == tn ? i0 + r : j0 + c;
+        if (q >= 0 && q < bn && i < n && (J != tn || j0 + c < n))
+            Vn[static_cast<size_t>(q) * a.stride + i] = e;
+    });
+    // rows of the panel past the matrix are zero
+    if (bn < kPivot)
+    {
+        int const x0 = J == tn ? i0 : j0;
+        for (int e = t; e < 64 * (kPivot - bn); e += 256)
+            if (x0 + e % 64 < n)
+                Vn[static_cast<size_t>(bn + e / 64) * a.stride + x0 + e % 64] = 0.;
+    }
+    if (I != J)
+        return;
+    // the next pivot block's inverse
+    __syncthreads();
+    each([&](int r, int c, double& e) {
+        int const rq = r - kk, cq = c - kk;
+        if (rq >= 0 && rq < kPivot && cq >= 0 && cq < kPivot)
+            P[rq][cq] = (rq < bn && cq < bn) ? e : rq == cq ? 1. : 0.;
+    });
+    __syncthreads();
+    InvertPivot(P, a.inv[parity ^ 1] + static_cast<size_t>(m) * kPivot * kPivot);
+}
+
+// Guard after inversion: a mesh block whose inverse has a non-positive or
+// non-finite diagonal entry (an indefinite coarse operator) is zeroed, which
+// leaves that mesh with the block-Jacobi preconditioner. One workgroup per mesh;
+// A holds minus the inverse.
+__global__ __launch_bounds__(256) void CoarseGuard(double* __restrict__ buf, CoarseArgs c)
+{
+    __shared__ int bad;
+    int const m = static_cast<int>(blockIdx.x);
+    int const n = kCoarseDofs * (c.meshAggBegin[m + 1] - c.meshAggBegin[m]);
+    double* A = buf + c.meshOffset[m];
+    if (threadIdx.x == 0)
+        bad = 0;
+    __syncthreads();
+    for (int i = static_cast<int>(threadIdx.x); i < n; i += static_cast<int>(blockDim.x))
+    {
+        double const d = -A[static_cast<size_t>(i) * n + i];
+        if (!(d > 0.) || !isfinite(d))
+            bad = 1;
+    }
+    __syncthreads();
+    if (!bad)
+        return;
+    for (int64_t k = threadIdx.x; k < static_cast<int64_t>(n) * n; k += blockDim.x)
+        A[k] = 0.;
+}
+
+// The guarded inverse from its lower triangle, rounded to FP32 for the CG's coarse
+// products (grid.y = mesh): it halves the bytes every iteration reads.
+__global__ __launch_bounds__(256) void CoarseToFloat(double const* __restrict__ buf, CoarseArgs c,
+                                                     float* __restrict__ out)
+{
+    int const m = static_cast<int>(blockIdx.y);
+    int const n = kCoarseDofs * (c.meshAggBegin[m + 1] - c.meshAggBegin[m]);
+    int64_t const idx = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (idx >= static_cast<int64_t>(n) * n)
+        return;
+    int64_t const i = idx / n, j = idx % n;
+    double const* A = buf + c.meshOffset[m];
+    out[c.meshOffset[m] + idx] = -static_cast<float>(i >= j ? A[i * n + j] : A[j * n + i]);
+}
+
 // Rotation offsets of the coarse space, one workgroup of 128 per aggregate g
 // (rows aggRows[aggPtr[g] .. aggPtr[g + 1]), positions xs of their vertices):
 // c the centroid, s the RMS radius, coarseD[row] = ((x - c) / s, 1), or 0 when

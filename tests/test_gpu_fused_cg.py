@@ -42,3 +42,31 @@ def test_zero_right_hand_side(gpu_device, solver):
     g, X, _ = scene()
     y, st = g.adjoint_solve(X, DT, np.zeros_like(X), solver=solver)
     assert st["iterations"] == 0 and np.all(y == 0.0)
+
+
+@pytest.mark.parametrize("cells", [(3, 3, 3), (12, 3, 3), (20, 4, 4), (44, 3, 4), (13, 17, 9)])
+def test_coarse_operator_sizes(gpu_device, cells):
+    """Coarse operators of a few rows to a few hundred, below, at and past the 32-row
+    pivots and 64-row tiles of their inversion: the two-level solution against the FP64
+    direct solve (the bound of the other solver tests), in fewer iterations than block
+    Jacobi takes."""
+    from oracle import adjoint as A
+    from oracle import oracle as O
+
+    X, E = meshes.cube_tet_grid(*cells, jitter=0.1, seed=5)
+    X *= np.array(cells)[:, None] / max(cells)
+    nT = E.shape[1]
+    mu, lam = meshes.lame_coefficients(meshes.log_uniform(np.random.default_rng(2), 1e5, 1e6, nT), 0.45)
+    dbc, rho = meshes.bottom_vertices(X), np.full(nT, 1e3)
+    g = pbat.gpu.vbd.Integrator(pbat.sim.vbd.Data().with_volume_mesh(X, E).with_material(rho, mu, lam)
+                                .with_dirichlet_vertices(dbc).construct())
+    o = O.OracleVbd(X, E, rhoe=rho, mue=mu, lambdae=lam, dbc=dbc)
+    b = np.sin(2.0 * X[[1, 2, 0]] + 0.3)
+    H, idx = A.hessian(o, X.T, DT)
+    ref = np.zeros(3 * o.nV)
+    ref[idx] = A.spla.spsolve(H, b.T.reshape(-1)[idx])
+    kw = dict(max_iterations=2000, tolerance=1e-6, check_every=10)
+    y, st = g.adjoint_solve(X, DT, b, solver="pcg_two_level", **kw)
+    _, jacobi = g.adjoint_solve(X, DT, b, solver="pcg_jacobi", **kw)
+    assert st["iterations"] < jacobi["iterations"]
+    assert np.linalg.norm(y - ref.reshape(-1, 3).T) <= 1e-4 * np.linalg.norm(ref)
