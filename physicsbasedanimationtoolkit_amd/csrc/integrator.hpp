@@ -126,12 +126,21 @@ struct StarRecords
     DeviceArray<int> tet;
     DeviceArray<int4> wideIds;
     DeviceArray<float4> wideGeo;
+    // handles of small meshes only (device::VbdStepLocal)
+    DeviceArray<int2> nbrL, localMeshes;
+    DeviceArray<device::LocalInc> incL;
+    DeviceArray<device::LocalRange> localRanges;
+    DeviceArray<int> localVerts, localPlace;
+    int localMaxVerts = 0;  // > 0: every mesh of the handle is small
+    int localMaxColour = 0; // largest colour of a mesh
+    int localThreads = 0;   // workgroup that holds every mesh's colours
     int maxNeighbours = 0; // of an updated vertex
     bool wide = false;     // a vertex has more than device::kMaxStarNeighbours
     void reset()
     {
         rowPtr.reset(), nbr.reset(), nbrE.reset(), inc.reset(), incE.reset(), shape.reset(), tet.reset();
-        wideIds.reset(), wideGeo.reset();
+        wideIds.reset(), wideGeo.reset(), nbrL.reset(), localMeshes.reset(), incL.reset(), localRanges.reset();
+        localVerts.reset(), localPlace.reset();
     }
 };
 
@@ -402,9 +411,10 @@ int EffectiveLanes(pbat_vbd_integrator const& h);
 int EffectivePerLane(pbat_vbd_integrator const& h);
 // Launch one colour's sweep over nVerts vertices with the current shape.
 void LaunchSweep(pbat_vbd_integrator& h, device::SweepArgs const& a, int nVerts);
-// Star records of the current moduli (tgp): the CSR constants, then the fixed-stride rows.
+// Star records of the current moduli (tgp): the CSR constants, then their copies
+// (fixed-stride rows, local records).
 void RebuildStarMaterial(pbat_vbd_integrator& h);
-void FillFixedStride(pbat_vbd_integrator& h);
+void FillStarCopies(pbat_vbd_integrator& h);
 device::SweepArgs MakeSweepArgs(pbat_vbd_integrator& h, float sdt, float sdt2);
 // One forward Step (gpu/impl/vbd/Integrator.cu:82-103): graph replay or eager launches.
 // sync = false (rollouts): the step is only queued; the caller clears the status

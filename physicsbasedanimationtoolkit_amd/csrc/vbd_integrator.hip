@@ -57,12 +57,25 @@ int StarLdsBytes(pbat_vbd_integrator const& h, int block, int L)
     return block / L * std::max(h.star.maxNeighbours, 1) * static_cast<int>(sizeof(float4));
 }
 
+int LocalLdsBytes(int maxVerts, int nColors);
+
+// Whether Step takes VbdStepLocal: small meshes, the automatic shape, plain or
+// Chebyshev-accelerated VBD iterations without contact.
+bool StepsLocally(pbat_vbd_integrator const& h)
+{
+    return h.star.localMaxVerts > 0 && h.lanes == 0 && h.perLane == 0 && !h.contact &&
+           (h.acceleration == PBAT_VBD_ACCELERATION_NONE || h.acceleration == PBAT_VBD_ACCELERATION_CHEBYSHEV ||
+            (h.acceleration == PBAT_VBD_ACCELERATION_TRUST_REGION && h.curved));
+}
+
 int EffectiveLanes(pbat_vbd_integrator const& h)
 {
     if (h.star.wide)
         return 64;
     int L = h.lanes;
-    if (L == 0)
+    if (L == 0 && StepsLocally(h))
+        L = h.star.localMaxColour <= device::kLocalFewVertices ? 8 : device::kLocalManyLanes; // of the largest mesh
+    else if (L == 0)
     {
         // enough lanes that each handles about 2 incidences of the busiest vertex, or
         // 3 when the colours are large: fewer lanes waste fewer of them on the
@@ -195,8 +208,13 @@ device::SweepArgs MakeSweepArgs(pbat_vbd_integrator& h, float sdt, float sdt2)
     return a;
 }
 
-void FillFixedStride(pbat_vbd_integrator& h)
+void FillStarCopies(pbat_vbd_integrator& h)
 {
+    if (h.star.localMaxVerts > 0)
+        hipLaunchKernelGGL(device::LocalRecords,
+                           dim3(static_cast<unsigned>((h.nUpdated * device::kLocalInc + 255) / 256)), dim3(256), 0,
+                           h.stream, h.star.rowPtr.ptr, h.star.nbr.ptr, h.star.inc.ptr, h.star.localPlace.ptr,
+                           h.star.nbrL.ptr, h.star.incL.ptr, static_cast<int>(h.nUpdated));
     if (!h.star.incE.ptr)
         return;
     int const width = std::max(h.star.maxNeighbours, h.ellStride);
@@ -218,7 +236,7 @@ void RebuildStarMaterial(pbat_vbd_integrator& h)
     if (n == 0)
         return;
     hipLaunchKernelGGL(device::StarMaterial, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, h.stream, a);
-    FillFixedStride(h);
+    FillStarCopies(h);
 }
 
 hipEvent_t NextEvent(pbat_vbd_integrator& h)
@@ -252,13 +270,6 @@ void CollectTiming(pbat_vbd_integrator& h)
 // Enqueue the launches of one Step (gpu/impl/vbd/Integrator.cu:82-103) and
 // return the number of sweep launches. With eventBrackets, one event pair
 // brackets each substep's back-to-back sweep launches.
-// sim/vbd/Kernels.h:97-102 in FP32 as gpu/impl/vbd/ChebyshevIntegrator.cu:28-33
-// evaluates it, operator precedence included: for k >= 2, 4/4 - rho2 * omega.
-float ChebyshevOmega(int k, float rho2, float omega)
-{
-    return (k == 0) ? 1.f : (k == 1) ? 2.f / (2.f - rho2) : 4.f / 4.f - rho2 * omega;
-}
-
 // Before iteration 0 of a substep (Anderson: remember x).
 void BeginAcceleration(pbat_vbd_integrator& h)
 {
@@ -286,7 +297,7 @@ void LaunchAcceleration(pbat_vbd_integrator& h, int k, float& omega)
     int const grid = (n + 255) / 256;
     if (h.acceleration == PBAT_VBD_ACCELERATION_CHEBYSHEV)
     {
-        omega = ChebyshevOmega(k, h.rho * h.rho, omega);
+        omega = device::ChebyshevOmega(k, h.rho * h.rho, omega);
         hipLaunchKernelGGL(device::ChebyshevUpdate, dim3(grid), dim3(256), 0, h.stream, h.xm.ptr, h.xkm1.ptr,
                            h.xkm2.ptr, n, k, omega);
         return;
@@ -436,6 +447,27 @@ bool LinearTrustRegion(pbat_vbd_integrator const& h)
     return h.acceleration == PBAT_VBD_ACCELERATION_TRUST_REGION && !h.curved;
 }
 
+// The whole step in one launch; returns the number of launches.
+int EnqueueLocalStep(pbat_vbd_integrator& h, float dt, int iterations, int substeps)
+{
+    float const sdt = dt / static_cast<float>(substeps);
+    device::LocalStepArgs a{};
+    a.nbr = h.star.nbrL.ptr, a.inc = h.star.incL.ptr;
+    a.ranges = h.star.localRanges.ptr, a.meshes = h.star.localMeshes.ptr, a.verts = h.star.localVerts.ptr;
+    a.xm = h.xm.ptr, a.xtil = h.xtil.ptr, a.xt = h.xt.ptr, a.vel = h.vel.ptr, a.vprev = h.vprev.ptr;
+    a.aext = h.aext.ptr;
+    a.nColors = static_cast<int>(h.colorBegin.size()) - 1;
+    a.iterations = iterations, a.substeps = substeps, a.strategy = h.strategy, a.maxVerts = h.star.localMaxVerts;
+    a.c = MakeSweepArgs(h, sdt, sdt * sdt).c;
+    a.nonfinite = h.statusDev;
+    if (h.acceleration == PBAT_VBD_ACCELERATION_CHEBYSHEV)
+        a.xkm1 = h.xkm1.ptr, a.xkm2 = h.xkm2.ptr, a.rho2 = h.rho * h.rho;
+    hipLaunchKernelGGL(device::VbdStepLocal, dim3(h.nMeshes), dim3(h.star.localThreads),
+                       LocalLdsBytes(a.maxVerts, a.nColors), h.stream, a);
+    PBAT_HIP(hipGetLastError());
+    return 1;
+}
+
 int EnqueueStep(pbat_vbd_integrator& h, float dt, int iterations, int substeps, bool eventBrackets)
 {
     float const sdt = dt / static_cast<float>(substeps);
@@ -520,10 +552,25 @@ void Step(pbat_vbd_integrator& h, float dt, int iterations, int substeps, bool s
         EnsureTrustRegionBuffers(h, iterations, substeps);
     if (sync)
         ClearStatus(h);
-    if (!h.useGraph)
+    bool const local = StepsLocally(h);
+    if (!h.useGraph || local)
     {
-        InvalidateGraph(h);
-        EnqueueStep(h, dt, iterations, substeps, h.timing);
+        if (!h.useGraph)
+            InvalidateGraph(h);
+        if (local)
+        {
+            if (h.timing)
+                PBAT_HIP(hipEventRecord(NextEvent(h), h.stream));
+            int const launched = EnqueueLocalStep(h, dt, iterations, substeps);
+            h.trLogCount = 0;
+            if (h.timing)
+            {
+                PBAT_HIP(hipEventRecord(NextEvent(h), h.stream));
+                h.pendingLaunches.push_back(launched);
+            }
+        }
+        else
+            EnqueueStep(h, dt, iterations, substeps, h.timing);
         if (!sync)
             return;
         if (h.timing)
@@ -722,6 +769,68 @@ void BuildAggregates(pbat_vbd_integrator& h, pbat_vbd_data const* d, std::vector
 constexpr int64_t kLastLevelCacheBytes = int64_t{256} << 20;
 
 static int TV4(int4 const& t, int l) { return l == 0 ? t.x : l == 1 ? t.y : l == 2 ? t.z : t.w; }
+
+int LocalLdsBytes(int maxVerts, int nColors)
+{
+    return 2 * maxVerts * static_cast<int>(sizeof(float4)) +
+           (nColors + 1) * static_cast<int>(sizeof(device::LocalRange));
+}
+
+// Tables of VbdStepLocal when every mesh of the handle is small: no colour beyond
+// kLocalMaxColour vertices, no row beyond the fixed-size ones, positions and inertial
+// targets of a mesh in 64 KB of LDS (16-bit offsets).
+void BuildLocal(pbat_vbd_integrator& h, std::vector<int> const& meshOfOrig)
+{
+    int const nC = static_cast<int>(h.colorBegin.size()) - 1, nM = h.nMeshes;
+    if (h.maxDegree > device::kLocalInc || h.star.maxNeighbours > device::kLocalNbr || nC <= 0 || h.nUpdated == 0 ||
+        h.nUpdated * device::kLocalInc >= (int64_t{1} << 31))
+        return;
+    std::vector<device::LocalRange> ranges(static_cast<size_t>(nM) * (nC + 1), device::LocalRange{0, 0, 0});
+    for (int64_t v = 0; v < h.nV; ++v)
+    {
+        // colours are grouped by mesh, and so are the fixed vertices behind them
+        int const c = static_cast<int>(std::upper_bound(h.colorBegin.begin(), h.colorBegin.end(), static_cast<int>(v)) -
+                                       h.colorBegin.begin()) - 1;
+        device::LocalRange& r = ranges[static_cast<size_t>(meshOfOrig[h.perm[v]]) * (nC + 1) + c];
+        if (r.count++ == 0)
+            r.vbeg = static_cast<int>(v);
+    }
+    std::vector<int2> meshes(static_cast<size_t>(nM));
+    std::vector<int> verts, place(static_cast<size_t>(h.nV));
+    int maxVerts = 0, maxColour = 0, threads = 64;
+    for (int m = 0; m < nM; ++m)
+    {
+        int places = 0, largest = 0;
+        int const first = static_cast<int>(verts.size());
+        for (int c = 0; c <= nC; ++c)
+        {
+            device::LocalRange& r = ranges[static_cast<size_t>(m) * (nC + 1) + c];
+            r.lbeg = places;
+            for (int k = 0; k < r.count; ++k)
+            {
+                place[r.vbeg + k] = places++;
+                verts.push_back(r.vbeg + k);
+            }
+            if (c < nC)
+                largest = std::max(largest, r.count);
+        }
+        maxColour = std::max(maxColour, largest);
+        threads = std::max(threads, largest * (largest <= device::kLocalFewVertices ? 8 : device::kLocalManyLanes));
+        meshes[m] = make_int2(first, places);
+        maxVerts = std::max(maxVerts, places);
+    }
+    if (maxColour > device::kLocalMaxColour || LocalLdsBytes(maxVerts, nC) > kStarLdsBytes)
+        return;
+    h.star.localMaxVerts = maxVerts, h.star.localMaxColour = maxColour;
+    h.star.localThreads = (threads + 63) / 64 * 64;
+    h.star.localRanges.upload(ranges, h.stream);
+    h.star.localMeshes.upload(meshes, h.stream);
+    h.star.localVerts.upload(verts, h.stream);
+    h.star.localPlace.upload(place, h.stream);
+    h.star.nbrL.allocate(static_cast<size_t>(h.nUpdated) * device::kLocalNbr);
+    h.star.incL.allocate(static_cast<size_t>(h.nUpdated) * device::kLocalInc);
+    PBAT_HIP(hipStreamSynchronize(h.stream)); // host temporaries
+}
 
 // vertexOffsets (batches): first vertex of each mesh in d's numbering, count + 1
 // entries; vertices of one colour are then grouped by mesh.
@@ -1038,9 +1147,10 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
         {
             h->star.nbrE.allocate(static_cast<size_t>(nUpd) * h->star.maxNeighbours);
             h->star.incE.allocate(static_cast<size_t>(nUpd) * h->maxDegree);
-            FillFixedStride(*h);
         }
     }
+    BuildLocal(*h, meshOfOrig);
+    FillStarCopies(*h);
 
     h->wgHost.resize(static_cast<size_t>(nT));
     h->lameHost.resize(static_cast<size_t>(2 * nT));
@@ -1545,6 +1655,23 @@ void Autotune(pbat_vbd_integrator& h, float dt, int sweeps, double* timingsUs, i
     int count = 0;
     try
     {
+        // the automatic shape of a handle of small meshes: all sweeps in one launch
+        h.lanes = h.perLane = 0;
+        if (StepsLocally(h))
+        {
+            EnqueueLocalStep(h, dt, 1, 1); // warm-up
+            PBAT_HIP(hipEventRecord(e0, h.stream));
+            EnqueueLocalStep(h, dt, sweeps, 1);
+            PBAT_HIP(hipEventRecord(e1, h.stream));
+            PBAT_HIP(hipEventSynchronize(e1));
+            float ms = 0.f;
+            PBAT_HIP(hipEventElapsedTime(&ms, e0, e1));
+            best = 1e3 * ms / sweeps;
+            bestC = {0, 0, h.xcdRemap, h.ntStream, h.useEll};
+            if (timingsUs)
+                std::fill(timingsUs, timingsUs + 5, 0.), timingsUs[5] = best;
+            ++count;
+        }
         for (Candidate const& c : cands)
         {
             h.lanes = c.L, h.perLane = c.K, h.xcdRemap = c.xcd, h.ntStream = c.nt, h.useEll = c.ell;

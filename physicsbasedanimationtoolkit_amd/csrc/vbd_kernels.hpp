@@ -583,8 +583,43 @@ struct StarMaterialArgs
     a.nbr[p0.x + k].y = __float_as_int(static_cast<float>(G));
 }
 
-// Substep begin (gpu/impl/vbd/Integrator.cu:190-248; sim/vbd/Kernels.h:24-94):
-// inertial target x~ = xt + h v + h^2 a and the initial iterate.
+// Initial iterate of a substep (gpu/impl/vbd/Integrator.cu:190-248; sim/vbd/Kernels.h:24-94)
+// from x_t, v, v_{t-1} (AdaptiveVbd) and the external acceleration.
+__device__ __forceinline__ float3 InitialIterate(float4 const& p, float4 const& u, float4 const& w, float4 const& g,
+                                                 float dt, float dt2, int strategy)
+{
+    if (strategy == 0) // Position
+        return make_float3(p.x, p.y, p.z);
+    if (strategy == 1) // Inertia
+        return make_float3(p.x + dt * u.x, p.y + dt * u.y, p.z + dt * u.z);
+    if (strategy == 2) // KineticEnergyMinimum
+        return make_float3(p.x + dt * u.x + dt2 * g.x, p.y + dt * u.y + dt2 * g.y, p.z + dt * u.z + dt2 * g.z);
+    float const an2 = g.x * g.x + g.y * g.y + g.z * g.z;
+    float at = 0.f;
+    if (an2 != 0.f)
+    {
+        if (strategy == 3) // AdaptiveVbd
+        {
+            float const dot = ((u.x - w.x) / dt) * g.x + ((u.y - w.y) / dt) * g.y + ((u.z - w.z) / dt) * g.z;
+            at = fminf(fmaxf(dot / an2, 0.f), 1.f);
+        }
+        else // AdaptivePbat
+        {
+            float const vn = sqrtf(u.x * u.x + u.y * u.y + u.z * u.z) + 1.17549435e-38f;
+            float const dot = (u.x / vn) * g.x + (u.y / vn) * g.y + (u.z / vn) * g.z;
+            at = fminf(fabsf(dot / an2), 1.f);
+        }
+    }
+    float const s = dt2 * at;
+    return make_float3(p.x + dt * u.x + s * g.x, p.y + dt * u.y + s * g.y, p.z + dt * u.z + s * g.z);
+}
+
+__device__ __forceinline__ float4 InertialTarget(float4 const& p, float4 const& u, float4 const& g, float dt, float dt2)
+{
+    return make_float4(p.x + dt * u.x + dt2 * g.x, p.y + dt * u.y + dt2 * g.y, p.z + dt * u.z + dt2 * g.z, 0.f);
+}
+
+// Substep begin: inertial target x~ = xt + h v + h^2 a and the initial iterate.
 [[maybe_unused]] static __global__ __launch_bounds__(256) void SubstepBegin(float4* __restrict__ xm, float4* __restrict__ xtil,
                                                     float4 const* __restrict__ xt, float4 const* __restrict__ vel,
                                                     float4 const* __restrict__ vprev, float4 const* __restrict__ aext,
@@ -596,36 +631,8 @@ struct StarMaterialArgs
     float4 const p = xt[i];
     float4 const u = vel[i];
     float4 const g = aext[i];
-    xtil[i] = make_float4(p.x + dt * u.x + dt2 * g.x, p.y + dt * u.y + dt2 * g.y, p.z + dt * u.z + dt2 * g.z, 0.f);
-    float3 x0;
-    if (strategy == 0) // Position
-        x0 = make_float3(p.x, p.y, p.z);
-    else if (strategy == 1) // Inertia
-        x0 = make_float3(p.x + dt * u.x, p.y + dt * u.y, p.z + dt * u.z);
-    else if (strategy == 2) // KineticEnergyMinimum
-        x0 = make_float3(p.x + dt * u.x + dt2 * g.x, p.y + dt * u.y + dt2 * g.y, p.z + dt * u.z + dt2 * g.z);
-    else
-    {
-        float const an2 = g.x * g.x + g.y * g.y + g.z * g.z;
-        float at = 0.f;
-        if (an2 != 0.f)
-        {
-            if (strategy == 3) // AdaptiveVbd
-            {
-                float4 const w = vprev[i];
-                float const dot = ((u.x - w.x) / dt) * g.x + ((u.y - w.y) / dt) * g.y + ((u.z - w.z) / dt) * g.z;
-                at = fminf(fmaxf(dot / an2, 0.f), 1.f);
-            }
-            else // AdaptivePbat
-            {
-                float const vn = sqrtf(u.x * u.x + u.y * u.y + u.z * u.z) + 1.17549435e-38f;
-                float const dot = (u.x / vn) * g.x + (u.y / vn) * g.y + (u.z / vn) * g.z;
-                at = fminf(fabsf(dot / an2), 1.f);
-            }
-        }
-        float const s = dt2 * at;
-        x0 = make_float3(p.x + dt * u.x + s * g.x, p.y + dt * u.y + s * g.y, p.z + dt * u.z + s * g.z);
-    }
+    xtil[i] = InertialTarget(p, u, g, dt, dt2);
+    float3 const x0 = InitialIterate(p, u, strategy == 3 ? vprev[i] : u, g, dt, dt2, strategy);
     float const mass = xm[i].w;
     xm[i] = make_float4(x0.x, x0.y, x0.z, mass);
 }
@@ -650,6 +657,249 @@ struct StarMaterialArgs
     if (nonfinite && !(isfinite(x.x) && isfinite(x.y) && isfinite(x.z) && isfinite(u.x) && isfinite(u.y) &&
                        isfinite(u.z)))
         *nonfinite = 1;
+}
+
+// ---- small meshes: a whole step in one launch --------------------------------
+// Star records of a vertex in fixed-size rows whose entries name places in LDS (a
+// mesh's positions, 16 bytes each) by their byte offset: kLocalNbr neighbours
+// (offset, Gamma as bits) and kLocalInc tets (the other vertices' offsets a | b << 16
+// and c, A, B); unused entries hold the vertex itself and zeros, so no entry needs a
+// test.
+struct LocalInc
+{
+    unsigned int ab, c;
+    float A, B;
+};
+constexpr int kLocalNbr = 16, kLocalInc = 24;
+
+// Vertices of one mesh and colour (the last entry of a mesh: its fixed vertices):
+// internal range [vbeg, vbeg + count), places in the mesh from lbeg.
+struct LocalRange
+{
+    int vbeg, count, lbeg;
+};
+
+struct LocalStepArgs
+{
+    int2 const* __restrict__ nbr;
+    LocalInc const* __restrict__ inc;
+    LocalRange const* __restrict__ ranges; // per mesh nColors + 1
+    int2 const* __restrict__ meshes;       // per mesh: (first entry of verts, vertices)
+    int const* __restrict__ verts;         // internal vertex of each place
+    float4* xm;
+    float4* xtil;
+    float4* xt;
+    float4* vel;
+    float4* vprev;
+    float4 const* __restrict__ aext;
+    float4* xkm1; // Chebyshev: the previous two iterates (else null)
+    float4* xkm2;
+    float rho2;
+    int nColors, iterations, substeps, strategy, maxVerts;
+    StepConstants c;
+    int* nonfinite;
+};
+
+// A mesh's largest colour up to which its vertices get 8 lanes each (the shortest
+// chain), else 2 (the least work per vertex), and up to which meshes are stepped in one
+// workgroup each. A workgroup of kLocalThreads has lanes for every vertex of a colour
+// at once. Cubes, us per colour against a launch's 3.0: 7^3 (56 vertices a colour)
+// 1.45, 8^3 (81) 2.5, 9^3 (113) 2.7, 10^3 (151) 3.1, 11^3 (198) 3.9. 4 lanes take 2.0,
+// 2.3, 2.7 and 3.3, but four steps of 8^3 leave velocities 1.02e-4 of their norm from
+// FP64, where 2 lanes leave 0.97e-4, as the launches do.
+constexpr int kLocalThreads = 512;
+constexpr int kLocalFewVertices = kLocalThreads / 8;
+constexpr int kLocalManyLanes = 2;
+constexpr int kLocalMaxColour = 128;
+
+// omega of the Chebyshev update after iteration k (sim/vbd/Kernels.h:97-102 in FP32
+// as gpu/impl/vbd/ChebyshevIntegrator.cu:28-33 evaluates it, operator precedence
+// included: for k >= 2, 4/4 - rho2 * omega).
+__host__ __device__ inline float ChebyshevOmega(int k, float rho2, float omega)
+{
+    return (k == 0) ? 1.f : (k == 1) ? 2.f / (2.f - rho2) : 4.f / 4.f - rho2 * omega;
+}
+
+// The iterations of one substep on one mesh by a workgroup, positions and inertial
+// targets in LDS, L lanes per vertex: the arithmetic of VbdSweep<L, .> in its order.
+// Every thread works on one vertex of a colour (threads past its end on the last
+// one, without writing). Its records are loaded into registers a colour ahead, as
+// soon as the current ones are used, so the loads pass behind the reduction, the
+// Newton step and the barrier; a pass is LDS reads, arithmetic and a barrier.
+template <int L>
+__device__ __forceinline__ void LocalIterations(LocalStepArgs const& a, float4* pos, float4 const* til,
+                                                LocalRange const* ranges, int2 mesh)
+{
+    constexpr int NK = kLocalNbr / L, NT = kLocalInc / L;
+    int const t = static_cast<int>(threadIdx.x), lane = t & (L - 1), r = t / L, nC = a.nColors;
+    int2 J[NK];
+    LocalInc I[NT];
+    auto load = [&](int v) {
+        int2 const* const n = a.nbr + v * kLocalNbr + lane;
+        LocalInc const* const e = a.inc + v * kLocalInc + lane;
+#pragma unroll
+        for (int j = 0; j < NK; ++j)
+            J[j] = n[j * L];
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+            I[j] = e[j * L];
+    };
+    auto at = [&](unsigned int offset) {
+        return *reinterpret_cast<float4 const*>(reinterpret_cast<char const*>(pos) + offset);
+    };
+    LocalRange rg = ranges[0];
+    int last = max(rg.count - 1, 0);
+    load(rg.vbeg + min(r, last));
+    float omega = 0.f;
+    for (int k = 0; k < a.iterations; ++k)
+    {
+        for (int c = 0; c < nC; ++c)
+        {
+            int const mine = min(r, last), v = rg.vbeg + mine, place = rg.lbeg + mine;
+            bool const write = lane == 0 && r < rg.count;
+            float4 const own = pos[place], xl = til[place];
+            rg = ranges[c + 1 == nC ? 0 : c + 1];
+            last = max(rg.count - 1, 0);
+            auto offset = [&](unsigned int j) {
+                float4 const q = at(j);
+                return make_float4(q.x - own.x, q.y - own.y, q.z - own.z, 0.f);
+            };
+            Block B{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            float gsum = 0.f;
+#pragma unroll
+            for (int j = 0; j < NK; ++j)
+            {
+                float const G = __int_as_float(J[j].y);
+                float4 const dj = offset(static_cast<unsigned int>(J[j].x));
+                B.g0 += G * dj.x, B.g1 += G * dj.y, B.g2 += G * dj.z;
+                gsum += G;
+            }
+            B.h00 -= gsum, B.h11 -= gsum, B.h22 -= gsum;
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                AccumulateTet(I[j].A, I[j].B, offset(I[j].ab & 65535u), offset(I[j].ab >> 16), offset(I[j].c), B);
+            load(rg.vbeg + min(r, last));
+            GroupSum<L>(B);
+            if (write)
+            {
+                float3 const dx = NewtonStep(B, own, xl, (a.c.kD != 0.f) ? a.xt[v] : own, a.c);
+                pos[place] = make_float4(own.x - dx.x, own.y - dx.y, own.z - dx.z, own.w);
+            }
+            __syncthreads();
+        }
+        if (a.xkm1)
+        {
+            // Chebyshev (ChebyshevUpdate); the arrays follow the internal order
+            omega = ChebyshevOmega(k, a.rho2, omega);
+            for (int i = t; i < mesh.y; i += static_cast<int>(blockDim.x))
+            {
+                int const v = a.verts[mesh.x + i];
+                float4 x = pos[i];
+                if (k > 1)
+                {
+                    float4 const b = a.xkm2[v];
+                    x.x = omega * (x.x - b.x) + b.x;
+                    x.y = omega * (x.y - b.y) + b.y;
+                    x.z = omega * (x.z - b.z) + b.z;
+                    pos[i] = x;
+                }
+                a.xkm2[v] = a.xkm1[v];
+                a.xkm1[v] = x;
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// A whole step of one small mesh per workgroup: the substeps' begin, every colour of
+// every iteration with a workgroup barrier between them, and the end. A launch per
+// colour takes 3 us however few vertices it has; a pass here, bound by the chain of
+// LDS reads, reduction, Newton step and barrier, takes 0.9 us on 5 vertices a colour
+// and 1.45 us on 56 (20 iterations: 3^3 280 -> 113 us, 7^3 452 -> 232; 48 meshes of
+// 2^3..6^3 465 -> 186). With the records loaded at the pass instead of a colour ahead a
+// pass took 2.0 us, with CSR rows, whose tail needs a loop, 1.3..1.5. Dynamic LDS: 2
+// maxVerts float4, then the mesh's ranges.
+[[maybe_unused]] static __global__ __launch_bounds__(kLocalThreads) void VbdStepLocal(LocalStepArgs a)
+{
+    extern __shared__ float4 localLds[];
+    float4* const pos = localLds;
+    float4* const til = localLds + a.maxVerts;
+    LocalRange* const ranges = reinterpret_cast<LocalRange*>(localLds + 2 * a.maxVerts);
+    int const m = static_cast<int>(blockIdx.x), t = static_cast<int>(threadIdx.x), nt = static_cast<int>(blockDim.x);
+    int2 const mesh = a.meshes[m];
+    for (int c = t; c <= a.nColors; c += nt)
+        ranges[c] = a.ranges[static_cast<size_t>(m) * (a.nColors + 1) + c];
+    __syncthreads();
+    int largest = 0;
+    for (int c = 0; c < a.nColors; ++c)
+        largest = max(largest, ranges[c].count);
+    float const dt = a.c.dt, dt2 = a.c.dt2;
+    bool bad = false;
+    for (int s = 0; s < a.substeps; ++s)
+    {
+        for (int i = t; i < mesh.y; i += nt)
+        {
+            int const v = a.verts[mesh.x + i];
+            float4 const p = a.xt[v], u = a.vel[v], g = a.aext[v];
+            float4 const l = InertialTarget(p, u, g, dt, dt2);
+            float3 const x0 = InitialIterate(p, u, a.strategy == 3 ? a.vprev[v] : u, g, dt, dt2, a.strategy);
+            a.xtil[v] = til[i] = l;
+            pos[i] = make_float4(x0.x, x0.y, x0.z, a.xm[v].w);
+        }
+        __syncthreads();
+        if (largest == 0) // every vertex of the mesh is fixed
+            ;
+        else if (largest <= kLocalFewVertices)
+            LocalIterations<8>(a, pos, til, ranges, mesh);
+        else
+            LocalIterations<kLocalManyLanes>(a, pos, til, ranges, mesh);
+        for (int i = t; i < mesh.y; i += nt)
+        {
+            int const v = a.verts[mesh.x + i];
+            float4 const x = pos[i], p = a.xt[v];
+            a.vprev[v] = a.vel[v];
+            float4 const u = make_float4((x.x - p.x) / dt, (x.y - p.y) / dt, (x.z - p.z) / dt, 0.f);
+            a.vel[v] = u;
+            a.xt[v] = make_float4(x.x, x.y, x.z, 0.f);
+            a.xm[v] = x;
+            bad = bad || !(isfinite(x.x) && isfinite(x.y) && isfinite(x.z) && isfinite(u.x) && isfinite(u.y) &&
+                           isfinite(u.z));
+        }
+        __syncthreads(); // the next substep's threads read xt of other vertices
+    }
+    if (bad && a.nonfinite)
+        *a.nonfinite = 1;
+}
+
+// Local records of the current star records, one thread per (vertex, entry);
+// place[v] is vertex v's place in its mesh.
+[[maybe_unused]] static __global__ __launch_bounds__(256) void LocalRecords(
+    int2 const* __restrict__ rowPtr, int2 const* __restrict__ nbr, StarInc const* __restrict__ inc,
+    int const* __restrict__ place, int2* __restrict__ nbrL, LocalInc* __restrict__ incL, int nRows)
+{
+    static_assert(kLocalNbr <= kLocalInc, "one thread per tet entry");
+    int const t = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    int const v = t / kLocalInc, k = t % kLocalInc;
+    if (v >= nRows)
+        return;
+    int2 const p0 = rowPtr[v], p1 = rowPtr[v + 1];
+    unsigned int const own = 16u * static_cast<unsigned int>(place[v]);
+    if (k < kLocalNbr)
+    {
+        bool const used = p0.x + k < p1.x;
+        int2 const q = used ? nbr[p0.x + k] : make_int2(v, 0);
+        nbrL[v * kLocalNbr + k] = make_int2(16 * place[q.x], q.y);
+    }
+    LocalInc out{own | own << 16, own, 0.f, 0.f};
+    if (p0.y + k < p1.y)
+    {
+        StarInc const q = inc[p0.y + k];
+        auto at = [&](unsigned int j) {
+            return 16u * static_cast<unsigned int>(place[nbr[p0.x + static_cast<int>(j)].x]);
+        };
+        out = LocalInc{at(q.pk & 255u) | at((q.pk >> 8) & 255u) << 16, at((q.pk >> 16) & 255u), q.A, q.B};
+    }
+    incL[v * kLocalInc + k] = out;
 }
 
 // Chebyshev semi-iterative update after iteration k (sim/vbd/Kernels.h:104-118,
