@@ -126,12 +126,13 @@ struct StarRecords
     DeviceArray<int> tet;
     DeviceArray<int4> wideIds;
     DeviceArray<float4> wideGeo;
-    // handles of small meshes only (device::VbdStepLocal)
+    // handles of small meshes only (device::VbdStepLocal, device::CgLocal)
     DeviceArray<int2> nbrL, localMeshes;
     DeviceArray<device::LocalInc> incL;
     DeviceArray<device::LocalRange> localRanges;
     DeviceArray<int> localVerts, localPlace;
-    int localMaxVerts = 0;  // > 0: every mesh of the handle is small
+    int localMaxRows = 0;   // > 0: the local tables are there; most updated vertices of a mesh
+    int localMaxVerts = 0;  // > 0: small enough for VbdStepLocal; most vertices of a mesh
     int localMaxColour = 0; // largest colour of a mesh
     int localThreads = 0;   // workgroup that holds every mesh's colours
     int maxNeighbours = 0; // of an updated vertex
@@ -193,6 +194,10 @@ struct RolloutState
     // major), the vertex of each row, and each row's mesh and aggregate, and each
     // aggregate's rows (CSR by aggVertPtr)
     int bsrOrder = -1;
+    // device::CgLocal: tables of the current pattern, inverse diagonals by place
+    DeviceArray<int4> cgLocalRows;
+    DeviceArray<int> cgLocalPlace;
+    DeviceArray<float4> cgLocalDinv;
     DeviceArray<int> rowVertex, meshOfRow, aggOfRow, aggRows;
     DeviceArray<int> incPtr, incCode;
     DeviceArray<int4> incSlot;

@@ -661,6 +661,7 @@ void BuildBsrPattern(pbat_vbd_integrator& h, bool aggregateOrder)
     R.cbSrcPtr.upload(cbPtr, h.stream);
     R.cbSrc.upload(cbSrc, h.stream);
     PBAT_HIP(hipStreamSynchronize(h.stream));
+    R.cgLocalRows.reset();
     R.bsrOrder = order;
 }
 
@@ -992,6 +993,45 @@ void ProjectInitialGuess(pbat_vbd_integrator& h, float4* y, float4 const* b, int
     hipLaunchKernelGGL(device::ProjCombine, dim3(Blocks(n)), dim3(256), 0, h.stream, a);
 }
 
+// The Gauss-Seidel-preconditioned solve of a handle of small meshes, H assembled and
+// the scalars cleared (CgLocal).
+SolveResult SolveLocal(pbat_vbd_integrator& h, device::CgState const& cg, float4* y, float4 const* b, int maxIterations)
+{
+    RolloutState& R = h.rollout;
+    int const n = static_cast<int>(h.nUpdated), nV = static_cast<int>(h.nV);
+    int const nC = static_cast<int>(h.colorBegin.size()) - 1;
+    if (R.cgLocalRows.n != static_cast<size_t>(nV))
+    {
+        R.cgLocalRows.allocate(static_cast<size_t>(nV));
+        R.cgLocalDinv.allocate(2 * static_cast<size_t>(nV));
+        R.cgLocalPlace.allocate(R.bsrCol.n);
+        hipLaunchKernelGGL(device::CgLocalRowTable, dim3(Blocks(nV)), dim3(256), 0, h.stream,
+                           static_cast<int const*>(R.bsrRowPtr.ptr), static_cast<int const*>(R.bsrCol.ptr),
+                           static_cast<int const*>(h.star.localVerts.ptr),
+                           static_cast<int const*>(h.star.localPlace.ptr), R.cgLocalRows.ptr, R.cgLocalPlace.ptr, n,
+                           nV);
+    }
+    device::CgLocalArgs a{};
+    a.rows = R.cgLocalRows.ptr, a.place = R.cgLocalPlace.ptr, a.nBlocks = static_cast<int>(R.bsrCol.n);
+    a.va = R.bsrA.ptr, a.vb = R.bsrB.ptr, a.vc = R.bsrC.ptr, a.dinvRows = R.dinv.ptr, a.dinv = R.cgLocalDinv.ptr;
+    a.ranges = h.star.localRanges.ptr, a.meshes = h.star.localMeshes.ptr, a.verts = h.star.localVerts.ptr;
+    auto vec = [](DeviceArray<double> const& v) { return reinterpret_cast<device::Vec3d*>(v.ptr); };
+    a.y = vec(R.yD), a.r = vec(R.rD), a.p = vec(R.pD), a.s = vec(R.sD), a.w = vec(R.wD);
+    a.z = R.z.ptr, a.out = y, a.b = b, a.cg = cg, a.nColors = nC, a.maxRows = h.star.localMaxRows;
+    size_t const lds = sizeof(float4) * a.maxRows + sizeof(device::LocalRange) * (nC + 1);
+    // launches of a few ms at most; the host looks between them
+    constexpr int kChunk = 128;
+    for (int it = 0; it < maxIterations; it += kChunk)
+    {
+        if (it > 0 && ReadLive(h) == 0)
+            break;
+        hipLaunchKernelGGL(device::CgLocal, dim3(h.nMeshes), dim3(device::kCgLocalThreads), lds, h.stream, a,
+                           it == 0 ? 1 : 0, std::min(kChunk, maxIterations - it));
+    }
+    PBAT_HIP(hipGetLastError());
+    return ReadResult(h);
+}
+
 SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y, float4 const* b,
                   pbat_vbd_adjoint_config const& cfg, int nHist, double* statsOut)
 {
@@ -1061,6 +1101,8 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
         PBAT_HIP(hipGetLastError());
         return out;
     }
+    if (cfg.solver == PBAT_VBD_ADJOINT_PCG && h.star.localMaxRows > 0 && n > 0 && R.bsrCol.n < (size_t{1} << 28))
+        return SolveLocal(h, cg, y, b, cfg.max_iterations);
     device::FusedArgs fa{};
     fa.rowPtr = R.bsrRowPtr.ptr, fa.col = R.bsrCol.ptr, fa.va = R.bsrA.ptr, fa.vb = R.bsrB.ptr, fa.vc = R.bsrC.ptr;
     auto vec = [](DeviceArray<double> const& v) { return reinterpret_cast<device::Vec3d*>(v.ptr); };

@@ -1154,6 +1154,361 @@ __global__ __launch_bounds__(128) void CgUpdate1(CgUpdateArgs a)
         StoreAggregate<kTwoLevel>(a.rrNew, a.rzNew, a.rc, g, sum);
 }
 
+// ---- small meshes: a whole CG solve in one workgroup --------------------------
+// CG preconditioned by symmetric coloured block Gauss-Seidel on meshes of at most
+// kCgLocalRows updated vertices, one workgroup per mesh. As launches an iteration is
+// 2 colours + 4 of them, 3 us each however few rows they have; here the passes are
+// workgroup barriers apart, z lies in LDS, and the one-reduction recurrence of the
+// fused solvers (FP64 vectors and products) takes its sums without a launch. The
+// forward pass from z = 0 reads the blocks left of the diagonal only and the reverse
+// pass, z_i -= D_i^-1 sum_(j > i) H_ij z_j, those right of it, whose FP64 sums it leaves
+// for the product: an iteration reads one and a half matrices instead of three.
+// One CU issues all of it: a pass takes 1 us for its chain of instructions alone, and
+// 10 ns a row. Blocks and rows by place, loaded a pass ahead, took 57 us per iteration
+// at 1,872 rows with 8 lanes a row (two rounds a colour) and 47 with 4; the blocks
+// packed by halves 48; chunks of 16 rows padded to one length, 1 KB a load, 56.
+constexpr int kCgLocalThreads = 1024, kCgLocalLanes = 4;
+
+struct CgLocalArgs
+{
+    int4 const* __restrict__ rows; // first block, end of the lower ones, first upper one, end
+    int const* __restrict__ place; // of each block's column in its mesh
+    float4 const* __restrict__ va;
+    float4 const* __restrict__ vb;
+    float const* __restrict__ vc;
+    LocalRange const* __restrict__ ranges; // per mesh nColors + 1
+    int2 const* __restrict__ meshes;       // per mesh: (first entry of verts, vertices)
+    int const* __restrict__ verts;         // row of each place
+    float4 const* __restrict__ dinvRows;
+    float4 const* __restrict__ b;
+    float4* out; // y0, then the solution; like b and dinvRows by row, the rest by place
+    float4* dinv;
+    Vec3d* y;
+    Vec3d* r;
+    Vec3d* p;
+    Vec3d* s;
+    Vec3d* w;
+    float4* z;
+    CgState cg;
+    int nColors, maxRows, nBlocks;
+};
+
+// Block extents of each place's row, and the places of its columns (ascending).
+[[maybe_unused]] static __global__ __launch_bounds__(256) void CgLocalRowTable(
+    int const* __restrict__ rowPtr, int const* __restrict__ col, int const* __restrict__ verts,
+    int const* __restrict__ placeOf, int4* __restrict__ rows, int* __restrict__ place, int nRows, int nV)
+{
+    int const e = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    int const i = e < nV ? verts[e] : nRows;
+    if (i >= nRows) // fixed vertices have no row
+        return;
+    int const kb = rowPtr[i], ke = rowPtr[i + 1];
+    int lower = kb, upper = kb;
+    for (int k = kb; k < ke; ++k)
+    {
+        int const j = col[k];
+        place[k] = placeOf[j];
+        lower += j < i, upper += j <= i;
+    }
+    rows[e] = make_int4(kb, lower, upper, ke);
+}
+
+// Blocks [lo, hi) of one row times z by the row's kCgLocalLanes lanes: up to kSlots of
+// a lane loaded ahead (Load), as many as the longest row of the wave takes (a load
+// costs its cycles for every lane, used or not), then summed (Sum), longer rows in a
+// loop.
+struct LocalRow
+{
+    static constexpr int kSlots = 4;
+    float4 A[kSlots], B[kSlots];
+    float C[kSlots];
+    int j[kSlots];
+    int lo, hi, slots;
+    template <class V>
+    __device__ __forceinline__ static V At(V const* p, unsigned int bytes)
+    {
+        return *reinterpret_cast<V const*>(reinterpret_cast<char const*>(p) + bytes);
+    }
+    __device__ __forceinline__ void Load(CgLocalArgs const& a, int lo_, int hi_, int lane)
+    {
+        lo = lo_ + lane, hi = hi_;
+        slots = 0;
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u)
+            if (__any(lo + u * kCgLocalLanes < hi))
+            {
+                slots = u + 1;
+                int const k = min(max(min(lo + u * kCgLocalLanes, hi - 1), 0), a.nBlocks - 1);
+                unsigned int const o = static_cast<unsigned int>(k) * 4u; // 32-bit offsets from scalar bases
+                A[u] = At(a.va, o * 4u), B[u] = At(a.vb, o * 4u), C[u] = At(a.vc, o), j[u] = At(a.place, o);
+            }
+    }
+    template <class T>
+    __device__ __forceinline__ static void Add(T (&h)[3], float4 const& A, float4 const& B, float C, float4 const& z)
+    {
+        T const x = z.x, y = z.y, w = z.z;
+        h[0] += A.x * x + A.y * y + A.z * w;
+        h[1] += A.w * x + B.x * y + B.y * w;
+        h[2] += B.z * x + B.w * y + C * w;
+    }
+    template <class T>
+    __device__ __forceinline__ void Sum(CgLocalArgs const& a, float4 const* z, T (&h)[3]) const
+    {
+        h[0] = h[1] = h[2] = T(0);
+#pragma unroll
+        for (int u = 0; u < kSlots; ++u)
+            if (u < slots)
+            {
+                float4 q = z[j[u]];
+                bool const used = lo + u * kCgLocalLanes < hi;
+                q = make_float4(used ? q.x : 0.f, used ? q.y : 0.f, used ? q.z : 0.f, 0.f);
+                Add(h, A[u], B[u], C[u], q);
+            }
+        if (slots == kSlots)
+            for (int k = lo + kSlots * kCgLocalLanes; k < hi; k += kCgLocalLanes)
+                Add(h, a.va[k], a.vb[k], a.vc[k], z[a.place[k]]);
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            h[c] = GroupSum<kCgLocalLanes>(h[c]);
+    }
+};
+
+// first: from y0 (out); else the iterations go on from the vectors and scalars that an
+// earlier launch left. At most `iterations` of them, so a launch always ends soon.
+[[maybe_unused]] static __global__ __launch_bounds__(kCgLocalThreads) void CgLocal(CgLocalArgs a, int first,
+                                                                                  int iterations)
+{
+    constexpr int L = kCgLocalLanes, G = kCgLocalThreads / L;
+    extern __shared__ float4 cgLds[];
+    float4* const zL = cgLds;
+    LocalRange* const ranges = reinterpret_cast<LocalRange*>(cgLds + a.maxRows);
+    __shared__ double red[kCgLocalThreads / 64][3];
+    int const m = static_cast<int>(blockIdx.x), nM = a.cg.nM, t = static_cast<int>(threadIdx.x);
+    int const lane = t & (L - 1), g = t / L, nC = a.nColors;
+    double* const P = a.cg.P + m;
+    if (!first && a.cg.F[kDone * nM + m] != 0)
+        return;
+    int const base = a.meshes[m].x;
+    int const* const verts = a.verts + base;
+    a.rows += base, a.dinv += 2 * base, a.z += base;
+    a.y += base, a.r += base, a.p += base, a.s += base, a.w += base;
+    for (int c = t; c <= nC; c += kCgLocalThreads)
+        ranges[c] = a.ranges[static_cast<size_t>(m) * (nC + 1) + c];
+    __syncthreads();
+    int const nR = ranges[nC].lbeg; // the fixed vertices follow
+    int const colour0 = ranges[0].count, lastColour = ranges[nC - 1].lbeg;
+    auto sum3 = [&](double u, double v, double w, double (&out)[3]) {
+        double const x[3] = {WaveSum(u), WaveSum(v), WaveSum(w)};
+        if ((t & 63) == 0)
+            red[t >> 6][0] = x[0], red[t >> 6][1] = x[1], red[t >> 6][2] = x[2];
+        __syncthreads();
+        out[0] = out[1] = out[2] = 0.;
+#pragma unroll
+        for (int k = 0; k < kCgLocalThreads / 64; ++k)
+            out[0] += red[k][0], out[1] += red[k][1], out[2] += red[k][2];
+    };
+    // Passes of the preconditioner: forward over colours 1 .. nC - 1, reverse over
+    // nC - 2 .. 0. A pass's first G rows are loaded during the pass before (their
+    // extents one pass earlier), so that they arrive behind its reductions and barrier.
+    int const nPasses = 2 * (nC - 1);
+    auto colourOf = [&](int k) { return k < nC - 1 ? k + 1 : 2 * nC - 3 - k; };
+    auto clamped = [&](LocalRange const& rg, int r) {
+        return max(rg.lbeg + min(r, rg.count - 1), 0); // a colour without rows: its neighbour's, unused
+    };
+    int4 e;
+    LocalRow q;
+    float4 D0, D1;
+    Vec3d rq;
+    auto extents = [&](int k, int r) { e = a.rows[clamped(ranges[colourOf(k)], r)]; };
+    auto blocks = [&](int k, int r) {
+        int const i = clamped(ranges[colourOf(k)], r);
+        bool const forward = k < nC - 1;
+        q.Load(a, forward ? e.x : e.z, forward ? e.y : e.w, lane);
+        D0 = a.dinv[2 * i], D1 = a.dinv[2 * i + 1];
+    };
+    // z = M^-1 r: the first colour's rows have z = D^-1 r already
+    auto precondition = [&] {
+        if (nPasses > 0)
+        {
+            extents(0, g);
+            blocks(0, g);
+            extents(min(1, nPasses - 1), g);
+        }
+        __syncthreads();
+        for (int k = 0; k < nPasses; ++k)
+        {
+            LocalRange const rg = ranges[colourOf(k)];
+            bool const forward = k < nC - 1;
+            // whole waves leave the loop together: Load asks every lane
+            for (int r0 = t / 64 * (64 / L); r0 < rg.count; r0 += G)
+            {
+                int const r = r0 + (t & 63) / L, i = clamped(rg, r);
+                if (r >= G)
+                {
+                    extents(k, r);
+                    blocks(k, r);
+                }
+                if (forward)
+                    rq = a.r[i];
+                bool const mine = lane == 0 && r < rg.count;
+                if (forward)
+                {
+                    float h[3];
+                    q.Sum(a, zL, h);
+                    if (mine)
+                        zL[i] = ApplyInverse(D0, D1, static_cast<float>(rq.x) - h[0],
+                                             static_cast<float>(rq.y) - h[1], static_cast<float>(rq.z) - h[2]);
+                }
+                else
+                {
+                    // the columns right of the diagonal are final: their share of H z
+                    double h[3];
+                    q.Sum(a, zL, h);
+                    if (mine)
+                    {
+                        float4 const d = ApplyInverse(D0, D1, static_cast<float>(h[0]), static_cast<float>(h[1]),
+                                                      static_cast<float>(h[2])),
+                                     z = zL[i];
+                        zL[i] = make_float4(z.x - d.x, z.y - d.y, z.z - d.z, 0.f);
+                        a.w[i] = Vec3d{h[0], h[1], h[2]};
+                    }
+                }
+            }
+            if (k + 1 < nPasses)
+            {
+                if (rg.count > G)
+                    extents(k + 1, g);
+                blocks(k + 1, g);
+                extents(min(k + 2, nPasses - 1), g);
+            }
+            __syncthreads();
+        }
+    };
+    // every row's product, body(place, r, sums): whole or without the blocks right of
+    // the diagonal
+    auto product = [&](bool whole, auto&& body) {
+        int r = g;
+        int4 x = a.rows[min(r, nR - 1)];
+        for (int w0 = t / 64 * (64 / L); w0 < nR; w0 += G, r += G)
+        {
+            q.Load(a, x.x, whole ? x.w : x.z, lane);
+            rq = a.r[min(r, nR - 1)];
+            x = a.rows[min(r + G, nR - 1)];
+            double h[3];
+            q.Sum(a, zL, h);
+            if (lane == 0 && r < nR)
+                body(r, rq, h);
+        }
+    };
+    // w = H z, gamma = r . z, delta = z . w, with the sum of rr
+    double gamma = 0., delta = 0., rr = 0., sums[3];
+    auto productAndSums = [&] {
+        gamma = delta = 0.;
+        product(false, [&](int i, Vec3d const& r, double const (&h)[3]) {
+            float4 const z = zL[i];
+            Vec3d w = i < lastColour ? a.w[i] : Vec3d{0., 0., 0.};
+            w.x += h[0], w.y += h[1], w.z += h[2];
+            a.w[i] = w;
+            gamma += r.x * z.x + r.y * z.y + r.z * z.z;
+            delta += z.x * w.x + z.y * w.y + z.z * w.z;
+        });
+        sum3(gamma, delta, rr, sums);
+        gamma = sums[0], delta = sums[1], rr = sums[2];
+    };
+    auto startRow = [&](int i, Vec3d const& r, float4 const& E0, float4 const& E1) {
+        if (i < colour0)
+            zL[i] = ApplyInverse(E0, E1, static_cast<float>(r.x), static_cast<float>(r.y), static_cast<float>(r.z));
+    };
+    double gammaOld = 0., alphaOld = 1., bb;
+    if (first)
+    {
+        for (int i = t; i < nR; i += kCgLocalThreads)
+            zL[i] = a.out[verts[i]];
+        __syncthreads();
+        bb = 0.;
+        product(true, [&](int i, Vec3d const&, double const (&h)[3]) {
+            float4 const b = a.b[verts[i]];
+            Vec3d const r{b.x - h[0], b.y - h[1], b.z - h[2]};
+            a.r[i] = r;
+            bb += Dot3(b, b);
+            rr += r.x * r.x + r.y * r.y + r.z * r.z;
+        });
+        sum3(bb, rr, 0., sums);
+        bb = sums[0], rr = sums[1];
+        bool const done = !(bb > 0.) || rr <= a.cg.tol2 * bb;
+        if (t == 0)
+        {
+            P[kBb * nM] = bb, P[kRrLast * nM] = rr;
+            a.cg.F[kDone * nM + m] = done ? 1 : 0;
+        }
+        if (done)
+            return;
+        __syncthreads(); // every thread has its sums
+        for (int i = t; i < nR; i += kCgLocalThreads)
+        {
+            int const row = verts[i];
+            float4 const y = zL[i], E0 = a.dinvRows[2 * row], E1 = a.dinvRows[2 * row + 1];
+            a.y[i] = Vec3d{y.x, y.y, y.z};
+            a.p[i] = a.s[i] = Vec3d{0., 0., 0.};
+            a.dinv[2 * i] = E0, a.dinv[2 * i + 1] = E1;
+            startRow(i, a.r[i], E0, E1);
+        }
+        __syncthreads(); // dinv, before the passes load it ahead
+        precondition();
+        productAndSums();
+    }
+    else
+    {
+        bb = P[kBb * nM], gamma = P[kGamma * nM], gammaOld = P[kGamma1 * nM], delta = P[kAlpha1 * nM];
+        alphaOld = P[kAlpha * nM];
+        for (int i = t; i < nR; i += kCgLocalThreads)
+            zL[i] = a.z[i];
+    }
+    int it = 0;
+    bool done = false;
+    while (it < iterations && !done)
+    {
+        double const beta = gammaOld != 0. ? gamma / gammaOld : 0.;
+        double const den = delta - beta * gamma / alphaOld;
+        double const alpha = den != 0. ? gamma / den : 0.;
+        gammaOld = gamma;
+        alphaOld = alpha != 0. ? alpha : 1.; // 0 only after a breakdown
+        rr = 0.;
+#pragma unroll 1
+        for (int i = t; i < nR; i += kCgLocalThreads)
+        {
+            float4 const z = zL[i], E0 = a.dinv[2 * i], E1 = a.dinv[2 * i + 1];
+            Vec3d const w = a.w[i];
+            Vec3d p = a.p[i], s = a.s[i], y = a.y[i], r = a.r[i];
+            p.x = z.x + beta * p.x, p.y = z.y + beta * p.y, p.z = z.z + beta * p.z;
+            s.x = w.x + beta * s.x, s.y = w.y + beta * s.y, s.z = w.z + beta * s.z;
+            y.x += alpha * p.x, y.y += alpha * p.y, y.z += alpha * p.z;
+            r.x -= alpha * s.x, r.y -= alpha * s.y, r.z -= alpha * s.z;
+            a.p[i] = p, a.s[i] = s, a.y[i] = y, a.r[i] = r;
+            rr += r.x * r.x + r.y * r.y + r.z * r.z;
+            startRow(i, r, E0, E1);
+        }
+        precondition();
+        productAndSums();
+        ++it;
+        done = rr <= a.cg.tol2 * bb;
+    }
+    for (int i = t; i < nR; i += kCgLocalThreads)
+    {
+        Vec3d const y = a.y[i];
+        a.out[verts[i]] =
+            make_float4(static_cast<float>(y.x), static_cast<float>(y.y), static_cast<float>(y.z), 0.f);
+        a.z[i] = zL[i];
+    }
+    if (t == 0)
+    {
+        P[kGamma * nM] = gamma, P[kGamma1 * nM] = gammaOld, P[kAlpha1 * nM] = delta, P[kAlpha * nM] = alphaOld;
+        P[kRrLast * nM] = rr;
+        a.cg.F[kDone * nM + m] = done ? 1 : 0;
+        a.cg.F[kIters * nM + m] += it;
+    }
+}
+
 // A solve's statistics without a host round trip: out = (largest per-mesh
 // iteration count, largest per-mesh |r| / |b| at its last iteration).
 __global__ __launch_bounds__(64) void SolveStats(CgState cg, double* __restrict__ out)

@@ -776,14 +776,14 @@ int LocalLdsBytes(int maxVerts, int nColors)
            (nColors + 1) * static_cast<int>(sizeof(device::LocalRange));
 }
 
-// Tables of VbdStepLocal when every mesh of the handle is small: no colour beyond
-// kLocalMaxColour vertices, no row beyond the fixed-size ones, positions and inertial
-// targets of a mesh in 64 KB of LDS (16-bit offsets).
+// Tables of handles whose meshes are all small: for CgLocal when none has more than
+// kCgLocalRows updated vertices, and for VbdStepLocal when none has a colour beyond
+// kLocalMaxColour vertices or a row beyond the fixed-size ones, and a mesh's positions
+// and inertial targets fit in 64 KB of LDS (16-bit offsets).
 void BuildLocal(pbat_vbd_integrator& h, std::vector<int> const& meshOfOrig)
 {
     int const nC = static_cast<int>(h.colorBegin.size()) - 1, nM = h.nMeshes;
-    if (h.maxDegree > device::kLocalInc || h.star.maxNeighbours > device::kLocalNbr || nC <= 0 || h.nUpdated == 0 ||
-        h.nUpdated * device::kLocalInc >= (int64_t{1} << 31))
+    if (nC <= 0 || h.nUpdated == 0)
         return;
     std::vector<device::LocalRange> ranges(static_cast<size_t>(nM) * (nC + 1), device::LocalRange{0, 0, 0});
     for (int64_t v = 0; v < h.nV; ++v)
@@ -797,7 +797,7 @@ void BuildLocal(pbat_vbd_integrator& h, std::vector<int> const& meshOfOrig)
     }
     std::vector<int2> meshes(static_cast<size_t>(nM));
     std::vector<int> verts, place(static_cast<size_t>(h.nV));
-    int maxVerts = 0, maxColour = 0, threads = 64;
+    int maxVerts = 0, maxRows = 0, maxColour = 0, threads = 64;
     for (int m = 0; m < nM; ++m)
     {
         int places = 0, largest = 0;
@@ -815,20 +815,27 @@ void BuildLocal(pbat_vbd_integrator& h, std::vector<int> const& meshOfOrig)
                 largest = std::max(largest, r.count);
         }
         maxColour = std::max(maxColour, largest);
+        maxRows = std::max(maxRows, ranges[static_cast<size_t>(m) * (nC + 1) + nC].lbeg);
         threads = std::max(threads, largest * (largest <= device::kLocalFewVertices ? 8 : device::kLocalManyLanes));
         meshes[m] = make_int2(first, places);
         maxVerts = std::max(maxVerts, places);
     }
-    if (maxColour > device::kLocalMaxColour || LocalLdsBytes(maxVerts, nC) > kStarLdsBytes)
+    if (maxRows > device::kCgLocalRows)
         return;
-    h.star.localMaxVerts = maxVerts, h.star.localMaxColour = maxColour;
-    h.star.localThreads = (threads + 63) / 64 * 64;
+    h.star.localMaxRows = maxRows;
     h.star.localRanges.upload(ranges, h.stream);
     h.star.localMeshes.upload(meshes, h.stream);
     h.star.localVerts.upload(verts, h.stream);
     h.star.localPlace.upload(place, h.stream);
-    h.star.nbrL.allocate(static_cast<size_t>(h.nUpdated) * device::kLocalNbr);
-    h.star.incL.allocate(static_cast<size_t>(h.nUpdated) * device::kLocalInc);
+    if (h.maxDegree <= device::kLocalInc && h.star.maxNeighbours <= device::kLocalNbr &&
+        h.nUpdated * device::kLocalInc < (int64_t{1} << 31) && maxColour <= device::kLocalMaxColour &&
+        LocalLdsBytes(maxVerts, nC) <= kStarLdsBytes)
+    {
+        h.star.localMaxVerts = maxVerts, h.star.localMaxColour = maxColour;
+        h.star.localThreads = (threads + 63) / 64 * 64;
+        h.star.nbrL.allocate(static_cast<size_t>(h.nUpdated) * device::kLocalNbr);
+        h.star.incL.allocate(static_cast<size_t>(h.nUpdated) * device::kLocalInc);
+    }
     PBAT_HIP(hipStreamSynchronize(h.stream)); // host temporaries
 }
 

@@ -712,6 +712,11 @@ constexpr int kLocalFewVertices = kLocalThreads / 8;
 constexpr int kLocalManyLanes = 2;
 constexpr int kLocalMaxColour = 128;
 
+// Most updated vertices of a mesh whose Gauss-Seidel-preconditioned solves run in one
+// workgroup (CgLocal). us per iteration there / as launches: 18 rows 7.6 / 48, 100 14.5 /
+// 55, 294 19 / 59, 648 24 / 61, 1,872 47 / 63, 2,730 66 / 65, 3,150 75 / 61.
+constexpr int kCgLocalRows = 2400;
+
 // omega of the Chebyshev update after iteration k (sim/vbd/Kernels.h:97-102 in FP32
 // as gpu/impl/vbd/ChebyshevIntegrator.cu:28-33 evaluates it, operator precedence
 // included: for k >= 2, 4/4 - rho2 * omega).

@@ -1,0 +1,62 @@
+"""Gauss-Seidel-preconditioned step-Hessian solves of small meshes in one workgroup: one
+tet, colours longer than a workgroup takes at once, rows longer than the lanes load
+ahead, batches with a fixed mesh and a zero right-hand side, and more iterations than one
+launch makes. |H y - b| <= 2e-5 |b| with H from the matrix-free product: the solver's
+tolerance of 1e-5 on its FP64 recurrence and a few 1e-6 for the FP32 blocks, solution
+and product."""
+import numpy as np
+import pytest
+
+from physicsbasedanimationtoolkit_amd import pbat
+
+from test_gpu_edge import fan
+from test_gpu_local import DT, build, grid, loose
+
+pytestmark = pytest.mark.gpu
+
+
+def pose(X, E, dbc=None, amplitude=0.02):
+    rng = np.random.default_rng(3)
+    free = np.ones(X.shape[1], bool)
+    if dbc is not None:
+        free[dbc] = False
+    x = X + amplitude * rng.standard_normal(X.shape) * free
+    return x.astype(np.float32), (rng.standard_normal(X.shape) * free).astype(np.float32), free
+
+
+def residual(g, x, y, b, free):
+    h = g.hessian_vector(x, DT, y).astype(np.float64)
+    return np.linalg.norm((h - b)[:, free]) / np.linalg.norm(b[:, free])
+
+
+@pytest.mark.parametrize("mesh,amplitude", [(loose(1), 0.02), (loose(300), 0.02), (loose(700), 0.02), (fan(40), 0.02),
+                                            (grid(4, 3, 5), 0.02), (grid(12, 11, 13), 0.004)],
+                         ids=["tet", "colours300", "launches", "fan40", "grid", "grid2000"])
+def test_residual(gpu_device, mesh, amplitude):
+    g = pbat.gpu.vbd.Integrator(build(*mesh)[0])
+    x, b, free = pose(*mesh, amplitude=amplitude)  # no tet inverts
+    y, stats = g.adjoint_solve(x, DT, b, solver="pcg", max_iterations=400, tolerance=1e-5)
+    assert stats["relative_residual"] <= 1e-5
+    assert residual(g, x, y, b, free) <= 2e-5
+    # a later launch goes on where the first one stopped, and an earlier end is kept
+    y, stats = g.adjoint_solve(x, DT, b, solver="pcg", max_iterations=140, tolerance=0.0)
+    assert stats["iterations"] == 140
+    assert residual(g, x, y, b, free) <= 2e-5
+    _, stats = g.adjoint_solve(x, DT, b, solver="pcg", max_iterations=1, tolerance=1e-30)
+    assert stats["iterations"] == 1
+
+
+def test_batch(gpu_device):
+    X, E, _ = grid(2, 2, 2)
+    scenes = [loose(1), (X, E, np.arange(X.shape[1])), grid(7, 3, 5), fan(40), grid(2, 9, 6)]
+    batch = pbat.gpu.vbd.BatchIntegrator([build(*s)[0] for s in scenes])
+    xs, bs, frees = zip(*[pose(*s) for s in scenes])
+    bs = [b * (k != 2) for k, b in enumerate(bs)]
+    y, _ = batch.adjoint_solve(np.concatenate(xs, axis=1), DT, np.concatenate(bs, axis=1), solver="pcg",
+                               max_iterations=400, tolerance=1e-5)
+    for k, (s, x, b, free) in enumerate(zip(scenes, xs, bs, frees)):
+        yk = y[:, batch.offsets[k]:batch.offsets[k + 1]]
+        if k in (1, 2):
+            assert not yk.any()
+        else:
+            assert residual(pbat.gpu.vbd.Integrator(build(*s)[0]), x, yk, b, free) <= 2e-5
