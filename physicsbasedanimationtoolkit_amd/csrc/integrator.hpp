@@ -149,6 +149,7 @@ struct StarRecords
 struct RolloutState
 {
     bool valid = false;
+    DeviceArray<float4> end[3]; // rollout_backward: the state it restores
     // changes whenever a rollout is started or discarded, so a caller holding a
     // rollout can tell whether rollout_backward would still differentiate it
     int64_t generation = 0;
@@ -272,6 +273,13 @@ struct pbat_vbd_integrator
     std::vector<int> perm;       // internal -> original vertex index
     std::vector<int> iperm;      // original -> internal
     std::vector<float> massOrig; // lumped masses in original order (FP32)
+    // host <-> device vertex data: iperm and massOrig on the device, pinned memory the
+    // kernels read and write
+    pbat_vbd::DeviceArray<int> ipermD;
+    pbat_vbd::DeviceArray<float> massD, stageCopy;
+    void* stage = nullptr;
+    void* stageDev = nullptr;
+    size_t stageBytes = 0;
     std::vector<int64_t> meshOffsets; // batch: first vertex of each mesh (count + 1), empty otherwise
     int nMeshes = 1;
     pbat_vbd::DeviceArray<int> meshOf; // mesh of each internal vertex (0 for a plain integrator)
@@ -397,6 +405,9 @@ struct pbat_vbd_integrator
         rollout.lastX.reset();
         fp64Solves.reset();
         objVtp.reset(), objInc.reset(), objX.reset(), objXtil.reset(), objGrad.reset(), objPart.reset();
+        ipermD.reset(), massD.reset(), stageCopy.reset();
+        if (stage)
+            (void)hipHostFree(stage);
         if (statusHost)
             (void)hipHostFree(statusHost);
         if (rollout.doneHost)
@@ -432,9 +443,14 @@ void ClearStatus(pbat_vbd_integrator& h);
 void CheckStatus(pbat_vbd_integrator& h);
 void InvalidateGraph(pbat_vbd_integrator& h);
 // Host <-> device copies of 3 x nV column-major matrices (original vertex order)
-// into / out of float4 arrays (internal order); w components from wsrc (or 0).
-void UploadVec(pbat_vbd_integrator& h, float4* dst, float const* src, float const* wsrc);
+// into / out of float4 arrays (internal order); w components: the masses (or 0), and
+// 0 in the optional second array. Done when they return.
+void UploadVec(pbat_vbd_integrator& h, float4* dst, float const* src, bool masses, float4* second = nullptr);
 void DownloadVec(pbat_vbd_integrator& h, float4 const* src, float* dst);
+// The same of a packed FP64 3 x nV array in internal order.
+void DownloadVec(pbat_vbd_integrator& h, double const* src, double* dst);
+// n FP64 device values to FP32 host ones.
+void DownloadFloats(pbat_vbd_integrator& h, double const* src, float* dst, size_t n);
 void CheckVertexArray(pbat_vbd_integrator const& h, void const* p, int64_t n, char const* what);
 pbat_vbd_integrator& Handle(pbat_vbd_integrator* h);
 // Vertex-triangle contact (vbd_contact.hip): set-up from the data, the step's active

@@ -1360,13 +1360,14 @@ void RolloutBackward(pbat_vbd_integrator& h, float const* dLdx, float const* dLd
     size_t const n = static_cast<size_t>(nV);
     float const dt = R.dt;
     // end state, restored at the end
-    DeviceArray<float4> endX, endV, endVp;
-    endX.allocate(n), endV.allocate(n), endVp.allocate(n);
-    SaveState(h, endX.ptr, endV.ptr, endVp.ptr);
+    for (auto& s : R.end)
+        if (s.n != n)
+            s.allocate(n);
+    SaveState(h, R.end[0].ptr, R.end[1].ptr, R.end[2].ptr);
     // loss gradients of the final state (updated vertices only)
-    UploadVec(h, R.xbar.ptr, dLdx, nullptr);
+    UploadVec(h, R.xbar.ptr, dLdx, false);
     if (dLdv)
-        UploadVec(h, R.vbar.ptr, dLdv, nullptr);
+        UploadVec(h, R.vbar.ptr, dLdv, false);
     else
         Zero4(h, R.vbar.ptr, nV);
     if (nV > nUpd)
@@ -1456,19 +1457,13 @@ void RolloutBackward(pbat_vbd_integrator& h, float const* dLdx, float const* dLd
             st.max_relative_residual = std::max(st.max_relative_residual, static_cast<float>(S[2 * k + 1]));
         }
     }
-    RestoreState(h, endX.ptr, endV.ptr, endVp.ptr);
+    RestoreState(h, R.end[0].ptr, R.end[1].ptr, R.end[2].ptr);
     if (dv0)
         DownloadVec(h, R.vbar.ptr, dv0);
     if (dx0)
         DownloadVec(h, R.xbar.ptr, dx0);
     if (dLogY)
-    {
-        std::vector<double> g(static_cast<size_t>(nT));
-        PBAT_HIP(hipMemcpyAsync(g.data(), R.grad.ptr, sizeof(double) * nT, hipMemcpyDeviceToHost, h.stream));
-        PBAT_HIP(hipStreamSynchronize(h.stream));
-        for (int e = 0; e < nT; ++e)
-            dLogY[e] = static_cast<float>(g[e]);
-    }
+        DownloadFloats(h, R.grad.ptr, dLogY, static_cast<size_t>(nT));
     PBAT_HIP(hipStreamSynchronize(h.stream));
     if (stats)
         *stats = st;
@@ -1484,19 +1479,24 @@ void SetLogYoung(pbat_vbd_integrator& h, float const* logY, int64_t nT)
     PBAT_HIP(hipSetDevice(h.device));
     RolloutState& R = h.rollout;
     std::vector<float> v(logY, logY + nT);
-    R.logY.upload(v, h.stream);
+    if (R.logY.n != v.size())
+        R.logY.allocate(v.size());
+    PBAT_HIP(hipMemcpyAsync(R.logY.ptr, v.data(), sizeof(float) * v.size(), hipMemcpyHostToDevice, h.stream));
     hipLaunchKernelGGL(device::SetLogYoung, dim3(Blocks(nT)), dim3(256), 0, h.stream, R.logY.ptr, h.matBase.ptr,
                        h.tgp.ptr, h.slotsRows.ptr, h.rows.ids.ptr, h.rows.g2.ptr, static_cast<int>(nT));
     RebuildStarMaterial(h);
     PBAT_HIP(hipGetLastError());
     PBAT_HIP(hipStreamSynchronize(h.stream));
-    for (int64_t e = 0; e < nT; ++e)
-    {
-        // (mu, lambda) of the traces follow the new moduli
-        float const scale = std::exp(v[e] - h.logYCurrent[e]);
-        h.lameHost[2 * e] *= scale;
-        h.lameHost[2 * e + 1] *= scale;
-    }
+    HostParallel(static_cast<int>(nT), std::clamp(static_cast<int>(nT) / 65536, 1, 8),
+                 [&](int begin, int end, int) {
+                     for (int64_t e = begin; e < end; ++e)
+                     {
+                         // (mu, lambda) of the traces follow the new moduli
+                         float const scale = std::exp(v[e] - h.logYCurrent[e]);
+                         h.lameHost[2 * e] *= scale;
+                         h.lameHost[2 * e + 1] *= scale;
+                     }
+                 });
     h.logYCurrent = v;
     R.Discard();
 }
@@ -1509,8 +1509,8 @@ void HessianVectorProduct(pbat_vbd_integrator& h, float const* x, float dt, floa
     PBAT_HIP(hipSetDevice(h.device));
     EnsureBuffers(h);
     RolloutState& R = h.rollout;
-    UploadVec(h, R.hold.ptr, x, h.massOrig.data());
-    UploadVec(h, R.p.ptr, p, nullptr);
+    UploadVec(h, R.hold.ptr, x, true);
+    UploadVec(h, R.p.ptr, p, false);
     int const nV = static_cast<int>(h.nV), nUpd = static_cast<int>(h.nUpdated);
     if (nV > nUpd)
         Zero4(h, R.p.ptr + nUpd, nV - nUpd);
@@ -1535,8 +1535,8 @@ void AdjointSolve(pbat_vbd_integrator& h, float const* x, float dt, float const*
     EnsureBuffers(h);
     RolloutState& R = h.rollout;
     int const nV = static_cast<int>(h.nV), nUpd = static_cast<int>(h.nUpdated);
-    UploadVec(h, R.hold.ptr, x, h.massOrig.data());
-    UploadVec(h, R.rhs.ptr, b, nullptr);
+    UploadVec(h, R.hold.ptr, x, true);
+    UploadVec(h, R.rhs.ptr, b, false);
     if (nV > nUpd)
         Zero4(h, R.rhs.ptr + nUpd, nV - nUpd);
     Zero4(h, R.y.ptr, nV);

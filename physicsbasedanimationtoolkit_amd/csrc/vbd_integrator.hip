@@ -639,32 +639,93 @@ void CheckVertexArray(pbat_vbd_integrator const& h, void const* p, int64_t n, ch
     }
 }
 
-// Copy a 3 x nV host matrix (original numbering) into a float4 device array
-// (internal numbering); w components come from wsrc (nullptr -> 0).
-void UploadVec(pbat_vbd_integrator& h, float4* dst, float const* src, float const* wsrc)
+// Pinned memory of the handle for vertex data, 24 bytes per vertex up to 8 MB (larger
+// data pass in pieces), and the device's copies of iperm and the masses.
+constexpr size_t kStageBytes = size_t{8} << 20;
+// Uploads beyond this are copied to the device first; below it the kernel reads the
+// pinned memory itself (125 vertices: set 29 -> 15 us either way, 4,913: 28 read, 34
+// copied, 274,625: 760 read, 733 copied).
+constexpr size_t kStageRead = size_t{64} << 10;
+
+void EnsureStage(pbat_vbd_integrator& h)
 {
-    std::vector<float4> buf(static_cast<size_t>(h.nV));
-    for (int64_t v = 0; v < h.nV; ++v)
-    {
-        int64_t const i = h.perm[v];
-        buf[v] = make_float4(src[3 * i], src[3 * i + 1], src[3 * i + 2], wsrc ? wsrc[i] : 0.f);
-    }
-    PBAT_HIP(hipMemcpyAsync(dst, buf.data(), buf.size() * sizeof(float4), hipMemcpyHostToDevice, h.stream));
+    if (h.stage)
+        return;
+    size_t const bytes = std::clamp<size_t>(24 * static_cast<size_t>(h.nV), 256 * 24, kStageBytes);
+    if (!h.ipermD.ptr)
+        h.ipermD.upload(h.iperm, h.stream);
+    if (!h.massD.ptr)
+        h.massD.upload(h.massOrig, h.stream);
+    if (!h.stageCopy.ptr)
+        h.stageCopy.allocate(bytes / sizeof(float));
     PBAT_HIP(hipStreamSynchronize(h.stream));
+    void *p = nullptr, *d = nullptr;
+    if (hipHostMalloc(&p, bytes + 64, hipHostMallocMapped) != hipSuccess || !p) // and a few results behind them
+        Fail(PBAT_VBD_ERROR_OUT_OF_MEMORY, "hipHostMalloc of the vertex data's pinned memory failed");
+    hipError_t const e = hipHostGetDevicePointer(&d, p, 0);
+    if (e != hipSuccess)
+        (void)hipHostFree(p);
+    PBAT_HIP(e);
+    h.stage = p, h.stageDev = d, h.stageBytes = bytes;
 }
 
-void DownloadVec(pbat_vbd_integrator& h, float4 const* src, float* dst)
+// f(first, count) over n items of `bytes` each in pieces that the pinned memory holds.
+template <class F>
+void InPieces(pbat_vbd_integrator& h, size_t n, size_t bytes, F&& f)
 {
-    std::vector<float4> buf(static_cast<size_t>(h.nV));
-    PBAT_HIP(hipMemcpyAsync(buf.data(), src, buf.size() * sizeof(float4), hipMemcpyDeviceToHost, h.stream));
-    PBAT_HIP(hipStreamSynchronize(h.stream));
-    for (int64_t v = 0; v < h.nV; ++v)
-    {
-        int64_t const i = h.perm[v];
-        dst[3 * i] = buf[v].x;
-        dst[3 * i + 1] = buf[v].y;
-        dst[3 * i + 2] = buf[v].z;
-    }
+    EnsureStage(h);
+    size_t const piece = h.stageBytes / bytes / 256 * 256; // whole workgroups, 16-byte aligned
+    for (size_t first = 0; first < n; first += piece)
+        f(first, std::min(piece, n - first));
+}
+
+// Copy a 3 x nV host matrix (original numbering) into a float4 device array
+// (internal numbering).
+void UploadVec(pbat_vbd_integrator& h, float4* dst, float const* src, bool masses, float4* second)
+{
+    InPieces(h, static_cast<size_t>(h.nV), 3 * sizeof(float), [&](size_t first, size_t n) {
+        std::memcpy(h.stage, src + 3 * first, 3 * sizeof(float) * n);
+        float const* from = static_cast<float const*>(h.stageDev);
+        if (3 * sizeof(float) * n > kStageRead)
+        {
+            PBAT_HIP(hipMemcpyAsync(h.stageCopy.ptr, h.stage, 3 * sizeof(float) * n, hipMemcpyHostToDevice, h.stream));
+            from = h.stageCopy.ptr;
+        }
+        hipLaunchKernelGGL(device::UploadVertices, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, h.stream,
+                           from, static_cast<int const*>(h.ipermD.ptr),
+                           masses ? static_cast<float const*>(h.massD.ptr) : nullptr, static_cast<int>(first),
+                           static_cast<int>(n), dst, second);
+        PBAT_HIP(hipGetLastError());
+        PBAT_HIP(hipStreamSynchronize(h.stream));
+    });
+}
+
+template <class T, class S>
+void Download(pbat_vbd_integrator& h, S const* src, T* dst)
+{
+    InPieces(h, static_cast<size_t>(h.nV), 3 * sizeof(T), [&](size_t first, size_t n) {
+        hipLaunchKernelGGL((device::DownloadVertices<T, S>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
+                           h.stream, src, static_cast<int const*>(h.ipermD.ptr), static_cast<int>(first),
+                           static_cast<int>(n), static_cast<T*>(h.stageDev));
+        PBAT_HIP(hipGetLastError());
+        PBAT_HIP(hipStreamSynchronize(h.stream));
+        std::memcpy(dst + 3 * first, h.stage, 3 * sizeof(T) * n);
+    });
+}
+
+void DownloadVec(pbat_vbd_integrator& h, float4 const* src, float* dst) { Download(h, src, dst); }
+
+void DownloadVec(pbat_vbd_integrator& h, double const* src, double* dst) { Download(h, src, dst); }
+
+void DownloadFloats(pbat_vbd_integrator& h, double const* src, float* dst, size_t n)
+{
+    InPieces(h, n, sizeof(float), [&](size_t first, size_t count) {
+        hipLaunchKernelGGL(device::ToFloats, dim3(static_cast<unsigned>((count + 255) / 256)), dim3(256), 0, h.stream,
+                           src + first, static_cast<float*>(h.stageDev), static_cast<int>(count));
+        PBAT_HIP(hipGetLastError());
+        PBAT_HIP(hipStreamSynchronize(h.stream));
+        std::memcpy(dst + first, h.stage, sizeof(float) * count);
+    });
 }
 
 // Aggregates of the adjoint's two-level preconditioner: each mesh's updated
@@ -1227,10 +1288,9 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
     }
     for (int64_t i = 0; i < nV; ++i)
         h->massOrig[i] = static_cast<float>(d->m[i]);
-    UploadVec(*h, h->xm.ptr, x32.data(), h->massOrig.data());
-    UploadVec(*h, h->xt.ptr, x32.data(), nullptr);
-    UploadVec(*h, h->vel.ptr, v32.data(), nullptr);
-    UploadVec(*h, h->aext.ptr, a32.data(), nullptr);
+    UploadVec(*h, h->xm.ptr, x32.data(), true, h->xt.ptr);
+    UploadVec(*h, h->vel.ptr, v32.data(), false);
+    UploadVec(*h, h->aext.ptr, a32.data(), false);
     SetUpContact(*h, d);
     PBAT_HIP(hipStreamSynchronize(h->stream));
     *out = h.release();
@@ -1273,8 +1333,8 @@ void EnsureObjectiveBuffers(pbat_vbd_integrator& h)
         h.objGrad.allocate(3 * nV);
     }
     size_t const nb = static_cast<size_t>(std::max<int64_t>((h.nV + 255) / 256, kObjectiveBlocks));
-    if (h.objPart.n != 6 * nb + 6)
-        h.objPart.allocate(6 * nb + 6);
+    if (h.objPart.n != 6 * nb)
+        h.objPart.allocate(6 * nb);
 }
 
 // sim::vbd::Integrator::ObjectiveFunction and ObjectiveFunctionGradient
@@ -1291,7 +1351,9 @@ void ObjectiveOnDevice(pbat_vbd_integrator& h, float4 const* x, float4 const* xt
     size_t const nb = static_cast<size_t>(std::max(gridG, kObjectiveBlocks));
     double* partF = h.objPart.ptr;
     double* partG = h.objPart.ptr + 3 * nb;
-    double* sums = h.objPart.ptr + 6 * nb; // (K, U, .) then (|g|^2, ., .)
+    EnsureStage(h);
+    // (K, U, .) then (|g|^2, ., .), in pinned memory
+    double* const sums = reinterpret_cast<double*>(static_cast<char*>(h.stageDev) + h.stageBytes);
     device::TrEpilogue none{};
     hipLaunchKernelGGL(device::ObjectiveTerms, dim3(kObjectiveBlocks), dim3(256), 0, h.stream, x, xtil,
                        static_cast<float4 const*>(nullptr), static_cast<int4 const*>(h.tetv.ptr),
@@ -1306,24 +1368,15 @@ void ObjectiveOnDevice(pbat_vbd_integrator& h, float4 const* x, float4 const* xt
     hipLaunchKernelGGL(device::SumPartials3, dim3(1), dim3(256), 0, h.stream, static_cast<double const*>(partG),
                        std::max(gridG, 1), sums + 3, static_cast<double const*>(nullptr), none);
     PBAT_HIP(hipGetLastError());
-    double s[6];
-    PBAT_HIP(hipMemcpyAsync(s, sums, sizeof(s), hipMemcpyDeviceToHost, h.stream));
-    std::vector<double> g;
     if (gradOrig)
-    {
-        g.resize(3 * static_cast<size_t>(nV));
-        PBAT_HIP(hipMemcpyAsync(g.data(), h.objGrad.ptr, g.size() * sizeof(double), hipMemcpyDeviceToHost,
-                                h.stream));
-    }
-    PBAT_HIP(hipStreamSynchronize(h.stream));
+        DownloadVec(h, static_cast<double const*>(h.objGrad.ptr), gradOrig);
+    else
+        PBAT_HIP(hipStreamSynchronize(h.stream));
+    double const* const s = reinterpret_cast<double const*>(static_cast<char const*>(h.stage) + h.stageBytes);
     if (f)
         *f = 0.5 * s[0] + dt2 * s[1];
     if (r2)
         *r2 = s[3];
-    if (gradOrig)
-        for (int v = 0; v < nV; ++v)
-            for (int d = 0; d < 3; ++d)
-                gradOrig[3 * static_cast<size_t>(h.perm[v]) + d] = g[3 * static_cast<size_t>(v) + d];
 }
 
 void Objective(pbat_vbd_integrator& h, float const* x, float const* xtilde, float dt, double* f, double* grad,
@@ -1337,12 +1390,12 @@ void Objective(pbat_vbd_integrator& h, float const* x, float const* xtilde, floa
     float4 const* xl = h.xtil.ptr;
     if (x)
     {
-        UploadVec(h, h.objX.ptr, x, h.massOrig.data());
+        UploadVec(h, h.objX.ptr, x, true);
         xd = h.objX.ptr;
     }
     if (xtilde)
     {
-        UploadVec(h, h.objXtil.ptr, xtilde, nullptr);
+        UploadVec(h, h.objXtil.ptr, xtilde, false);
         xl = h.objXtil.ptr;
     }
     ObjectiveOnDevice(h, xd, xl, dt, f, grad, r2);
@@ -1899,8 +1952,7 @@ extern "C" int pbat_vbd_integrator_set_positions(pbat_vbd_integrator* h, const f
         CheckVertexArray(H, x, n, "positions");
         PBAT_HIP(hipSetDevice(H.device));
         H.rollout.Discard();
-        UploadVec(H, H.xm.ptr, x, H.massOrig.data());
-        UploadVec(H, H.xt.ptr, x, nullptr);
+        UploadVec(H, H.xm.ptr, x, true, H.xt.ptr);
     });
 }
 
@@ -1911,8 +1963,7 @@ extern "C" int pbat_vbd_integrator_set_velocities(pbat_vbd_integrator* h, const 
         CheckVertexArray(H, v, n, "velocities");
         PBAT_HIP(hipSetDevice(H.device));
         H.rollout.Discard();
-        UploadVec(H, H.vel.ptr, v, nullptr);
-        UploadVec(H, H.vprev.ptr, v, nullptr);
+        UploadVec(H, H.vel.ptr, v, false, H.vprev.ptr);
     });
 }
 
@@ -1923,7 +1974,7 @@ extern "C" int pbat_vbd_integrator_set_external_acceleration(pbat_vbd_integrator
         CheckVertexArray(H, a, n, "external acceleration");
         PBAT_HIP(hipSetDevice(H.device));
         H.rollout.Discard();
-        UploadVec(H, H.aext.ptr, a, nullptr);
+        UploadVec(H, H.aext.ptr, a, false);
     });
 }
 

