@@ -1300,6 +1300,8 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
 void WriteDense(std::string const& path, int64_t rows, int64_t cols, std::vector<double> const& colMajor,
                 int digits = 9);
 
+int GradientBlocks(int64_t nV) { return static_cast<int>((nV * device::kGradientLanes + 255) / 256); }
+
 // Buffers of the FP64 objective (allocated on first use). The vertex -> (tet,
 // local index) CSR over every vertex, Dirichlet ones included, comes from the
 // device's element table, in ascending tet order per vertex.
@@ -1332,7 +1334,7 @@ void EnsureObjectiveBuffers(pbat_vbd_integrator& h)
         h.objX.allocate(nV), h.objXtil.allocate(nV);
         h.objGrad.allocate(3 * nV);
     }
-    size_t const nb = static_cast<size_t>(std::max<int64_t>((h.nV + 255) / 256, kObjectiveBlocks));
+    size_t const nb = static_cast<size_t>(std::max(GradientBlocks(h.nV), kObjectiveBlocks));
     if (h.objPart.n != 6 * nb)
         h.objPart.allocate(6 * nb);
 }
@@ -1347,7 +1349,7 @@ void ObjectiveOnDevice(pbat_vbd_integrator& h, float4 const* x, float4 const* xt
 {
     EnsureObjectiveBuffers(h);
     int const nV = static_cast<int>(h.nV), nT = static_cast<int>(h.nT);
-    int const gridG = (nV + 255) / 256;
+    int const gridG = GradientBlocks(h.nV);
     size_t const nb = static_cast<size_t>(std::max(gridG, kObjectiveBlocks));
     double* partF = h.objPart.ptr;
     double* partG = h.objPart.ptr + 3 * nb;
