@@ -23,6 +23,7 @@
 #include <exception>
 #include <functional>
 #include <string>
+#include <limits>
 #include <thread>
 #include <vector>
 
@@ -1046,8 +1047,14 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
     int const gridN = Blocks(n);
     bool const twoLevel = cfg.solver == PBAT_VBD_ADJOINT_PCG_TWO_LEVEL && h.nAggregates > 0;
     bool const fused = cfg.solver == PBAT_VBD_ADJOINT_PCG_JACOBI || cfg.solver == PBAT_VBD_ADJOINT_PCG_TWO_LEVEL;
-    // fused chunks hold an even number of iterations: the two direction buffers swap
-    int const check = fused ? (std::max(1, cfg.check_every) + 1) / 2 * 2 : std::max(1, cfg.check_every);
+    // fused chunks hold an even number of iterations, since the buffers of the sums swap,
+    // and few of them when the launches queued behind the last iteration are long to pass:
+    // 5 us each at 224,000 rows (a rollout of 64 meshes: 136.1 ms in chunks of 10, 132.3
+    // in chunks of 4), 2 us at 12,000, where more graph launches cost as much (a solve
+    // 2.99 ms, 3.04)
+    int const maxChunk = n >= 65536 ? 4 : std::numeric_limits<int>::max();
+    int const check = fused ? std::min((std::max(1, cfg.check_every) + 1) / 2 * 2, maxChunk)
+                            : std::max(1, cfg.check_every);
     AssembleBsr(h, xs, dt, fused);
     // the fused solvers work on aggregate-major rows: y and b gathered into that
     // order here, y scattered back at the end
