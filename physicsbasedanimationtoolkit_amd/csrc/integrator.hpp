@@ -202,6 +202,7 @@ struct RolloutState
     DeviceArray<int> rowVertex, meshOfRow, aggOfRow, aggRows;
     DeviceArray<int> incPtr, incCode;
     DeviceArray<int4> incSlot;
+    DeviceArray<uint2> rowSources; // set: device::RowAssembleShort
     DeviceArray<float4> bsrA, bsrB;
     DeviceArray<float> bsrC;
     int bsrMaxRow = 0;

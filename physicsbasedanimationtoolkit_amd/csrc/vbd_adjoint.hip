@@ -19,11 +19,12 @@
 #include "vbd_hessian_kernels.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <exception>
 #include <functional>
-#include <string>
 #include <limits>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -481,12 +482,50 @@ void BuildBsrPattern(pbat_vbd_integrator& h, bool aggregateOrder)
     R.bsrBlockRow.upload(blockRow, h.stream);
     R.bsrA.allocate(nBlocks), R.bsrB.allocate(nBlocks), R.bsrC.allocate(nBlocks);
     R.rowVertex.upload(rowVertex, h.stream);
+    // sources of the off-diagonal blocks for RowAssembleShort, if it takes the pattern
+    std::vector<uint2> sources;
+    if (maxRow <= 32)
+    {
+        std::atomic<bool> fits{true};
+        sources.assign(nBlocks, make_uint2(~0u, ~0u));
+        HostParallel(nUpd, nParts, [&](int r0, int r1, int) {
+            unsigned char used[32];
+            for (int s = r0; s < r1 && fits; ++s)
+            {
+                std::fill(std::begin(used), std::end(used), static_cast<unsigned char>(0));
+                bool ok = incPtr[s + 1] - incPtr[s] <= 32;
+                for (int t = incPtr[s]; t < incPtr[s + 1] && ok; ++t)
+                {
+                    int const s4[4] = {incSlot[t].x, incSlot[t].y, incSlot[t].z, incSlot[t].w};
+                    for (int l = 0; l < 4; ++l)
+                    {
+                        if (l == (incCode[t] & 3) || s4[l] < 0)
+                            continue;
+                        int const n = used[s4[l]]++;
+                        uint2& w = sources[rowPtr[s] + s4[l]];
+                        if (n < 8)
+                            (n < 4 ? w.x : w.y) ^= (255u ^ static_cast<unsigned>(4 * (t - incPtr[s]) + l)) << (8 * (n & 3));
+                        else
+                            ok = false;
+                    }
+                }
+                if (!ok)
+                    fits = false;
+            }
+        });
+        if (!fits)
+            sources.clear();
+    }
+    R.rowSources.reset();
     if (maxRow <= kRowAssembleMaxRow)
     {
         // row-major assembly: the rows' incidences and their tets' row positions
         R.incPtr.upload(incPtr, h.stream);
         R.incCode.upload(incCode, h.stream);
-        R.incSlot.upload(incSlot, h.stream);
+        if (!sources.empty())
+            R.rowSources.upload(sources, h.stream), R.incSlot.reset();
+        else
+            R.incSlot.upload(incSlot, h.stream);
     }
     else
     {
@@ -694,7 +733,10 @@ void AssembleBsr(pbat_vbd_integrator& h, float4 const* xs, float dt, bool aggreg
     a.dinv = R.dinv.ptr, a.rowVertex = R.rowVertex.ptr;
     dim3 const grid((p.nRows + 1) / 2);
     int const nb = (R.bsrMaxRow + 31) / 32;
-    if (nb <= 1)
+    a.sources = R.rowSources.ptr;
+    if (a.sources)
+        hipLaunchKernelGGL(device::RowAssembleShort, grid, dim3(64), 0, h.stream, a);
+    else if (nb <= 1)
         hipLaunchKernelGGL(device::RowAssemble<1>, grid, dim3(64), 0, h.stream, a);
     else if (nb == 2)
         hipLaunchKernelGGL(device::RowAssemble<2>, grid, dim3(64), 0, h.stream, a);

@@ -193,6 +193,32 @@ struct TetHessian
     }
 };
 
+template <int kCtrl>
+__device__ __forceinline__ double DppRead(double x)
+{
+    int const lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), kCtrl, 0xF, 0xF, false);
+    int const hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), kCtrl, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+
+template <int L>
+__device__ __forceinline__ double GroupSum(double x)
+{
+    if constexpr (L >= 2)
+        x += DppRead<0xB1>(x);
+    if constexpr (L >= 4)
+        x += DppRead<0x4E>(x);
+    if constexpr (L >= 8)
+        x += DppRead<0x141>(x);
+    if constexpr (L >= 16)
+        x += DppRead<0x140>(x);
+    if constexpr (L >= 32)
+        x += __shfl_xor(x, 16);
+    if constexpr (L >= 64)
+        x += __shfl_xor(x, 32);
+    return x;
+}
+
 // Row-major assembly: incidences of row i (tet e, local vertex la of the row
 // vertex) in incCode[incPtr[i] .. incPtr[i + 1]) as 4 e + la, ascending e;
 // incSlot holds, per incidence, the position in the row of the tet's local
@@ -205,6 +231,7 @@ struct RowAssembleArgs
     int const* __restrict__ incPtr;
     int const* __restrict__ incCode;
     int4 const* __restrict__ incSlot;
+    uint2 const* __restrict__ sources; // RowAssembleShort
     int const* __restrict__ rowPtr;
     int const* __restrict__ col;
     int nRows;
@@ -361,6 +388,94 @@ __global__ __launch_bounds__(64) void RowAssemble(RowAssembleArgs a)
                                     static_cast<float>(H[7]));
         a.v.c[kBlock] = static_cast<float>(H[8]);
     }
+}
+
+// The same for patterns whose rows have at most 32 blocks and 32 incidences and whose
+// off-diagonal blocks have at most 8 sources: the sources of a block are listed (bytes
+// 4 incidence + local vertex, ascending, 255 behind the last), so no lane looks for
+// them, the staged values lie value-major (lanes on different banks), and the
+// symmetric diagonal is summed as 6 values across DPP rows. 224,000 rows 346 -> 189 us,
+// 36,000 rows 63 -> 34; what is left is the FP64 arithmetic of a tet per lane.
+[[maybe_unused]] static __global__ __launch_bounds__(64) void RowAssembleShort(RowAssembleArgs a)
+{
+    constexpr int L = 32;
+    __shared__ float stage[2][36][L + 1];
+    int const lane = static_cast<int>(threadIdx.x) & (L - 1), half = static_cast<int>(threadIdx.x) >> 5;
+    int const i = static_cast<int>(blockIdx.x) * 2 + half;
+    int kb = 0, ke = 0, rb = 0, nb = 0;
+    if (i < a.nRows)
+        kb = a.incPtr[i], ke = a.incPtr[i + 1], rb = a.rowPtr[i], nb = a.rowPtr[i + 1] - rb;
+    uint2 const list = lane < nb ? a.sources[rb + lane] : make_uint2(~0u, ~0u);
+    bool const isDiag = lane < nb && a.col[rb + lane] == i;
+    double d6[6] = {0., 0., 0., 0., 0., 0.};
+    if (kb + lane < ke)
+    {
+        int const code = a.incCode[kb + lane];
+        int const e = code >> 2, la = code & 3;
+        TetHessian const T(a.xs, a.tetv[e], a.tgp[3 * e], a.tgp[3 * e + 1], a.tgp[3 * e + 2]);
+        double ga[3], ca[3];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+        {
+            ga[c] = la == 0 ? T.g[0][c] : la == 1 ? T.g[1][c] : la == 2 ? T.g[2][c] : T.g[3][c];
+            ca[c] = la == 0 ? T.cg[0][c] : la == 1 ? T.cg[1][c] : la == 2 ? T.cg[2][c] : T.cg[3][c];
+        }
+        // the block (la, la), whose skew part vanishes
+        double const dg = T.wmu * (ga[0] * ga[0] + ga[1] * ga[1] + ga[2] * ga[2]);
+        d6[0] = dg + T.wlam * ca[0] * ca[0], d6[1] = T.wlam * ca[0] * ca[1], d6[2] = T.wlam * ca[0] * ca[2];
+        d6[3] = dg + T.wlam * ca[1] * ca[1], d6[4] = T.wlam * ca[1] * ca[2], d6[5] = dg + T.wlam * ca[2] * ca[2];
+        auto put = [&](int lb, double const (&H)[9]) {
+#pragma unroll
+            for (int c = 0; c < 9; ++c)
+                stage[half][9 * lb + c][lane] = static_cast<float>(H[c]);
+        };
+        double H[9];
+        T.Block<0>(ga, ca, H), put(0, H);
+        T.Block<1>(ga, ca, H), put(1, H);
+        T.Block<2>(ga, ca, H), put(2, H);
+        T.Block<3>(ga, ca, H), put(3, H);
+    }
+#pragma unroll
+    for (int c = 0; c < 6; ++c)
+        d6[c] = GroupSum<L>(d6[c]);
+    __syncthreads();
+    if (lane >= nb)
+        return;
+    double H[9];
+    if (isDiag)
+    {
+        double const m = double(a.xs[a.rowVertex[i]].w) * a.invDt2;
+        H[0] = d6[0] + m, H[4] = d6[3] + m, H[8] = d6[5] + m;
+        H[1] = H[3] = d6[1], H[2] = H[6] = d6[2], H[5] = H[7] = d6[4];
+        Inverse3 const C(H[0], H[1], H[2], H[4], H[5], H[8]);
+        a.dinv[2 * i] = make_float4(static_cast<float>(C.c00 * C.inv), static_cast<float>(C.c01 * C.inv),
+                                    static_cast<float>(C.c02 * C.inv), static_cast<float>(C.c11 * C.inv));
+        a.dinv[2 * i + 1] =
+            make_float4(static_cast<float>(C.c12 * C.inv), static_cast<float>(C.c22 * C.inv), 0.f, 0.f);
+    }
+    else
+    {
+#pragma unroll
+        for (int c = 0; c < 9; ++c)
+            H[c] = 0.;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+        {
+            unsigned int const b = ((k < 4 ? list.x : list.y) >> (8 * (k & 3))) & 255u;
+            if (b == 255u)
+                break;
+            float const* const from = &stage[half][9 * (b & 3u)][b >> 2];
+#pragma unroll
+            for (int c = 0; c < 9; ++c)
+                H[c] += from[c * (L + 1)];
+        }
+    }
+    int const k = rb + lane;
+    a.v.a[k] = make_float4(static_cast<float>(H[0]), static_cast<float>(H[1]), static_cast<float>(H[2]),
+                           static_cast<float>(H[3]));
+    a.v.b[k] = make_float4(static_cast<float>(H[4]), static_cast<float>(H[5]), static_cast<float>(H[6]),
+                           static_cast<float>(H[7]));
+    a.v.c[k] = static_cast<float>(H[8]);
 }
 
 enum class BsrMode : int
@@ -536,14 +651,6 @@ inline ChebyConstants MakeCheby()
 
 // Sum over the wave in a fixed order, in every lane: 16-lane rows by DPP, then
 // the four row sums in order.
-template <int kCtrl>
-__device__ __forceinline__ double DppRead(double x)
-{
-    int const lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), kCtrl, 0xF, 0xF, false);
-    int const hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), kCtrl, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-
 __device__ __forceinline__ double ReadLane(double x, int lane)
 {
     return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
@@ -661,24 +768,6 @@ __device__ __forceinline__ float4 ApplyInverse(float4 const& D0, float4 const& D
 {
     return make_float4(D0.x * x + D0.y * y + D0.z * z, D0.y * x + D0.w * y + D1.x * z, D0.z * x + D1.x * y + D1.y * z,
                        0.f);
-}
-
-template <int L>
-__device__ __forceinline__ double GroupSum(double x)
-{
-    if constexpr (L >= 2)
-        x += DppRead<0xB1>(x);
-    if constexpr (L >= 4)
-        x += DppRead<0x4E>(x);
-    if constexpr (L >= 8)
-        x += DppRead<0x141>(x);
-    if constexpr (L >= 16)
-        x += DppRead<0x140>(x);
-    if constexpr (L >= 32)
-        x += __shfl_xor(x, 16);
-    if constexpr (L >= 64)
-        x += __shfl_xor(x, 32);
-    return x;
 }
 
 // Blocks of the row that thread t works on, of the rows [first, end).
