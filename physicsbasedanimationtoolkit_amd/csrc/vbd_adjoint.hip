@@ -924,7 +924,7 @@ int ReadLive(pbat_vbd_integrator& h)
     return static_cast<int>(std::count(done.begin(), done.end(), 0));
 }
 
-// Host-mapped copy of the per-mesh done flags (written by CgFinish) and the
+// Host-mapped copy of the per-mesh done flags (written by CgUpdate1) and the
 // chunk-end events, allocated on first use.
 void EnsureDoneHost(pbat_vbd_integrator& h)
 {
@@ -998,7 +998,8 @@ SolveResult ReadResult(pbat_vbd_integrator& h)
 //   (4) BsrPoly: w = H z, z . w.
 // 32^3 workload, per iteration: 27.4 us in four launches with the classical
 // recurrences and the coarse correction of block Jacobi alone.
-// The symmetric Gauss-Seidel preconditioner keeps the four-launch iteration
+// The symmetric Gauss-Seidel preconditioner runs in one launch on small meshes
+// (SolveLocal); larger ones keep the launches per colour:
 //   q = H p and p . q; y, r update with z = 0; a forward and a reverse coloured
 //   Gauss-Seidel pass for z with r . z; one workgroup: scalars; p = z + beta p.
 //
@@ -1272,7 +1273,7 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
     }
     // Fused iterations: the host polls the live-mesh count one chunk behind.
     // Chunk c + 1 is queued before the host waits for the end of chunk c and
-    // reads the done flags the finish kernel mirrors into host memory, so the
+    // reads the done flags CgUpdate1 mirrors into host memory, so the
     // device does not idle during the poll. A chunk queued after every mesh has
     // converged (or that starts with every mesh converged) changes nothing: each
     // of its kernels returns at once for a mesh whose done flag is set.
