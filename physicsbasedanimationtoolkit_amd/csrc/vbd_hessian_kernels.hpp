@@ -1385,6 +1385,12 @@ struct LocalRow
         ranges[c] = a.ranges[static_cast<size_t>(m) * (nC + 1) + c];
     __syncthreads();
     int const nR = ranges[nC].lbeg; // the fixed vertices follow
+    if (nR == 0) // every vertex of the mesh is fixed: no row to read
+    {
+        if (t == 0)
+            P[kBb * nM] = P[kRrLast * nM] = 0., a.cg.F[kDone * nM + m] = 1;
+        return;
+    }
     int const colour0 = ranges[0].count, lastColour = ranges[nC - 1].lbeg;
     auto sum3 = [&](double u, double v, double w, double (&out)[3]) {
         double const x[3] = {WaveSum(u), WaveSum(v), WaveSum(w)};

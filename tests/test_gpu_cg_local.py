@@ -46,17 +46,20 @@ def test_residual(gpu_device, mesh, amplitude):
     assert stats["iterations"] == 1
 
 
-def test_batch(gpu_device):
+@pytest.mark.parametrize("fixed", [0, 1, 4])
+def test_batch(gpu_device, fixed):
     X, E, _ = grid(2, 2, 2)
-    scenes = [loose(1), (X, E, np.arange(X.shape[1])), grid(7, 3, 5), fan(40), grid(2, 9, 6)]
+    scenes = [loose(1), grid(7, 3, 5), fan(40), grid(2, 9, 6)]
+    scenes.insert(fixed, (X, E, np.arange(X.shape[1])))
     batch = pbat.gpu.vbd.BatchIntegrator([build(*s)[0] for s in scenes])
     xs, bs, frees = zip(*[pose(*s) for s in scenes])
-    bs = [b * (k != 2) for k, b in enumerate(bs)]
+    zero = 2 if fixed < 2 else 1  # the (7, 3, 5) grid
+    bs = [b * (k != zero) for k, b in enumerate(bs)]
     y, _ = batch.adjoint_solve(np.concatenate(xs, axis=1), DT, np.concatenate(bs, axis=1), solver="pcg",
                                max_iterations=400, tolerance=1e-5)
     for k, (s, x, b, free) in enumerate(zip(scenes, xs, bs, frees)):
         yk = y[:, batch.offsets[k]:batch.offsets[k + 1]]
-        if k in (1, 2):
+        if k in (fixed, zero):
             assert not yk.any()
         else:
             assert residual(pbat.gpu.vbd.Integrator(build(*s)[0]), x, yk, b, free) <= 2e-5
