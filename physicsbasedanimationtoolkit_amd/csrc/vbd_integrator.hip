@@ -660,7 +660,8 @@ void EnsureStage(pbat_vbd_integrator& h)
         h.stageCopy.allocate(bytes / sizeof(float));
     PBAT_HIP(hipStreamSynchronize(h.stream));
     void *p = nullptr, *d = nullptr;
-    if (hipHostMalloc(&p, bytes + 64, hipHostMallocMapped) != hipSuccess || !p) // and a few results behind them
+    if (hipHostMalloc(&p, bytes + 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        !p) // and a few results behind them
         Fail(PBAT_VBD_ERROR_OUT_OF_MEMORY, "hipHostMalloc of the vertex data's pinned memory failed");
     hipError_t const e = hipHostGetDevicePointer(&d, p, 0);
     if (e != hipSuccess)
