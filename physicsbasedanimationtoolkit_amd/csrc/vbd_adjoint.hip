@@ -1056,7 +1056,7 @@ SolveResult SolveLocal(pbat_vbd_integrator& h, device::CgState const& cg, float4
                            nV);
     }
     device::CgLocalArgs a{};
-    a.rows = R.cgLocalRows.ptr, a.place = R.cgLocalPlace.ptr, a.nBlocks = static_cast<int>(R.bsrCol.n);
+    a.rows = R.cgLocalRows.ptr, a.place = R.cgLocalPlace.ptr;
     a.va = R.bsrA.ptr, a.vb = R.bsrB.ptr, a.vc = R.bsrC.ptr, a.dinvRows = R.dinv.ptr, a.dinv = R.cgLocalDinv.ptr;
     a.ranges = h.star.localRanges.ptr, a.meshes = h.star.localMeshes.ptr, a.verts = h.star.localVerts.ptr;
     auto vec = [](DeviceArray<double> const& v) { return reinterpret_cast<device::Vec3d*>(v.ptr); };

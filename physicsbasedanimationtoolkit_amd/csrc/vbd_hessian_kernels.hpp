@@ -1279,7 +1279,7 @@ struct CgLocalArgs
     Vec3d* w;
     float4* z;
     CgState cg;
-    int nColors, maxRows, nBlocks;
+    int nColors, maxRows;
 };
 
 // Block extents of each place's row, and the places of its columns (ascending).
@@ -1305,7 +1305,8 @@ struct CgLocalArgs
 // Blocks [lo, hi) of one row times z by the row's kCgLocalLanes lanes: up to kSlots of
 // a lane loaded ahead (Load), as many as the longest row of the wave takes (a load
 // costs its cycles for every lane, used or not), then summed (Sum), longer rows in a
-// loop.
+// loop. Slots past the end hold a block of the same row, summed with a zero vector:
+// another mesh's block could be non-finite. first is the row's first block.
 struct LocalRow
 {
     static constexpr int kSlots = 4;
@@ -1318,7 +1319,7 @@ struct LocalRow
     {
         return *reinterpret_cast<V const*>(reinterpret_cast<char const*>(p) + bytes);
     }
-    __device__ __forceinline__ void Load(CgLocalArgs const& a, int lo_, int hi_, int lane)
+    __device__ __forceinline__ void Load(CgLocalArgs const& a, int first, int lo_, int hi_, int lane)
     {
         lo = lo_ + lane, hi = hi_;
         slots = 0;
@@ -1327,7 +1328,7 @@ struct LocalRow
             if (__any(lo + u * kCgLocalLanes < hi))
             {
                 slots = u + 1;
-                int const k = min(max(min(lo + u * kCgLocalLanes, hi - 1), 0), a.nBlocks - 1);
+                int const k = max(min(lo + u * kCgLocalLanes, hi - 1), first);
                 unsigned int const o = static_cast<unsigned int>(k) * 4u; // 32-bit offsets from scalar bases
                 A[u] = At(a.va, o * 4u), B[u] = At(a.vb, o * 4u), C[u] = At(a.vc, o), j[u] = At(a.place, o);
             }
@@ -1418,7 +1419,7 @@ struct LocalRow
     auto blocks = [&](int k, int r) {
         int const i = clamped(ranges[colourOf(k)], r);
         bool const forward = k < nC - 1;
-        q.Load(a, forward ? e.x : e.z, forward ? e.y : e.w, lane);
+        q.Load(a, e.x, forward ? e.x : e.z, forward ? e.y : e.w, lane);
         D0 = a.dinv[2 * i], D1 = a.dinv[2 * i + 1];
     };
     // z = M^-1 r: the first colour's rows have z = D^-1 r already
@@ -1486,7 +1487,7 @@ struct LocalRow
         int4 x = a.rows[min(r, nR - 1)];
         for (int w0 = t / 64 * (64 / L); w0 < nR; w0 += G, r += G)
         {
-            q.Load(a, x.x, whole ? x.w : x.z, lane);
+            q.Load(a, x.x, x.x, whole ? x.w : x.z, lane);
             rq = a.r[min(r, nR - 1)];
             x = a.rows[min(r + G, nR - 1)];
             double h[3];
