@@ -1080,13 +1080,39 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
     for (int64_t v = 0; v < nUpd; ++v)
         h->maxDegree = std::max<int64_t>(h->maxDegree, P[v + 1] - P[v]);
     size_t const nIncUpd = static_cast<size_t>(P[nUpd]);
-    // The adjoint's incidence records: the tet's other three vertices (local order)
-    // with their GP rows, w*mu (in the id word) and w*lambda. The sweep's star
-    // records: with gamma_k = g_k . g (the other rows with the own row g) and kappa =
-    // det of the other three rows, A = w lambda kappa^2 and B = kappa (w lambda +
-    // w mu) per tet and Gamma_j = sum of w mu gamma_k per neighbour, from the FP64 GP
-    // and material; shape keeps (gamma_a, gamma_b, gamma_c, kappa) for later changes
-    // of the moduli.
+    // Incidence k's tet: its other three vertices (local order) with their GP rows g_k,
+    // gamma_k = g_k . g with the own row g, and kappa = det of the other three rows.
+    struct TetShape
+    {
+        int ids[3];
+        double g[3][3], gamma[3], kappa;
+    };
+    auto shapeOf = [&](int64_t k) {
+        int64_t const e = d->GVGe[k];
+        int const il = static_cast<int>(d->GVGilocal[k]);
+        double const* G = d->GP + 12 * e; // G(r, c) = G[4c + r]
+        TetShape T{};
+        int n = 0;
+        for (int j = 0; j < 4; ++j)
+        {
+            if (j == il)
+                continue;
+            T.ids[n] = TV4(TV[e], j);
+            for (int c = 0; c < 3; ++c)
+                T.g[n][c] = G[4 * c + j], T.gamma[n] += G[4 * c + j] * G[4 * c + il];
+            ++n;
+        }
+        T.kappa = T.g[0][0] * (T.g[1][1] * T.g[2][2] - T.g[1][2] * T.g[2][1]) -
+                  T.g[0][1] * (T.g[1][0] * T.g[2][2] - T.g[1][2] * T.g[2][0]) +
+                  T.g[0][2] * (T.g[1][0] * T.g[2][1] - T.g[1][1] * T.g[2][0]);
+        return T;
+    };
+    // The adjoint's incidence records: the tet's other three vertices with their GP
+    // rows, w*mu (in the id word) and w*lambda. The sweep's star records: A = w lambda
+    // kappa^2 and B = kappa (w lambda + w mu) per tet and Gamma_j = sum of w mu gamma_k
+    // per neighbour (wide rows: each tet's w mu gamma_k), from the FP64 GP and material
+    // and rounded once; shape keeps (gamma_a, gamma_b, gamma_c, kappa) for later
+    // changes of the moduli.
     {
         std::vector<int4> slots(static_cast<size_t>(nT), make_int4(-1, -1, -1, -1));
         HostIncidenceRecords R;
@@ -1119,43 +1145,26 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
                 size_t const slot = static_cast<size_t>(P[v] + (k - k0));
                 int4& sl = slots[e];
                 (il == 0 ? sl.x : il == 1 ? sl.y : il == 2 ? sl.z : sl.w) = static_cast<int>(slot);
-                double const* G = d->GP + 12 * e; // G(r, c) = G[4c + r]
                 double const wmu = d->wg[e] * d->lame[2 * e], wlam = d->wg[e] * d->lame[2 * e + 1];
-                int ids[3], n = 0;
-                double gd[3][3], own[3];
-                for (int c = 0; c < 3; ++c)
-                    own[c] = G[4 * c + il];
-                for (int j = 0; j < 4; ++j)
-                {
-                    if (j == il)
-                        continue;
-                    ids[n] = TV4(TV[e], j);
-                    for (int c = 0; c < 3; ++c)
-                        gd[n][c] = G[4 * c + j];
-                    ++n;
-                }
+                TetShape const T = shapeOf(k);
                 float4 const m = G4[3 * e + 2]; // (., w*mu, w*lambda, alpha)
                 int wmuBits;
                 std::memcpy(&wmuBits, &m.y, sizeof(int));
-                auto f = [&](int r, int c) { return static_cast<float>(gd[r][c]); };
-                R.ids[slot] = make_int4(ids[0], ids[1], ids[2], wmuBits);
+                auto f = [&](int r, int c) { return static_cast<float>(T.g[r][c]); };
+                R.ids[slot] = make_int4(T.ids[0], T.ids[1], T.ids[2], wmuBits);
                 R.g0[slot] = make_float4(f(0, 0), f(0, 1), f(0, 2), f(1, 0));
                 R.g1[slot] = make_float4(f(1, 1), f(1, 2), f(2, 0), f(2, 1));
                 R.g2[slot] = make_float2(f(2, 2), m.z);
-                auto dot = [](double const* a, double const* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; };
-                double const kappa = gd[0][0] * (gd[1][1] * gd[2][2] - gd[1][2] * gd[2][1]) -
-                                     gd[0][1] * (gd[1][0] * gd[2][2] - gd[1][2] * gd[2][0]) +
-                                     gd[0][2] * (gd[1][0] * gd[2][1] - gd[1][1] * gd[2][0]);
-                double const gamma[3] = {dot(gd[0], own), dot(gd[1], own), dot(gd[2], own)};
                 for (int j = 0; j < 3; ++j)
-                    sum[at[ids[j]]] += wmu * gamma[j];
+                    sum[at[T.ids[j]]] += wmu * T.gamma[j];
                 // positions of a wide row do not fit; VbdSweepWide reads none
-                inc[slot] = device::StarInc{static_cast<unsigned>(at[ids[0]]) | static_cast<unsigned>(at[ids[1]]) << 8 |
-                                                static_cast<unsigned>(at[ids[2]]) << 16,
-                                            static_cast<float>(wlam * kappa * kappa),
-                                            static_cast<float>(kappa * (wlam + wmu))};
-                shape[slot] = make_float4(static_cast<float>(gamma[0]), static_cast<float>(gamma[1]),
-                                          static_cast<float>(gamma[2]), static_cast<float>(kappa));
+                inc[slot] = device::StarInc{static_cast<unsigned>(at[T.ids[0]]) |
+                                                static_cast<unsigned>(at[T.ids[1]]) << 8 |
+                                                static_cast<unsigned>(at[T.ids[2]]) << 16,
+                                            static_cast<float>(wlam * T.kappa * T.kappa),
+                                            static_cast<float>(T.kappa * (wlam + wmu))};
+                shape[slot] = make_float4(static_cast<float>(T.gamma[0]), static_cast<float>(T.gamma[1]),
+                                          static_cast<float>(T.gamma[2]), static_cast<float>(T.kappa));
                 tet[slot] = static_cast<int>(e);
             }
             // a row too long for the 8-bit positions, or more neighbours than 32 bits index
@@ -1185,14 +1194,17 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
         {
             std::vector<int4> wideIds(nIncUpd);
             std::vector<float4> wideGeo(nIncUpd);
-            for (size_t k = 0; k < nIncUpd; ++k)
-            {
-                float const wmu = G4[3 * static_cast<size_t>(tet[k]) + 2].y;
-                int bits;
-                std::memcpy(&bits, &inc[k].A, sizeof(int));
-                wideIds[k] = make_int4(R.ids[k].x, R.ids[k].y, R.ids[k].z, bits);
-                wideGeo[k] = make_float4(wmu * shape[k].x, wmu * shape[k].y, wmu * shape[k].z, inc[k].B);
-            }
+            for (int64_t v = 0; v < nUpd; ++v)
+                for (int slot = P[v]; slot < P[v + 1]; ++slot)
+                {
+                    TetShape const T = shapeOf(d->GVGp[h->perm[v]] + (slot - P[v]));
+                    double const wmu = d->wg[tet[slot]] * d->lame[2 * static_cast<size_t>(tet[slot])];
+                    auto f = [&](int j) { return static_cast<float>(wmu * T.gamma[j]); };
+                    int bits;
+                    std::memcpy(&bits, &inc[slot].A, sizeof(int));
+                    wideIds[slot] = make_int4(T.ids[0], T.ids[1], T.ids[2], bits);
+                    wideGeo[slot] = make_float4(f(0), f(1), f(2), inc[slot].B);
+                }
             h->star.wideIds.upload(wideIds, h->stream);
             h->star.wideGeo.upload(wideGeo, h->stream);
             PBAT_HIP(hipStreamSynchronize(h->stream));
