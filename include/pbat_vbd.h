@@ -204,7 +204,17 @@ typedef struct pbat_vbd_sweep_config {
 
 /* Set / read the sweep shape. get_ reports the values in effect (automatic
  * choices resolved). fixed_stride = 1 fails if the mesh's degree spread made
- * the library skip the fixed-stride copy at construction. */
+ * the library skip the fixed-stride copy at construction. With the automatic
+ * shape (lanes and incidences 0, the default), handles whose meshes are all
+ * small (no colour of a mesh beyond 128 vertices, no vertex beyond 16
+ * neighbours or 24 tets, a mesh's positions and targets within 64 KB) and that
+ * step plain or Chebyshev iterations without contact run a whole step in one
+ * launch, a workgroup per mesh. get_ then reports the lanes per vertex of the
+ * largest mesh there, and setting these values keeps that step; any other
+ * shape takes one launch per colour. The automatic shape depends on all meshes
+ * of a handle, and lanes that sum a vertex's terms in another order round
+ * differently: a mesh gives the same bits alone and in a batch when both are
+ * set to one shape that takes the launches. */
 int pbat_vbd_integrator_set_sweep_config(pbat_vbd_integrator* h, const pbat_vbd_sweep_config* config);
 int pbat_vbd_integrator_get_sweep_config(pbat_vbd_integrator* h, pbat_vbd_sweep_config* config);
 /* Autotuner: times `sweeps` full colour sweeps at substep dt for every

@@ -2083,8 +2083,10 @@ extern "C" int pbat_vbd_integrator_set_sweep_config(pbat_vbd_integrator* h, cons
         if (config->fixed_stride && H.ellStride == 0)
             Fail(PBAT_VBD_ERROR_INVALID_ARGUMENT,
                  "fixed-stride incidence rows are not available for this mesh (degree spread too large)");
-        H.lanes = lanes;
-        H.perLane = perLane;
+        // the shape get_ reports for the one-launch step keeps that step: setting what was
+        // read changes nothing
+        if (!StepsLocally(H) || lanes != EffectiveLanes(H) || perLane != EffectivePerLane(H))
+            H.lanes = lanes, H.perLane = perLane;
         H.xcdRemap = config->xcd_remap != 0;
         H.ntStream = config->nontemporal != 0;
         H.useEll = config->fixed_stride != 0;

@@ -223,7 +223,9 @@ class Integrator:
                          nontemporal: bool = False, fixed_stride: bool | None = None) -> None:
         """Sweep-kernel shape: lanes per vertex (0 = auto), incidences prefetched per
         lane (0 = auto, else 1..4), XCD-aware workgroup order, non-temporal stream
-        loads, fixed-stride (ELL) incidence rows (None = keep the current layout)."""
+        loads, fixed-stride (ELL) incidence rows (None = keep the current layout). Small
+        meshes run a whole step in one launch while the shape is automatic or what
+        ``sweep_config`` reports for it."""
         if fixed_stride is None:
             fixed_stride = self.sweep_config()["fixed_stride"]
         c = _native.SweepConfig(int(lanes), int(incidences_per_lane), int(bool(xcd_remap)), int(bool(nontemporal)),
