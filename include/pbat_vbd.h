@@ -222,7 +222,10 @@ int pbat_vbd_integrator_get_sweep_config(pbat_vbd_integrator* h, pbat_vbd_sweep_
  * on/off, fixed-stride/CSR rows) and keeps the fastest; the simulation state
  * is restored afterwards. timings (nullable, >= 192 doubles) receives up to 32
  * rows of (lanes, incidences per lane, xcd remap, non-temporal, fixed stride,
- * microseconds per sweep); *n_candidates the number of candidates timed. */
+ * microseconds per sweep); *n_candidates the number of candidates timed. Handles
+ * that can run a step in one launch time it as the first row, with lanes and
+ * incidences 0 (the automatic shape) and its begin and end kernels in the time;
+ * the other settings have no effect there. */
 int pbat_vbd_integrator_autotune(pbat_vbd_integrator* h, float dt, int32_t sweeps, double* timings,
                                  int32_t* n_candidates);
 /* Capture each Step's launch sequence in a hipGraph and replay it (default on). */
@@ -403,8 +406,9 @@ int pbat_vbd_integrator_trust_region_log(pbat_vbd_integrator* h, double* t, int3
  * bracket each replay of the captured step graph (which also holds the substep
  * begin/end kernels), or, with graph capture off, each substep's back-to-back
  * sweep launches. pbat_vbd_integrator_sweep_timing returns (summed event ms,
- * number of sweep launches inside the brackets) since the last reset. No
- * reference counterpart. */
+ * number of sweep launches inside the brackets) since the last reset. A step in
+ * one launch (see pbat_vbd_sweep_config) counts as one sweep launch, its begin
+ * and end included. No reference counterpart. */
 int pbat_vbd_integrator_set_timing(pbat_vbd_integrator* h, int32_t enabled);
 int pbat_vbd_integrator_sweep_timing(pbat_vbd_integrator* h, double* total_ms, int64_t* launches, int32_t reset);
 

@@ -1672,7 +1672,9 @@ void TracedStep(pbat_vbd_integrator& h, float dt, int iterations, int substeps, 
 // fastest. Device state is saved before and restored after, so the simulation
 // is unchanged. Candidates: lanes L in {2..64} with the natural prefetch depth
 // K = ceil(maxDegree / L) (when K <= 4), each with and without the XCD order
-// and with and without non-temporal loads of the incidence stream.
+// and with and without non-temporal loads of the incidence stream. Handles of small
+// meshes time the one-launch step first and, so that every candidate has its row, at
+// most kMaxTuneRows - 1 launch shapes.
 constexpr int kMaxTuneRows = 32;
 
 void Autotune(pbat_vbd_integrator& h, float dt, int sweeps, double* timingsUs, int32_t* nCandidates)
@@ -1725,15 +1727,20 @@ void Autotune(pbat_vbd_integrator& h, float dt, int sweeps, double* timingsUs, i
                     cands.push_back({L, K, x != 0, nt != 0, ell != 0});
     }
     bool const oldE = h.useEll;
+    h.lanes = h.perLane = 0;
+    bool const local = StepsLocally(h);
+    h.lanes = oldL, h.perLane = oldK;
+    if (local && cands.size() == kMaxTuneRows)
+        cands.pop_back();
     double best = 1e300;
     Candidate bestC{EffectiveLanes(h), EffectivePerLane(h), h.xcdRemap, h.ntStream, h.useEll};
     int count = 0;
     try
     {
         // the automatic shape of a handle of small meshes: all sweeps in one launch
-        h.lanes = h.perLane = 0;
-        if (StepsLocally(h))
+        if (local)
         {
+            h.lanes = h.perLane = 0;
             EnqueueLocalStep(h, dt, 1, 1); // warm-up
             PBAT_HIP(hipEventRecord(e0, h.stream));
             EnqueueLocalStep(h, dt, sweeps, 1);

@@ -242,7 +242,8 @@ class Integrator:
 
     def autotune(self, dt: float = 0.01, sweeps: int = 10):
         """Pick the fastest sweep shape by timing full sweeps; state is unchanged.
-        Returns rows (lanes, incidences per lane, xcd remap, non-temporal, fixed stride, us per sweep)."""
+        Returns rows (lanes, incidences per lane, xcd remap, non-temporal, fixed stride, us per sweep);
+        lanes = incidences = 0: the step in one launch, which handles of small meshes time first."""
         t = np.zeros(192)
         n = ctypes.c_int32()
         _native.check(self._lib.pbat_vbd_integrator_autotune(self._h, float(dt), int(sweeps),
@@ -329,7 +330,8 @@ class Integrator:
         _native.check(self._lib.pbat_vbd_integrator_set_timing(self._h, int(bool(enabled))))
 
     def sweep_timing(self, reset: bool = False):
-        """(summed HIP-event milliseconds of sweep launches, number of launches)"""
+        """(summed HIP-event milliseconds of sweep launches, number of launches); a step in
+        one launch counts as one"""
         ms, n = ctypes.c_double(), ctypes.c_int64()
         _native.check(self._lib.pbat_vbd_integrator_sweep_timing(self._h, ctypes.byref(ms), ctypes.byref(n),
                                                                  int(bool(reset))))
@@ -428,8 +430,9 @@ class BatchIntegrator(Integrator):
     """One integrator for many independent meshes (no reference counterpart).
 
     The meshes are stepped together: one launch per colour covers the whole
-    batch, and each mesh is swept in the same order as its own ``Integrator``
-    would sweep it. ``x``/``v`` are the meshes' ``3 x nV_b`` matrices
+    batch (batches of small meshes: one launch covers the step), and each mesh is
+    swept in the same order as its own ``Integrator`` would sweep it; its bits are
+    the same when both are set to one sweep shape that takes the launches. ``x``/``v`` are the meshes' ``3 x nV_b`` matrices
     concatenated in batch order; ``mesh_positions()`` splits them.
     """
 
