@@ -1250,7 +1250,7 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
         std::vector<void const*> const ptrs{
             R.y.ptr,         R.r.ptr,           R.z.ptr,           R.z2.ptr,         R.p.ptr,
             R.yD.ptr,        R.rD.ptr,          R.pD.ptr,          R.sD.ptr,         R.wD.ptr,
-            R.aggDone.ptr,           R.rhs.ptr,         R.hold.ptr,       R.dinv.ptr,
+            R.q.ptr,         R.aggDone.ptr,     R.rhs.ptr,         R.hold.ptr,       R.dinv.ptr,
             R.scal.ptr,      R.flags.ptr,       R.coarseF.ptr,     R.rc.ptr,         R.zc.ptr,
             R.bsrRowPtr.ptr, R.bsrCol.ptr,      R.bsrA.ptr,        R.bsrB.ptr,       R.bsrC.ptr,
             h.meshOf.ptr,    R.meshOfRow.ptr,   R.aggOfRow.ptr,    R.bsrChunks.ptr,  R.aggInfo.ptr,
