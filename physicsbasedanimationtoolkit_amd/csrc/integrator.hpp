@@ -428,9 +428,9 @@ int EffectiveLanes(pbat_vbd_integrator const& h);
 int EffectivePerLane(pbat_vbd_integrator const& h);
 // Launch one colour's sweep over nVerts vertices with the current shape.
 void LaunchSweep(pbat_vbd_integrator& h, device::SweepArgs const& a, int nVerts);
-// Star records of the current moduli (tgp): the CSR constants, then their copies
-// (fixed-stride rows, local records).
+// Star records of the current moduli (tgp) in every layout.
 void RebuildStarMaterial(pbat_vbd_integrator& h);
+// The copies of the CSR star records (fixed-stride rows, local records).
 void FillStarCopies(pbat_vbd_integrator& h);
 device::SweepArgs MakeSweepArgs(pbat_vbd_integrator& h, float sdt, float sdt2);
 // One forward Step (gpu/impl/vbd/Integrator.cu:82-103): graph replay or eager launches.
@@ -452,6 +452,9 @@ void DownloadVec(pbat_vbd_integrator& h, float4 const* src, float* dst);
 void DownloadVec(pbat_vbd_integrator& h, double const* src, double* dst);
 // n FP64 device values to FP32 host ones.
 void DownloadFloats(pbat_vbd_integrator& h, double const* src, float* dst, size_t n);
+// n floats in the handle's pinned memory for a kernel to read, or null if they are too
+// many; the stream is synchronised before the next use of that memory.
+float const* StageFloats(pbat_vbd_integrator& h, float const* src, size_t n);
 void CheckVertexArray(pbat_vbd_integrator const& h, void const* p, int64_t n, char const* what);
 pbat_vbd_integrator& Handle(pbat_vbd_integrator* h);
 // Vertex-triangle contact (vbd_contact.hip): set-up from the data, the step's active

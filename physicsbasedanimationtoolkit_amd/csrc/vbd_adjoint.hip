@@ -1529,24 +1529,37 @@ void SetLogYoung(pbat_vbd_integrator& h, float const* logY, int64_t nT)
     PBAT_HIP(hipSetDevice(h.device));
     RolloutState& R = h.rollout;
     std::vector<float> v(logY, logY + nT);
-    if (R.logY.n != v.size())
-        R.logY.allocate(v.size());
-    PBAT_HIP(hipMemcpyAsync(R.logY.ptr, v.data(), sizeof(float) * v.size(), hipMemcpyHostToDevice, h.stream));
-    hipLaunchKernelGGL(device::SetLogYoung, dim3(Blocks(nT)), dim3(256), 0, h.stream, R.logY.ptr, h.matBase.ptr,
+    float const* from = StageFloats(h, v.data(), v.size());
+    if (!from)
+    {
+        if (R.logY.n != v.size())
+            R.logY.allocate(v.size());
+        PBAT_HIP(hipMemcpyAsync(R.logY.ptr, v.data(), sizeof(float) * v.size(), hipMemcpyHostToDevice, h.stream));
+        from = R.logY.ptr;
+    }
+    hipLaunchKernelGGL(device::SetLogYoung, dim3(Blocks(nT)), dim3(256), 0, h.stream, from, h.matBase.ptr,
                        h.tgp.ptr, h.slotsRows.ptr, h.rows.ids.ptr, h.rows.g2.ptr, static_cast<int>(nT));
     RebuildStarMaterial(h);
     PBAT_HIP(hipGetLastError());
+    // meanwhile the (mu, lambda) of the traces follow the new moduli
+    auto scaleLame = [&](int begin, int end, int) {
+        for (int64_t e = begin; e < end; ++e)
+        {
+            float const scale = std::exp(v[e] - h.logYCurrent[e]);
+            h.lameHost[2 * e] *= scale;
+            h.lameHost[2 * e + 1] *= scale;
+        }
+    };
+    try
+    {
+        HostParallel(static_cast<int>(nT), std::clamp(static_cast<int>(nT) / 65536, 1, 8), scaleLame);
+    }
+    catch (...)
+    {
+        (void)hipStreamSynchronize(h.stream); // the values are still being read
+        throw;
+    }
     PBAT_HIP(hipStreamSynchronize(h.stream));
-    HostParallel(static_cast<int>(nT), std::clamp(static_cast<int>(nT) / 65536, 1, 8),
-                 [&](int begin, int end, int) {
-                     for (int64_t e = begin; e < end; ++e)
-                     {
-                         // (mu, lambda) of the traces follow the new moduli
-                         float const scale = std::exp(v[e] - h.logYCurrent[e]);
-                         h.lameHost[2 * e] *= scale;
-                         h.lameHost[2 * e + 1] *= scale;
-                     }
-                 });
     h.logYCurrent = v;
     R.Discard();
 }

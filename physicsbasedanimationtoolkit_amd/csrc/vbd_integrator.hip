@@ -230,13 +230,13 @@ void RebuildStarMaterial(pbat_vbd_integrator& h)
     a.rowPtr = h.star.rowPtr.ptr, a.nbr = h.star.nbr.ptr, a.inc = h.star.inc.ptr;
     a.shape = h.star.shape.ptr, a.tet = h.star.tet.ptr, a.tgp = h.tgp.ptr;
     a.wideIds = h.star.wideIds.ptr, a.wideGeo = h.star.wideGeo.ptr;
-    a.nRows = static_cast<int>(h.nUpdated);
-    a.width = std::max<int>(h.star.maxNeighbours, static_cast<int>(h.maxDegree));
-    int64_t const n = h.nUpdated * a.width;
-    if (n == 0)
+    a.nbrE = h.star.nbrE.ptr, a.incE = h.star.incE.ptr, a.nbrL = h.star.nbrL.ptr, a.incL = h.star.incL.ptr;
+    a.nRows = static_cast<int>(h.nUpdated), a.nbrStride = h.star.maxNeighbours, a.incStride = h.ellStride;
+    if (h.nUpdated == 0)
         return;
-    hipLaunchKernelGGL(device::StarMaterial, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, h.stream, a);
-    FillStarCopies(h);
+    int64_t const grid = (h.nUpdated * device::kMaterialLanes + 255) / 256;
+    hipLaunchKernelGGL(device::StarMaterial, dim3(static_cast<unsigned>(std::min<int64_t>(grid, 1 << 20))), dim3(256),
+                       0, h.stream, a);
 }
 
 hipEvent_t NextEvent(pbat_vbd_integrator& h)
@@ -678,6 +678,15 @@ void InPieces(pbat_vbd_integrator& h, size_t n, size_t bytes, F&& f)
     size_t const piece = h.stageBytes / bytes / 256 * 256; // whole workgroups, 16-byte aligned
     for (size_t first = 0; first < n; first += piece)
         f(first, std::min(piece, n - first));
+}
+
+float const* StageFloats(pbat_vbd_integrator& h, float const* src, size_t n)
+{
+    EnsureStage(h);
+    if (n * sizeof(float) > std::min(kStageRead, h.stageBytes))
+        return nullptr;
+    std::memcpy(h.stage, src, n * sizeof(float));
+    return static_cast<float const*>(h.stageDev);
 }
 
 // Copy a 3 x nV host matrix (original numbering) into a float4 device array
