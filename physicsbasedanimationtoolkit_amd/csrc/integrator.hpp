@@ -127,10 +127,13 @@ struct StarRecords
     DeviceArray<int4> wideIds;
     DeviceArray<float4> wideGeo;
     // handles of small meshes only (device::VbdStepLocal, device::CgLocal)
-    DeviceArray<int2> nbrL, localMeshes;
+    DeviceArray<int2> nbrL;
     DeviceArray<device::LocalInc> incL;
-    DeviceArray<device::LocalRange> localRanges;
-    DeviceArray<int> localVerts, localPlace;
+    DeviceArray<int> localTables; // holds the four below
+    int2 const* localMeshes = nullptr;
+    device::LocalRange const* localRanges = nullptr;
+    int const* localVerts = nullptr;
+    int const* localPlace = nullptr;
     int localMaxRows = 0;   // > 0: the local tables are there; most updated vertices of a mesh
     int localMaxVerts = 0;  // > 0: small enough for VbdStepLocal; most vertices of a mesh
     int localMaxColour = 0; // largest colour of a mesh
@@ -140,8 +143,7 @@ struct StarRecords
     void reset()
     {
         rowPtr.reset(), nbr.reset(), nbrE.reset(), inc.reset(), incE.reset(), shape.reset(), tet.reset();
-        wideIds.reset(), wideGeo.reset(), nbrL.reset(), localMeshes.reset(), incL.reset(), localRanges.reset();
-        localVerts.reset(), localPlace.reset();
+        wideIds.reset(), wideGeo.reset(), nbrL.reset(), incL.reset(), localTables.reset();
     }
 };
 
@@ -409,8 +411,6 @@ struct pbat_vbd_integrator
         ipermD.reset(), massD.reset(), stageCopy.reset();
         if (stage)
             (void)hipHostFree(stage);
-        if (statusHost)
-            (void)hipHostFree(statusHost);
         if (rollout.doneHost)
             (void)hipHostFree(rollout.doneHost);
         for (hipEvent_t e : rollout.chunkEvent)

@@ -1051,14 +1051,14 @@ SolveResult SolveLocal(pbat_vbd_integrator& h, device::CgState const& cg, float4
         R.cgLocalPlace.allocate(R.bsrCol.n);
         hipLaunchKernelGGL(device::CgLocalRowTable, dim3(Blocks(nV)), dim3(256), 0, h.stream,
                            static_cast<int const*>(R.bsrRowPtr.ptr), static_cast<int const*>(R.bsrCol.ptr),
-                           static_cast<int const*>(h.star.localVerts.ptr),
-                           static_cast<int const*>(h.star.localPlace.ptr), R.cgLocalRows.ptr, R.cgLocalPlace.ptr, n,
+                           h.star.localVerts,
+                           h.star.localPlace, R.cgLocalRows.ptr, R.cgLocalPlace.ptr, n,
                            nV);
     }
     device::CgLocalArgs a{};
     a.rows = R.cgLocalRows.ptr, a.place = R.cgLocalPlace.ptr;
     a.va = R.bsrA.ptr, a.vb = R.bsrB.ptr, a.vc = R.bsrC.ptr, a.dinvRows = R.dinv.ptr, a.dinv = R.cgLocalDinv.ptr;
-    a.ranges = h.star.localRanges.ptr, a.meshes = h.star.localMeshes.ptr, a.verts = h.star.localVerts.ptr;
+    a.ranges = h.star.localRanges, a.meshes = h.star.localMeshes, a.verts = h.star.localVerts;
     auto vec = [](DeviceArray<double> const& v) { return reinterpret_cast<device::Vec3d*>(v.ptr); };
     a.y = vec(R.yD), a.r = vec(R.rD), a.p = vec(R.pD), a.s = vec(R.sD), a.w = vec(R.wD);
     a.z = R.z.ptr, a.out = y, a.b = b, a.cg = cg, a.nColors = nC, a.maxRows = h.star.localMaxRows;

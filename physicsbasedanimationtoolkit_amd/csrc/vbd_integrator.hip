@@ -213,7 +213,7 @@ void FillStarCopies(pbat_vbd_integrator& h)
     if (h.star.localMaxVerts > 0)
         hipLaunchKernelGGL(device::LocalRecords,
                            dim3(static_cast<unsigned>((h.nUpdated * device::kLocalInc + 255) / 256)), dim3(256), 0,
-                           h.stream, h.star.rowPtr.ptr, h.star.nbr.ptr, h.star.inc.ptr, h.star.localPlace.ptr,
+                           h.stream, h.star.rowPtr.ptr, h.star.nbr.ptr, h.star.inc.ptr, h.star.localPlace,
                            h.star.nbrL.ptr, h.star.incL.ptr, static_cast<int>(h.nUpdated));
     if (!h.star.incE.ptr)
         return;
@@ -453,7 +453,7 @@ int EnqueueLocalStep(pbat_vbd_integrator& h, float dt, int iterations, int subst
     float const sdt = dt / static_cast<float>(substeps);
     device::LocalStepArgs a{};
     a.nbr = h.star.nbrL.ptr, a.inc = h.star.incL.ptr;
-    a.ranges = h.star.localRanges.ptr, a.meshes = h.star.localMeshes.ptr, a.verts = h.star.localVerts.ptr;
+    a.ranges = h.star.localRanges, a.meshes = h.star.localMeshes, a.verts = h.star.localVerts;
     a.xm = h.xm.ptr, a.xtil = h.xtil.ptr, a.xt = h.xt.ptr, a.vel = h.vel.ptr, a.vprev = h.vprev.ptr;
     a.aext = h.aext.ptr;
     a.nColors = static_cast<int>(h.colorBegin.size()) - 1;
@@ -639,42 +639,40 @@ void CheckVertexArray(pbat_vbd_integrator const& h, void const* p, int64_t n, ch
     }
 }
 
-// Pinned memory of the handle for vertex data, 24 bytes per vertex up to 8 MB (larger
-// data pass in pieces), and the device's copies of iperm and the masses.
+// Pinned memory of the handle for vertex data, 24 bytes per vertex (whole workgroups of
+// 256) up to 8 MB, larger data pass in pieces; behind it the objective's sums and the step
+// status, 64 bytes each. One allocation, since one costs 25 us of a handle's creation and
+// 25 of its end (125 vertices: 90 us less than with the status apart, a local table each
+// and the copy below always there). Also the device's copies of iperm and the masses.
 constexpr size_t kStageBytes = size_t{8} << 20;
 // Uploads beyond this are copied to the device first; below it the kernel reads the
 // pinned memory itself (125 vertices: set 29 -> 15 us either way, 4,913: 28 read, 34
-// copied, 274,625: 760 read, 733 copied).
+// copied, 274,625, the caller's transposition included: 760 read, 733 copied).
 constexpr size_t kStageRead = size_t{64} << 10;
 
-void EnsureStage(pbat_vbd_integrator& h)
+void AllocateStage(pbat_vbd_integrator& h)
 {
-    if (h.stage)
-        return;
-    size_t const bytes = std::clamp<size_t>(24 * static_cast<size_t>(h.nV), 256 * 24, kStageBytes);
-    if (!h.ipermD.ptr)
-        h.ipermD.upload(h.iperm, h.stream);
-    if (!h.massD.ptr)
-        h.massD.upload(h.massOrig, h.stream);
-    if (!h.stageCopy.ptr)
+    size_t const groups = (static_cast<size_t>(h.nV) + 255) / 256;
+    size_t const bytes = std::min<size_t>(groups * 256 * 24, kStageBytes);
+    h.ipermD.upload(h.iperm, h.stream);
+    h.massD.upload(h.massOrig, h.stream);
+    if (3 * sizeof(float) * static_cast<size_t>(h.nV) > kStageRead)
         h.stageCopy.allocate(bytes / sizeof(float));
-    PBAT_HIP(hipStreamSynchronize(h.stream));
     void *p = nullptr, *d = nullptr;
-    if (hipHostMalloc(&p, bytes + 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
-        !p) // and a few results behind them
+    if (hipHostMalloc(&p, bytes + 128, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess || !p)
         Fail(PBAT_VBD_ERROR_OUT_OF_MEMORY, "hipHostMalloc of the vertex data's pinned memory failed");
-    hipError_t const e = hipHostGetDevicePointer(&d, p, 0);
-    if (e != hipSuccess)
-        (void)hipHostFree(p);
-    PBAT_HIP(e);
-    h.stage = p, h.stageDev = d, h.stageBytes = bytes;
+    h.stage = p, h.stageBytes = bytes; // freed with the handle from here on
+    PBAT_HIP(hipHostGetDevicePointer(&d, p, 0));
+    h.stageDev = d;
+    h.statusHost = reinterpret_cast<int*>(static_cast<char*>(p) + bytes + 64);
+    h.statusDev = reinterpret_cast<int*>(static_cast<char*>(d) + bytes + 64);
+    *h.statusHost = 0;
 }
 
 // f(first, count) over n items of `bytes` each in pieces that the pinned memory holds.
 template <class F>
 void InPieces(pbat_vbd_integrator& h, size_t n, size_t bytes, F&& f)
 {
-    EnsureStage(h);
     size_t const piece = h.stageBytes / bytes / 256 * 256; // whole workgroups, 16-byte aligned
     for (size_t first = 0; first < n; first += piece)
         f(first, std::min(piece, n - first));
@@ -682,7 +680,6 @@ void InPieces(pbat_vbd_integrator& h, size_t n, size_t bytes, F&& f)
 
 float const* StageFloats(pbat_vbd_integrator& h, float const* src, size_t n)
 {
-    EnsureStage(h);
     if (n * sizeof(float) > std::min(kStageRead, h.stageBytes))
         return nullptr;
     std::memcpy(h.stage, src, n * sizeof(float));
@@ -894,10 +891,21 @@ void BuildLocal(pbat_vbd_integrator& h, std::vector<int> const& meshOfOrig)
     if (maxRows > device::kCgLocalRows)
         return;
     h.star.localMaxRows = maxRows;
-    h.star.localRanges.upload(ranges, h.stream);
-    h.star.localMeshes.upload(meshes, h.stream);
-    h.star.localVerts.upload(verts, h.stream);
-    h.star.localPlace.upload(place, h.stream);
+    // one array: meshes, ranges, verts, place
+    std::vector<int> tables;
+    auto append = [&](auto const& v) {
+        static_assert(sizeof(v[0]) % sizeof(int) == 0, "tables of 32-bit entries");
+        size_t const at = tables.size(), n = v.size() * (sizeof(v[0]) / sizeof(int));
+        tables.resize(at + n);
+        std::memcpy(tables.data() + at, v.data(), n * sizeof(int));
+        return at;
+    };
+    size_t const atMeshes = append(meshes), atRanges = append(ranges), atVerts = append(verts), atPlace = append(place);
+    h.star.localTables.upload(tables, h.stream);
+    int const* const t = h.star.localTables.ptr;
+    h.star.localMeshes = reinterpret_cast<int2 const*>(t + atMeshes);
+    h.star.localRanges = reinterpret_cast<device::LocalRange const*>(t + atRanges);
+    h.star.localVerts = t + atVerts, h.star.localPlace = t + atPlace;
     if (h.maxDegree <= device::kLocalInc && h.star.maxNeighbours <= device::kLocalNbr &&
         h.nUpdated * device::kLocalInc < (int64_t{1} << 31) && maxColour <= device::kLocalMaxColour &&
         LocalLdsBytes(maxVerts, nC) <= kStarLdsBytes)
@@ -1100,16 +1108,16 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
         int64_t const e = d->GVGe[k];
         int const il = static_cast<int>(d->GVGilocal[k]);
         double const* G = d->GP + 12 * e; // G(r, c) = G[4c + r]
-        TetShape T{};
-        int n = 0;
-        for (int j = 0; j < 4; ++j)
+        static constexpr int kOthers[4][3] = {{1, 2, 3}, {0, 2, 3}, {0, 1, 3}, {0, 1, 2}};
+        double const own[3] = {G[il], G[4 + il], G[8 + il]};
+        TetShape T;
+        for (int n = 0; n < 3; ++n)
         {
-            if (j == il)
-                continue;
+            int const j = kOthers[il][n];
             T.ids[n] = TV4(TV[e], j);
             for (int c = 0; c < 3; ++c)
-                T.g[n][c] = G[4 * c + j], T.gamma[n] += G[4 * c + j] * G[4 * c + il];
-            ++n;
+                T.g[n][c] = G[4 * c + j];
+            T.gamma[n] = T.g[n][0] * own[0] + T.g[n][1] * own[1] + T.g[n][2] * own[2];
         }
         T.kappa = T.g[0][0] * (T.g[1][1] * T.g[2][2] - T.g[1][2] * T.g[2][1]) -
                   T.g[0][1] * (T.g[1][0] * T.g[2][2] - T.g[1][2] * T.g[2][0]) +
@@ -1136,17 +1144,7 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
         for (int64_t v = 0; v < nUpd; ++v)
         {
             int64_t const i = h->perm[v], k0 = d->GVGp[i], k1 = d->GVGp[i + 1];
-            row.clear();
-            for (int64_t k = k0; k < k1; ++k)
-                for (int j = 0; j < 4; ++j)
-                {
-                    int const q = TV4(TV[d->GVGe[k]], j);
-                    if (q != static_cast<int>(v) && at[q] < 0)
-                        at[q] = 0, row.push_back(q);
-                }
-            for (size_t s = 0; s < row.size(); ++s)
-                at[row[s]] = static_cast<int>(s);
-            sum.assign(row.size(), 0.);
+            row.clear(), sum.clear();
             for (int64_t k = k0; k < k1; ++k)
             {
                 int64_t const e = d->GVGe[k];
@@ -1165,7 +1163,12 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
                 R.g1[slot] = make_float4(f(1, 1), f(1, 2), f(2, 0), f(2, 1));
                 R.g2[slot] = make_float2(f(2, 2), m.z);
                 for (int j = 0; j < 3; ++j)
-                    sum[at[T.ids[j]]] += wmu * T.gamma[j];
+                {
+                    int& place = at[T.ids[j]];
+                    if (place < 0)
+                        place = static_cast<int>(row.size()), row.push_back(T.ids[j]), sum.push_back(0.);
+                    sum[place] += wmu * T.gamma[j];
+                }
                 // positions of a wide row do not fit; VbdSweepWide reads none
                 inc[slot] = device::StarInc{static_cast<unsigned>(at[T.ids[0]]) |
                                                 static_cast<unsigned>(at[T.ids[1]]) << 8 |
@@ -1283,20 +1286,8 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
         h->trPartials.allocate(3 * static_cast<size_t>(kObjectiveBlocks) + 3);
     }
     h->energy.allocate(3);
-    {
-        void* p = nullptr;
-        if (hipHostMalloc(&p, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess || !p)
-            Fail(PBAT_VBD_ERROR_OUT_OF_MEMORY, "hipHostMalloc of the step status failed");
-        h->statusHost = static_cast<int*>(p);
-        std::memset(p, 0, 64);
-        void* dp = nullptr;
-        PBAT_HIP(hipHostGetDevicePointer(&dp, p, 0));
-        h->statusDev = static_cast<int*>(dp);
-        h->fp64Solves.allocate(1);
-        unsigned int const zero = 0;
-        PBAT_HIP(hipMemcpyAsync(h->fp64Solves.ptr, &zero, sizeof(zero), hipMemcpyHostToDevice, h->stream));
-        PBAT_HIP(hipStreamSynchronize(h->stream));
-    }
+    h->fp64Solves.allocate(1);
+    PBAT_HIP(hipMemsetAsync(h->fp64Solves.ptr, 0, sizeof(unsigned int), h->stream));
     PBAT_HIP(hipMemsetAsync(h->xtil.ptr, 0, sizeof(float4) * nV, h->stream));
     PBAT_HIP(hipMemsetAsync(h->vprev.ptr, 0, sizeof(float4) * nV, h->stream));
 
@@ -1310,6 +1301,7 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
     }
     for (int64_t i = 0; i < nV; ++i)
         h->massOrig[i] = static_cast<float>(d->m[i]);
+    AllocateStage(*h);
     UploadVec(*h, h->xm.ptr, x32.data(), true, h->xt.ptr);
     UploadVec(*h, h->vel.ptr, v32.data(), false);
     UploadVec(*h, h->aext.ptr, a32.data(), false);
@@ -1375,7 +1367,6 @@ void ObjectiveOnDevice(pbat_vbd_integrator& h, float4 const* x, float4 const* xt
     size_t const nb = static_cast<size_t>(std::max(gridG, kObjectiveBlocks));
     double* partF = h.objPart.ptr;
     double* partG = h.objPart.ptr + 3 * nb;
-    EnsureStage(h);
     // (K, U, .) then (|g|^2, ., .), in pinned memory
     double* const sums = reinterpret_cast<double*>(static_cast<char*>(h.stageDev) + h.stageBytes);
     device::TrEpilogue none{};
