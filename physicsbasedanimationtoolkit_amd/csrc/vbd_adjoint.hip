@@ -1090,12 +1090,15 @@ SolveResult Solve(pbat_vbd_integrator& h, float4 const* xs, float dt, float4* y,
     int const gridN = Blocks(n);
     bool const twoLevel = cfg.solver == PBAT_VBD_ADJOINT_PCG_TWO_LEVEL && h.nAggregates > 0;
     bool const fused = cfg.solver == PBAT_VBD_ADJOINT_PCG_JACOBI || cfg.solver == PBAT_VBD_ADJOINT_PCG_TWO_LEVEL;
-    // fused chunks hold an even number of iterations, since the buffers of the sums swap,
-    // and few of them when the launches queued behind the last iteration are long to pass:
-    // 5 us each at 224,000 rows (a rollout of 64 meshes: 136.1 ms in chunks of 10, 132.3
-    // in chunks of 4), 2 us at 12,000, where more graph launches cost as much (a solve
-    // 2.99 ms, 3.04)
-    int const maxChunk = n >= 65536 ? 4 : std::numeric_limits<int>::max();
+    // fused chunks hold an even number of iterations, since the buffers of the sums swap.
+    // Two-level chunks of large handles hold at most 4: the launches queued behind the
+    // last iteration take 5 us each to pass at 224,000 rows, where a rollout's solves are
+    // short (64 meshes: 136.1 ms in chunks of 10, 132.3 in chunks of 4). One solve, us in
+    // chunks of 4 / 10: 57,800 rows 5,262 / 5,263, 67,200 5,442 / 5,437, 115,000 12,657 /
+    // 12,679, 238,000 15,780 / 15,924; 12,000 rows 3,040 / 2,990. Block Jacobi's two
+    // launches an iteration pass sooner and each graph launch costs as much: 67,200 rows
+    // 2,650 / 2,524, 115,000 4,213 / 3,985
+    int const maxChunk = twoLevel && n >= 65536 ? 4 : std::numeric_limits<int>::max();
     int const check = fused ? std::min((std::max(1, cfg.check_every) + 1) / 2 * 2, maxChunk)
                             : std::max(1, cfg.check_every);
     AssembleBsr(h, xs, dt, fused);
