@@ -230,8 +230,6 @@ struct SweepArgs
 };
 
 typedef int v2i __attribute__((ext_vector_type(2)));
-typedef float v2f __attribute__((ext_vector_type(2)));
-typedef float v4f __attribute__((ext_vector_type(4)));
 
 // Loads of the star records and of the adjoint's incidence records, optionally
 // with the non-temporal hint.
