@@ -36,8 +36,24 @@ inline void CountDeviceBytes(int64_t delta)
     {                                                                                                             \
         hipError_t const _e = (call);                                                                             \
         if (_e != hipSuccess)                                                                                     \
+        {                                                                                                         \
+            (void)hipGetLastError(); /* reported here, and not by a later look at the thread's error */           \
             Fail(PBAT_VBD_ERROR_HIP, std::string(#call) + ": " + hipGetErrorString(_e));                          \
+        }                                                                                                         \
     } while (0)
+
+// A launch checked by its own status, where an earlier failed call of the thread (which
+// hipGetLastError would report) must not fail it.
+template <class... P, class... A>
+void Launch(void (*kernel)(P...), dim3 grid, dim3 block, size_t lds, hipStream_t s, A&&... args)
+{
+    static_assert(sizeof...(P) == sizeof...(A), "one argument per parameter");
+    auto launch = [&](P... p) {
+        void* pointers[] = {static_cast<void*>(&p)...};
+        return hipLaunchKernel(reinterpret_cast<void const*>(kernel), grid, block, pointers, lds, s);
+    };
+    PBAT_HIP(launch(args...));
+}
 
 template <class T>
 struct DeviceArray
@@ -78,6 +94,7 @@ struct DeviceArray
         if (e != hipSuccess)
         {
             ptr = nullptr;
+            (void)hipGetLastError();
             Fail(PBAT_VBD_ERROR_OUT_OF_MEMORY, std::string("hipMalloc failed: ") + hipGetErrorString(e));
         }
         n = count;

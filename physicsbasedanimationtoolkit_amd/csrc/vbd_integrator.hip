@@ -462,9 +462,8 @@ int EnqueueLocalStep(pbat_vbd_integrator& h, float dt, int iterations, int subst
     a.nonfinite = h.statusDev;
     if (h.acceleration == PBAT_VBD_ACCELERATION_CHEBYSHEV)
         a.xkm1 = h.xkm1.ptr, a.xkm2 = h.xkm2.ptr, a.rho2 = h.rho * h.rho;
-    hipLaunchKernelGGL(device::VbdStepLocal, dim3(h.nMeshes), dim3(h.star.localThreads),
-                       LocalLdsBytes(a.maxVerts, a.nColors), h.stream, a);
-    PBAT_HIP(hipGetLastError());
+    Launch(device::VbdStepLocal, dim3(h.nMeshes), dim3(h.star.localThreads), LocalLdsBytes(a.maxVerts, a.nColors),
+           h.stream, a);
     return 1;
 }
 
@@ -659,8 +658,12 @@ void AllocateStage(pbat_vbd_integrator& h)
     if (3 * sizeof(float) * static_cast<size_t>(h.nV) > kStageRead)
         h.stageCopy.allocate(bytes / sizeof(float));
     void *p = nullptr, *d = nullptr;
-    if (hipHostMalloc(&p, bytes + 128, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess || !p)
+    hipError_t const e = hipHostMalloc(&p, bytes + 128, hipHostMallocMapped | hipHostMallocCoherent);
+    if (e != hipSuccess || !p)
+    {
+        (void)hipGetLastError();
         Fail(PBAT_VBD_ERROR_OUT_OF_MEMORY, "hipHostMalloc of the vertex data's pinned memory failed");
+    }
     h.stage = p, h.stageBytes = bytes; // freed with the handle from here on
     PBAT_HIP(hipHostGetDevicePointer(&d, p, 0));
     h.stageDev = d;
@@ -698,11 +701,8 @@ void UploadVec(pbat_vbd_integrator& h, float4* dst, float const* src, bool masse
             PBAT_HIP(hipMemcpyAsync(h.stageCopy.ptr, h.stage, 3 * sizeof(float) * n, hipMemcpyHostToDevice, h.stream));
             from = h.stageCopy.ptr;
         }
-        hipLaunchKernelGGL(device::UploadVertices, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, h.stream,
-                           from, static_cast<int const*>(h.ipermD.ptr),
-                           masses ? static_cast<float const*>(h.massD.ptr) : nullptr, static_cast<int>(first),
-                           static_cast<int>(n), dst, second);
-        PBAT_HIP(hipGetLastError());
+        Launch(device::UploadVertices, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, h.stream, from,
+               h.ipermD.ptr, masses ? h.massD.ptr : nullptr, static_cast<int>(first), static_cast<int>(n), dst, second);
         PBAT_HIP(hipStreamSynchronize(h.stream));
     });
 }
@@ -711,10 +711,8 @@ template <class T, class S>
 void Download(pbat_vbd_integrator& h, S const* src, T* dst)
 {
     InPieces(h, static_cast<size_t>(h.nV), 3 * sizeof(T), [&](size_t first, size_t n) {
-        hipLaunchKernelGGL((device::DownloadVertices<T, S>), dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0,
-                           h.stream, src, static_cast<int const*>(h.ipermD.ptr), static_cast<int>(first),
-                           static_cast<int>(n), static_cast<T*>(h.stageDev));
-        PBAT_HIP(hipGetLastError());
+        Launch(device::DownloadVertices<T, S>, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, h.stream, src,
+               h.ipermD.ptr, static_cast<int>(first), static_cast<int>(n), static_cast<T*>(h.stageDev));
         PBAT_HIP(hipStreamSynchronize(h.stream));
         std::memcpy(dst + 3 * first, h.stage, 3 * sizeof(T) * n);
     });
@@ -727,9 +725,8 @@ void DownloadVec(pbat_vbd_integrator& h, double const* src, double* dst) { Downl
 void DownloadFloats(pbat_vbd_integrator& h, double const* src, float* dst, size_t n)
 {
     InPieces(h, n, sizeof(float), [&](size_t first, size_t count) {
-        hipLaunchKernelGGL(device::ToFloats, dim3(static_cast<unsigned>((count + 255) / 256)), dim3(256), 0, h.stream,
-                           src + first, static_cast<float*>(h.stageDev), static_cast<int>(count));
-        PBAT_HIP(hipGetLastError());
+        Launch(device::ToFloats, dim3(static_cast<unsigned>((count + 255) / 256)), dim3(256), 0, h.stream, src + first,
+               static_cast<float*>(h.stageDev), static_cast<int>(count));
         PBAT_HIP(hipStreamSynchronize(h.stream));
         std::memcpy(dst + first, h.stage, sizeof(float) * count);
     });
