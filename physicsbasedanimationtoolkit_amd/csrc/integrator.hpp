@@ -305,7 +305,7 @@ struct pbat_vbd_integrator
     pbat_vbd::DeviceArray<int> meshOf; // mesh of each internal vertex (0 for a plain integrator)
     // Aggregates of updated vertices for the adjoint's two-level preconditioner:
     // ids contiguous per mesh; each mesh's coarse operator is a dense block of
-    // (3 x its aggregates)^2 doubles.
+    // (kCoarseDofs x its aggregates)^2 doubles.
     int nAggregates = 0;
     std::vector<int> aggBegin;          // per mesh: first aggregate id (nMeshes + 1)
     std::vector<int64_t> coarseOffset;  // per mesh: first double of its dense block (nMeshes + 1)

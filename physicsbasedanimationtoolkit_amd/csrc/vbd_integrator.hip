@@ -20,7 +20,8 @@
 //    vertices of one colour share no tet, so no vertex reads what another
 //    vertex of its colour writes;
 //  - the substep-begin/-end work is two fused elementwise kernels, and the
-//    whole launch sequence of a Step is captured once in a hipGraph and replayed.
+//    whole launch sequence of a Step is captured once in a hipGraph and replayed;
+//  - meshes with small colours step in one launch, a workgroup each.
 #include "pbat_vbd.h"
 #include "status.hpp"
 #include "vbd_kernels.hpp"
@@ -82,7 +83,7 @@ int EffectiveLanes(pbat_vbd_integrator const& h)
         // reduction and the Newton step, more shorten the chain of a small launch.
         // Degree 24, us per launch at 16 x 2 / 8 x 3: 10^3 3.14 / 3.32, 32^3 3.43 /
         // 3.52, 48^3 (14,400 vertices a colour) 4.65 / 4.51, 64^3 6.33 / 6.37, 80^3
-        // 9.25 / 8.53, 256 meshes (107,000 a colour) 13.4 / 11.3
+        // 9.25 / 8.53, 256 meshes (107,000 a colour) 13.3 / 11.5
         int const d = static_cast<int>(std::max<int64_t>(h.maxDegree, 1));
         int64_t const colours = std::max<int64_t>(static_cast<int64_t>(h.colorBegin.size()) - 1, 1);
         int const perLane = h.nUpdated >= kLargeColour * colours ? 3 : 2;
@@ -646,7 +647,7 @@ void CheckVertexArray(pbat_vbd_integrator const& h, void const* p, int64_t n, ch
 constexpr size_t kStageBytes = size_t{8} << 20;
 // Uploads beyond this are copied to the device first; below it the kernel reads the
 // pinned memory itself (125 vertices: set 29 -> 15 us either way, 4,913: 28 read, 34
-// copied, 274,625, the caller's transposition included: 760 read, 733 copied).
+// copied, 274,625: 27 us less copied).
 constexpr size_t kStageRead = size_t{64} << 10;
 
 void AllocateStage(pbat_vbd_integrator& h)
@@ -1225,7 +1226,7 @@ void Create(pbat_vbd_data const* d, pbat_vbd_integrator** out, std::vector<int64
     // dependent load less: 6.33 instead of 6.76 us a launch on 64^3) while the records
     // fit the 256 MB last-level cache; beyond it the unpadded CSR rows, read with
     // non-temporal loads that leave the cache to the positions, are faster (256
-    // meshes, 373 MB of records: 11.3 us against 13.6).
+    // meshes, 373 MB of records: 11.5 us against 13.4).
     if (nUpd > 0 && h->maxDegree > 0 &&
         h->maxDegree * nUpd * 100 <= 135 * static_cast<int64_t>(nIncUpd) && h->maxDegree * nUpd < (int64_t{1} << 31))
     {

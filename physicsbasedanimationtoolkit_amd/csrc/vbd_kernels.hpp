@@ -330,7 +330,8 @@ struct ContactSlots
 // Newton update in place: vertices of one colour share no tet, so none reads
 // what another vertex of the colour writes.
 // What bounds it: on 256 meshes (107,000 vertices a colour, 373 MB of records,
-// beyond the last-level cache) the stream of records, 4.1 TB/s; on 64^3 that
+// beyond the last-level cache) the stream of records, 4.1 TB/s of the 4.9 that the
+// counters see with positions and targets; on 64^3 that
 // stream (15 MB a launch) and the VALU next to a fixed ~3 us of launch ramp and
 // dependent loads; on small meshes the latter alone. Per launch, best shape: 64^3
 // 6.33 us, 80^3 8.5, 256 meshes 11.5. With 32 B and three 16-byte position gathers
@@ -604,9 +605,10 @@ __device__ __forceinline__ float4 InertialTarget(float4 const& p, float4 const& 
 // Vertices [first, first + count) of a packed host matrix (3 values per vertex, the
 // host's order, in pinned memory that src / out maps) into or out of the device's order,
 // 256 per workgroup, packed through LDS so that the link sees whole 16-byte accesses.
-// As a host loop over the vertices with a pageable copy, get took 478 us at 64^3
-// (274,625 vertices) and 56 at 32^3, now 170 and 31; set, with the caller's transposition,
-// 1,450 and 179, now 730 and 113.
+// As a host loop over the vertices with a pageable copy, get took 482 us at 64^3
+// (274,625 vertices) and 58 at 32^3, now 182 and 31; set of a C-ordered matrix, the
+// caller's transposition included, 1,430 and 184, now 328 and 61 (vertex-major: 826 and
+// 107, now 150 and 37).
 template <class T>
 struct alignas(16) Quad16
 {
@@ -720,9 +722,12 @@ struct LocalStepArgs
 // chain), else 2 (the least work per vertex), and up to which meshes are stepped in one
 // workgroup each. A workgroup of kLocalThreads has lanes for every vertex of a colour
 // at once. Cubes, us per colour against a launch's 3.0: 7^3 (56 vertices a colour)
-// 1.45, 8^3 (81) 2.5, 9^3 (113) 2.7, 10^3 (151) 3.1, 11^3 (198) 3.9. 4 lanes take 2.0,
-// 2.3, 2.7 and 3.3, but four steps of 8^3 leave velocities 1.02e-4 of their norm from
-// FP64, where 2 lanes leave 0.97e-4, as the launches do.
+// 1.45, 8^3 (81) 2.5, 9^3 (113) 2.7, 10^3 (151) 3.1, 11^3 (198) 3.9. 4 lanes are not
+// built; a trial took 2.0, 2.3, 2.7 and 3.3, at the same precision (velocities after four
+// steps of 8^3, mean distance from FP64 over 12 meshes: 0.88e-4 of their norm with 2
+// lanes, 0.91e-4 with 4, 0.90e-4 at 16 x 2, 0.82..0.99e-4 by mesh).
+// Batches, us a step of 20 iterations here / as launches in their best shape: 512 of 5^3
+// 195 / 591, 1,024 of 7^3 921 / 1,079, of 8^3 1,018 / 1,440, of 9^3 1,334 / 2,086.
 constexpr int kLocalThreads = 512;
 constexpr int kLocalFewVertices = kLocalThreads / 8;
 constexpr int kLocalManyLanes = 2;
@@ -730,7 +735,9 @@ constexpr int kLocalMaxColour = 128;
 
 // Most updated vertices of a mesh whose Gauss-Seidel-preconditioned solves run in one
 // workgroup (CgLocal). us per iteration there / as launches: 18 rows 7.6 / 48, 100 14.5 /
-// 55, 294 19 / 59, 648 24 / 61, 1,872 47 / 63, 2,730 66 / 65, 3,150 75 / 61.
+// 55, 294 19 / 59, 648 24 / 61, 1,872 47 / 63, 2,730 66 / 65, 3,150 75 / 61. Batches, us a
+// solve: 512 meshes of 180 rows 1,178 / 3,728, of 648 rows 3,272 / 9,545, of 1,210 rows
+// 6,620 / 19,344; 256 of 2,028 rows 6,558 / 14,414.
 constexpr int kCgLocalRows = 2400;
 
 // omega of the Chebyshev update after iteration k (sim/vbd/Kernels.h:97-102 in FP32
